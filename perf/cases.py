@@ -171,7 +171,12 @@ def work(case: dict) -> dict:
     if kind == 'dense':
         return {'bytes': float(4 * used * row + 4 * used * heads), 'flops': dense}
     ideal = -(-target // TILE)
-    kept = min(target, _get(case, 'keep') * ideal * TILE) + text
+    kept = 0.0  # kept target keys of a query row, averaged over the shapes
+    shapes = _get(case, 'shapes').split(',')
+    for st, sh, sw in map(_grid, shapes):
+        n = -(-t // st) * -(-h // sh) * -(-w // sw)
+        kept += min(1.0, _get(case, 'keep') * ideal * ideal / n / n) * target / len(shapes)
+    kept += text
     if _get(case, 'ref'):
         rt, rh, rw = _grid(case['ref'])
         kept += min(1.0, case['ref_keep']) * rt * rh * rw
