@@ -174,19 +174,79 @@ struct PGemm {
   float* out;
 };
 
-constexpr int kKB = 32;       // k per staged block
-constexpr int kRow = kKB + 4; // LDS row pitch (floats)
+constexpr int kKB = 32;  // k per staged block
+
+// Eight consecutive weights of one k as loaded (8 bytes of e4m3, 16 of bf16,
+// 32 of fp32) and their decode to fp32: bf16(e4m3 * scale) for e4m3 (the
+// hardware's OCP fp8 conversion is exact, as is the product's rounding).
+struct WRaw {
+  u32x4 lo, hi;
+};
+
+__device__ __forceinline__ WRaw load_w8(const void* w, int dtype, int64_t i) {
+  WRaw r;
+  if (dtype == 2) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    const u32x2 v = *reinterpret_cast<const u32x2*>(static_cast<const uint8_t*>(w) + i);
+    r.lo = u32x4{v[0], v[1], 0u, 0u};
+  } else if (dtype == 0) {
+    r.lo = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(w) + i);
+  } else {
+    r.lo = *reinterpret_cast<const u32x4*>(static_cast<const float*>(w) + i);
+    r.hi = *reinterpret_cast<const u32x4*>(static_cast<const float*>(w) + i + 4);
+  }
+  return r;
+}
+
+__device__ __forceinline__ void decode_w8(const WRaw& r, int dtype, float scale, float (&v)[8]) {
+  if (dtype == 2) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const auto x = __builtin_amdgcn_cvt_pk_f32_fp8((int)r.lo[h], false);
+      const auto y = __builtin_amdgcn_cvt_pk_f32_fp8((int)r.lo[h], true);
+      const uint32_t b0 = pack_bf16x2(x[0] * scale, x[1] * scale);
+      const uint32_t b1 = pack_bf16x2(y[0] * scale, y[1] * scale);
+      v[4 * h] = bf16_to_f32(b0 & 0xffffu);
+      v[4 * h + 1] = bf16_to_f32(b0 >> 16);
+      v[4 * h + 2] = bf16_to_f32(b1 & 0xffffu);
+      v[4 * h + 3] = bf16_to_f32(b1 >> 16);
+    }
+  } else if (dtype == 0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[2 * j] = bf16_to_f32(r.lo[j] & 0xffffu);
+      v[2 * j + 1] = bf16_to_f32(r.lo[j] >> 16);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[j] = __uint_as_float(r.lo[j]);
+      v[4 + j] = __uint_as_float(r.hi[j]);
+    }
+  }
+}
 
 // Workgroup: 64 x 64 outputs, 4 waves of 32 x 32. Per block of 32 k, A's 64
 // rows and B's 64 columns go to LDS k-contiguous ([row][k], B transposed:
-// [n][k]) with coalesced 16-byte loads (the projection is decoded on the
-// way); the next block's loads are in flight while the current block's 16
-// products per wave run from LDS. Rows and columns past the matrix are
-// staged from clamped real rows and not stored.
-template <bool EMBED>
+// [n][k]) with coalesced loads; two blocks are in registers or in flight
+// while the current block's 16 products per wave run from LDS. Rows and
+// columns past the matrix are staged from clamped real rows and not stored.
+// LDS row r is 8 chunks of four k, chunk c at c ^ swz(r), swz(r) = (r ^ r / 8)
+// mod 8: the 16-byte fragment reads, A's 16-byte stores and the 4-byte
+// transposed stores of B then spread over all banks.
+//
+// VEC (n_out % 8 == 0, aligned weights): a thread moves eight weights of one
+// k as one load and decodes them when it stores them. The element-wise form
+// (other shapes) loads and decodes each weight behind its own bounds check:
+// a block then waits for eight loads in turn. fp8, 384 x 128 projections:
+// 8 tiles x 8 heads 36.3 -> 15.3 us, 592 x 48 77.5 -> 46.5 us, 1,648 x 48
+// 213 -> 110 us (18 us and 51 us at the fp32 matrix rate for the last two;
+// what is left is one chain of 12 blocks per workgroup at ~1.2 us each and,
+// at 592 x 48, only 960 workgroups). Every embedding is the same bit for bit.
+template <bool EMBED, bool VEC>
 __global__ void __launch_bounds__(256) pgemm_kernel(PGemm p) {
-  __shared__ __attribute__((aligned(16))) float As[2][kBM][kRow];
-  __shared__ __attribute__((aligned(16))) float Bs[2][kBN][kRow];
+  __shared__ __attribute__((aligned(16))) float As[2][kBM][kKB];
+  __shared__ __attribute__((aligned(16))) float Bs[2][kBN][kKB];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int li = lane & 31, g = lane >> 5;
   const int64_t hp = blockIdx.z;
@@ -202,63 +262,73 @@ __global__ void __launch_bounds__(256) pgemm_kernel(PGemm p) {
     wscale = (p.w_dtype == 2 && head_ok) ? p.w_scale[head] : 1.f;
   }
   const int64_t wbase = head * p.k * p.n;
+  auto swz = [](int r) { return (r ^ (r >> 3)) & 7; };
   // staging: thread t moves k 4 (t % 8) .. + 3 of rows t / 8 and t / 8 + 32
   // of A (and of k_hat); for the projection, k t / 8 of columns 8 (t % 8) ..
   // + 7
-  const int sr = tid >> 3, sk = 4 * (tid & 7);
+  const int sr = tid >> 3, sc = tid & 7;
   struct Stage {
     f32x4 a[2], b[2];
     float w[8];
+    WRaw raw;
+    bool w_ok;
   };
   auto load = [&](Stage& st, int64_t k0) {
-    f32x4 (&ra)[2] = st.a;
-    f32x4 (&rb)[2] = st.b;
-    float (&rw)[8] = st.w;
-    const int64_t kk = k0 + sk;
+    const int64_t kk = k0 + 4 * sc;
+    const int64_t kc = min(kk, p.k - 4);  // past k: a real chunk, replaced by zeros
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int64_t gm = min(mb + sr + 32 * h, p.m - 1);
-      ra[h] = kk < p.k ? *reinterpret_cast<const f32x4*>(p.a + (hp * p.m + gm) * p.k + kk)
-                       : f32x4{0.f, 0.f, 0.f, 0.f};
+      st.a[h] = *reinterpret_cast<const f32x4*>(p.a + (hp * p.m + gm) * p.k + kc);
       if (!EMBED) {
         const int64_t gn = min(nb + sr + 32 * h, p.n - 1);
-        rb[h] = kk < p.k ? *reinterpret_cast<const f32x4*>(p.b + (hp * p.n + gn) * p.k + kk)
-                         : f32x4{0.f, 0.f, 0.f, 0.f};
+        st.b[h] = *reinterpret_cast<const f32x4*>(p.b + (hp * p.n + gn) * p.k + kc);
+      }
+      if (kk >= p.k) {
+        st.a[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (!EMBED) st.b[h] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
     }
-    if (EMBED) {
+    if (EMBED && VEC) {
+      const int64_t wk = k0 + sr, gn = nb + 8 * sc;
+      st.w_ok = wk < p.k && gn < p.n && head_ok;
+      st.raw = load_w8(p.w, p.w_dtype, wbase + min(wk, p.k - 1) * p.n + min(gn, p.n - 8));
+    } else if (EMBED) {
       const int64_t wk = k0 + sr;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const int64_t gn = nb + 8 * (tid & 7) + j;
-        rw[j] = (wk < p.k && gn < p.n && head_ok) ? load_w(p.w, p.w_dtype, wbase + wk * p.n + gn, wscale)
-                                                 : 0.f;
+        const int64_t gn = nb + 8 * sc + j;
+        st.w[j] = (wk < p.k && gn < p.n && head_ok)
+                      ? load_w(p.w, p.w_dtype, wbase + wk * p.n + gn, wscale) : 0.f;
       }
     }
   };
-  auto store = [&](const Stage& st, int buf) {
-    const f32x4 (&ra)[2] = st.a;
-    const f32x4 (&rb)[2] = st.b;
-    const float (&rw)[8] = st.w;
+  auto store = [&](Stage& st, int buf) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      *reinterpret_cast<f32x4*>(&As[buf][sr + 32 * h][sk]) = ra[h];
-      if (!EMBED) *reinterpret_cast<f32x4*>(&Bs[buf][sr + 32 * h][sk]) = rb[h];
+      const int at = 4 * (sc ^ swz(sr + 32 * h));
+      *reinterpret_cast<f32x4*>(&As[buf][sr + 32 * h][at]) = st.a[h];
+      if (!EMBED) *reinterpret_cast<f32x4*>(&Bs[buf][sr + 32 * h][at]) = st.b[h];
     }
     if (EMBED) {
+      if (VEC) decode_w8(st.raw, p.w_dtype, wscale, st.w);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) Bs[buf][8 * (tid & 7) + j][sr] = rw[j];
+      for (int j = 0; j < 8; ++j) {
+        const int col = 8 * sc + j;
+        Bs[buf][col][4 * ((sr >> 2) ^ swz(col)) + (sr & 3)] = !VEC || st.w_ok ? st.w[j] : 0.f;
+      }
     }
   };
   f32x16 acc;
 #pragma unroll
   for (int e = 0; e < 16; ++e) acc[e] = 0.f;
   const int nblk = (int)((p.k + kKB - 1) / kKB);
+  const int ra = wm + li, rb = wn + li;
   auto products = [&](int buf) {
 #pragma unroll
     for (int c = 0; c < kKB / 8; ++c) {
-      const f32x4 a = *reinterpret_cast<const f32x4*>(&As[buf][wm + li][8 * c + 4 * g]);
-      const f32x4 b = *reinterpret_cast<const f32x4*>(&Bs[buf][wn + li][8 * c + 4 * g]);
+      const f32x4 a = *reinterpret_cast<const f32x4*>(&As[buf][ra][4 * ((2 * c + g) ^ swz(ra))]);
+      const f32x4 b = *reinterpret_cast<const f32x4*>(&Bs[buf][rb][4 * ((2 * c + g) ^ swz(rb))]);
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], b[j], acc, 0, 0, 0);
     }
@@ -267,20 +337,20 @@ __global__ void __launch_bounds__(256) pgemm_kernel(PGemm p) {
   // in LDS being multiplied: the loads run two blocks ahead of their use
   Stage r0, r1;
   load(r0, 0);
+  load(r1, kKB);           // block 1 (zeros past k)
   store(r0, 0);
-  load(r0, kKB);           // block 1 (zeros past k)
-  load(r1, 2 * kKB);       // block 2
+  load(r0, 2 * kKB);       // block 2
   __syncthreads();
   for (int kb = 0; kb < nblk; kb += 2) {
     products(0);
     if (kb + 1 >= nblk) break;
-    store(r0, 1);          // block kb + 1
-    load(r0, (int64_t)(kb + 3) * kKB);
+    store(r1, 1);          // block kb + 1
+    load(r1, (int64_t)(kb + 3) * kKB);
     __syncthreads();
     products(1);
     if (kb + 2 >= nblk) break;
-    store(r1, 0);          // block kb + 2
-    load(r1, (int64_t)(kb + 4) * kKB);
+    store(r0, 0);          // block kb + 2
+    load(r0, (int64_t)(kb + 4) * kKB);
     __syncthreads();
   }
   // lane (li, g) holds column nb + wn + li, rows mb + wm + 8 (e / 4) + 4 g + e % 4
@@ -328,7 +398,11 @@ extern "C" int veda_predictor_embed(const float* feats, int64_t n_heads, int64_t
     p.a = feats; p.w = w; p.w_dtype = w_dtype; p.w_scale = w_scale; p.w_heads = w_heads;
     p.heads = heads; p.m = n_tiles; p.n = n_out; p.k = k_dim; p.residual = residual;
     p.out = out;
-    pgemm_kernel<true><<<grid, 256, 0, s>>>(p);
+    // whole groups of eight columns, each as one aligned load
+    if (n_out % 8 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0)
+      pgemm_kernel<true, true><<<grid, 256, 0, s>>>(p);
+    else
+      pgemm_kernel<true, false><<<grid, 256, 0, s>>>(p);
   } else {
     embed_kernel<<<grid, 256, 0, s>>>(feats, n_tiles, k_dim, w, w_dtype, w_scale, w_heads, heads,
                                       n_out, residual, out);
@@ -351,7 +425,7 @@ extern "C" int veda_predictor_logits(const float* a, const float* b, int64_t n_h
     PGemm p{};
     p.a = a; p.b = b; p.heads = heads; p.m = n_q; p.n = n_k; p.k = dim; p.scale = scale;
     p.gain = gain; p.log_count = log_count; p.accumulate = accumulate; p.out = out;
-    pgemm_kernel<false><<<grid, 256, 0, s>>>(p);
+    pgemm_kernel<false, true><<<grid, 256, 0, s>>>(p);
   } else {
     logits_kernel<<<grid, 256, 0, s>>>(a, b, n_q, n_k, dim, scale, gain, heads, log_count,
                                        accumulate, out);
