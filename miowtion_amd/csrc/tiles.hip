@@ -50,6 +50,8 @@ constexpr int kSlotsPerWave = kTile / kWaves;  // 32
 constexpr int kCopyWaves = 16;                 // waves of the plain gather and the scatter
 constexpr int kPoolUnroll = 4;                 // rows in flight per wave of the pooled gather
 constexpr int kPoolOccupancy = 8;              // its waves per SIMD (caps its registers)
+constexpr int kPoolSplit = 8;                  // waves per item where there are few items
+constexpr int64_t kPoolSplitItems = 2560;      // pool only: items from which one wave takes one
 
 struct Row8 {
   uint32_t w[4];  // 8 bf16 values
@@ -258,13 +260,30 @@ __device__ __forceinline__ void pool_keys(const Row8& r, s16x2* k_max, s16x2* k_
   }
 }
 
-// Gather with first-order pooling: one wave per (tile, group of heads),
-// over all 128 slots of the tile, so the pooled statistics stay in the
-// lane's registers (no cross-wave reduction, no barrier); the workgroup's
-// waves take consecutive head groups of one tile (adjacent bytes of each
-// source row).
-template <int D>
-__global__ void __launch_bounds__(64 * kWaves, kPoolOccupancy) pool_gather_kernel(
+// Gather with first-order pooling. Work item = (tile, group of heads).
+// SPLIT = 1: one wave per item, over all 128 slots of the tile, so the pooled
+// statistics stay in the lane's registers (no cross-wave reduction, no
+// barrier); the workgroup's waves take consecutive head groups of one tile
+// (adjacent bytes of each source row). SPLIT = kPoolSplit: the item's waves
+// take 16 slots each, all 16 rows in flight, and wave 0 reduces through LDS.
+//
+// Both forms add each 16-slot group's rows in order and then the groups in
+// order, so a head's statistics have the same bits whichever form the
+// launch takes (the heads of a layer may come in any chunks).
+//
+// The one-wave form is a serial chain of 32 dependent index and row loads
+// per wave, the split form one such round. us per launch, one wave / split:
+//   items              16          1,188        2,376        3,168        7,104
+//   pool only       25.8 / 7.2  43.1 / 24.1  51.3 / 44.4  63.2 / 69.7  136.5 / 145.0
+//   with the rows   30.9 / 9.4  71.6 / 55.4   123 / 102    170 / 142    343 / 297
+// (7,104 items: 57,720 rows x 48 heads, 5.65 TB/s with the rows). When the
+// rows are written as well, 16 rows in flight per wave and 8 waves on a
+// tile's 16 KB of adjacent output always win; the pooling alone is read
+// bandwidth, which fewer, longer waves hold a little better once there are
+// about ten items per CU, so it changes form there (kPoolSplitItems).
+template <int D, int SPLIT>
+__global__ void __launch_bounds__(SPLIT == 1 ? 64 * kWaves : 64 * SPLIT,
+                                  SPLIT == 1 ? kPoolOccupancy : 2) pool_gather_kernel(
     const uint16_t* __restrict__ x, int64_t x_rows, int64_t x_heads,
     int64_t xs, int64_t xh, const int64_t* __restrict__ gather_index,
     const int32_t* __restrict__ slot_valid,
@@ -273,10 +292,13 @@ __global__ void __launch_bounds__(64 * kWaves, kPoolOccupancy) pool_gather_kerne
     uint16_t* __restrict__ out, int64_t os, int64_t oh, float* __restrict__ feats) {
   constexpr int kChunks = D / 8;
   constexpr int kHeadsPerGroup = 64 / kChunks;
+  constexpr int kGroup = kTile / kPoolSplit;  // slots per partial sum
+  constexpr int kSlots = kTile / SPLIT;       // slots per wave
+  constexpr int kUnroll = SPLIT == 1 ? kPoolUnroll : kGroup;
   const int n_groups = (int)((n_heads + kHeadsPerGroup - 1) / kHeadsPerGroup);
-  const int64_t item =
-      (int64_t)blockIdx.x * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (item >= n_tiles * n_groups) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t item = SPLIT == 1 ? (int64_t)blockIdx.x * kWaves + wave : (int64_t)blockIdx.x;
+  if (item >= n_tiles * n_groups) return;  // SPLIT > 1: one workgroup per item, never taken
   const int64_t tile = item / n_groups;
   const int group = (int)(item % n_groups);
   const int lane = threadIdx.x & 63;
@@ -288,49 +310,82 @@ __global__ void __launch_bounds__(64 * kWaves, kPoolOccupancy) pool_gather_kerne
   // lanes of a missing head read head 0 of the row and keep zeros
   const int64_t lane_off = (src_head_ok ? head : 0) * xh + chunk * 8;
   const int count = valid_count[tile];
-  float s_sum[8];
+  const int first = SPLIT == 1 ? 0 : wave * kSlots;  // this wave's first slot of the tile
+  float s_sum[8], s_part[8];
   s16x2 k_max[4], k_min[4];  // order keys of the bf16 pairs
 #pragma unroll
-  for (int e = 0; e < 8; ++e) s_sum[e] = 0.f;
+  for (int e = 0; e < 8; ++e) s_sum[e] = s_part[e] = 0.f;
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
     k_max[w] = s16x2{-32768, -32768};
     k_min[w] = s16x2{32767, 32767};
   }
-  // 8 slots at a time; the slots before `count` are the tile's real rows
-  // (every layout puts them first): max / min over those, the sum over all
-  // (the padding rows are zero).
+  // kUnroll slots at a time; the slots before `count` are the tile's real
+  // rows (every layout puts them first): max / min over those, the sum over
+  // all (the padding rows are zero).
 #pragma unroll 1
-  for (int i0 = 0; i0 < kTile; i0 += kPoolUnroll) {
+  for (int i0 = first; i0 < first + kSlots; i0 += kUnroll) {
     // wave-uniform slots: the index reads are scalar loads, all issued first
-    int64_t src[kPoolUnroll];
-    bool ok[kPoolUnroll];
+    int64_t src[kUnroll];
+    bool ok[kUnroll];
 #pragma unroll
-    for (int j = 0; j < kPoolUnroll; ++j) {
+    for (int j = 0; j < kUnroll; ++j) {
       const int64_t slot = tile * kTile + i0 + j;
       src[j] = gather_index[slot];
       ok[j] = slot_valid[slot] != 0;
     }
-    Row8 r[kPoolUnroll];
+    Row8 r[kUnroll];
 #pragma unroll
-    for (int j = 0; j < kPoolUnroll; ++j) {
+    for (int j = 0; j < kUnroll; ++j) {
       r[j] = Row8{{0u, 0u, 0u, 0u}};
       if (ok[j] && src[j] >= 0 && src[j] < x_rows)
         r[j] = load_row8_nt(x + src[j] * xs + lane_off);
     }
     if (!src_head_ok) {
 #pragma unroll
-      for (int j = 0; j < kPoolUnroll; ++j) r[j] = Row8{{0u, 0u, 0u, 0u}};
+      for (int j = 0; j < kUnroll; ++j) r[j] = Row8{{0u, 0u, 0u, 0u}};
     }
 #pragma unroll
-    for (int j = 0; j < kPoolUnroll; ++j)
+    for (int j = 0; j < kUnroll; ++j)
       if (head_ok && out != nullptr)
         store_row8_nt(out + (tile * kTile + i0 + j) * os + hp * oh + chunk * 8, r[j]);
 #pragma unroll
-    for (int j = 0; j < kPoolUnroll; ++j) {
+    for (int j = 0; j < kUnroll; ++j) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) s_sum[e] += elem(r[j], e);
+      for (int e = 0; e < 8; ++e) s_part[e] += elem(r[j], e);
       if (i0 + j < count) pool_keys(r[j], k_max, k_min);  // wave-uniform branch
+    }
+    if (SPLIT == 1 && (i0 + kUnroll) % kGroup == 0) {  // the end of a 16-slot group
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        s_sum[e] += s_part[e];
+        s_part[e] = 0.f;
+      }
+    }
+  }
+  if constexpr (SPLIT > 1) {
+    __shared__ __attribute__((aligned(16))) uint32_t red[SPLIT][4][64][4];  // sums (2), max, min keys
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    auto put = [&](int part, uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+      *reinterpret_cast<u32x4_t*>(red[wave][part][lane]) = u32x4_t{a, b, c, d};
+    };
+    auto bits = [](float f) { return __float_as_uint(f); };
+    auto key = [](s16x2 v) { return __builtin_bit_cast(uint32_t, v); };
+    put(0, bits(s_part[0]), bits(s_part[1]), bits(s_part[2]), bits(s_part[3]));
+    put(1, bits(s_part[4]), bits(s_part[5]), bits(s_part[6]), bits(s_part[7]));
+    put(2, key(k_max[0]), key(k_max[1]), key(k_max[2]), key(k_max[3]));
+    put(3, key(k_min[0]), key(k_min[1]), key(k_min[2]), key(k_min[3]));
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int w = 0; w < SPLIT; ++w) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s_sum[e] += __uint_as_float(red[w][e >> 2][lane][e & 3]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        k_max[q] = __builtin_elementwise_max(k_max[q], __builtin_bit_cast(s16x2, red[w][2][lane][q]));
+        k_min[q] = __builtin_elementwise_min(k_min[q], __builtin_bit_cast(s16x2, red[w][3][lane][q]));
+      }
     }
   }
   if (!head_ok) return;
@@ -511,10 +566,17 @@ extern "C" int veda_gather_tiles(const void* x, int64_t x_rows, int64_t x_heads,
   gather_kernel<D, P, S2, W><<<grid, 64 * W, 0, s>>>(                                          \
       xx, x_rows, x_heads, x_stride_s, x_stride_h, gather_index, slot_valid, valid_count,      \
       n_tiles, heads, n_heads, oo, out_stride_s, out_stride_h, feats, sq, var)
-#define VEDA_POOL_GATHER(D)                                                                   \
-  pool_gather_kernel<D><<<(unsigned)((n_wg + kWaves - 1) / kWaves), 64 * kWaves, 0, s>>>(      \
+#define VEDA_POOL_FORM(D, SPLIT, GRID, THREADS)                                               \
+  pool_gather_kernel<D, SPLIT><<<(unsigned)(GRID), THREADS, 0, s>>>(                           \
       xx, x_rows, x_heads, x_stride_s, x_stride_h, gather_index, slot_valid, valid_count,      \
       n_tiles, heads, n_heads, oo, out_stride_s, out_stride_h, feats)
+#define VEDA_POOL_GATHER(D)                                                                   \
+  do {                                                                                        \
+    if (out != nullptr || n_wg < kPoolSplitItems)                                             \
+      VEDA_POOL_FORM(D, kPoolSplit, n_wg, 64 * kPoolSplit);                                   \
+    else                                                                                      \
+      VEDA_POOL_FORM(D, 1, (n_wg + kWaves - 1) / kWaves, 64 * kWaves);                        \
+  } while (0)
   if (head_dim == 128) {
     if (!feats) VEDA_GATHER(128, false, false, kCopyWaves);
     else if (!sq) VEDA_POOL_GATHER(128);
@@ -526,6 +588,7 @@ extern "C" int veda_gather_tiles(const void* x, int64_t x_rows, int64_t x_heads,
   }
 #undef VEDA_GATHER
 #undef VEDA_POOL_GATHER
+#undef VEDA_POOL_FORM
   return check_launch("veda_gather_tiles");
 }
 

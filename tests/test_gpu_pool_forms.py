@@ -1,0 +1,47 @@
+"""The pooled gather's two forms (one wave per tile and head group, or the
+tile's slots split over waves) give the same bits: a launch of few heads or
+tiles takes one form, a launch of many the other, and a layer's heads come in
+any chunks. Heads that do not fill a group, partial tiles, both head_dims."""
+
+import pytest
+import torch
+
+from miowtion_amd import kernels
+from oracle import predictor as op
+from oracle import tiling as ot
+from tests import helpers
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('dim', [64, 128])
+@pytest.mark.parametrize('heads', [1, 3, 5])
+def test_pooling_matches_oracle_and_written_rows_change_nothing(dim, heads):
+    spec = helpers.small_layout()
+    lay, olay = helpers.product_layout(*spec, device='cuda'), helpers.oracle_layout(*spec)
+    x, = helpers.qkv(lay.seq_len, heads, dim, seed=heads, n=1)
+    tiles, feats = kernels.gather_and_pool(x.cuda(), lay, None)
+    alone, = kernels.pool_seq(x.cuda(), lay, None)
+    assert torch.equal(feats, alone)
+    want = ot.gather_tiles(x, olay, None)
+    assert torch.equal(tiles.cpu(), want)
+    pooled = op.pool_tiles(want, olay)
+    got = feats.cpu()
+    assert torch.equal(got[..., dim:], pooled[..., dim:])
+    # 128 fp32 additions of values below 5: 128 * 2^-24 * 5 per element of a mean
+    torch.testing.assert_close(got[..., :dim], pooled[..., :dim], rtol=0, atol=128 * 5 * 2.0 ** -24)
+
+
+def test_head_chunks_keep_the_bits():
+    """440 tiles x 28 heads pool as 3,080 items (one wave each); a chunk of
+    four heads as 440 (split), and the rows written along with them split."""
+    spec = ([(0, (40, 22, 64))], 56320, 56320, '4x2x16')
+    lay = helpers.product_layout(*spec, device='cuda')
+    x = torch.randn(56320, 28, 128, generator=torch.Generator('cuda').manual_seed(1),
+                    device='cuda').to(torch.bfloat16)
+    heads = torch.arange(28, device='cuda')
+    assert lay.n_tiles * 28 // 4 > 2560 > lay.n_tiles
+    whole, = kernels.pool_seq(x, lay, heads)
+    parts = torch.cat([kernels.pool_seq(x, lay, h)[0] for h in heads.split(4)])
+    assert torch.equal(whole, parts)
+    assert torch.equal(whole, kernels.gather_and_pool(x, lay, heads)[1])
