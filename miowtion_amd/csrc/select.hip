@@ -8,11 +8,16 @@
 // lane-strided so every LDS access is conflict-free. k_hi rounds of a
 // wave-wide max over the lanes' current heads extract the winners in
 // descending order; the winning lane's next head is one LDS read. The
-// rounds are a latency chain, so occupancy is what the kernel runs on: the
-// LDS holds only the row's columns (dynamic size, 20 KB per workgroup at
-// 592 columns: 8 workgroups per CU instead of the 2 a 2048-column array
-// allows). Folding the column into the key makes every key distinct, so the
-// order is total: higher score first, lower column first on equal scores.
+// rounds are what the kernel spends its time on, so the LDS holds only the
+// row's columns (dynamic size, 20 KB per workgroup at 592 columns: 8
+// workgroups per CU instead of the 2 a 2048-column array allows), and a
+// round takes the max of the 32-bit score keys alone (about a third of the
+// instructions of a max over the 64-bit keys); only when several lanes hold
+// the same score does a second max pick the lowest column (48 heads x 592
+// columns, k_hi 35: 112 -> 79 us; x 1,632, k_hi 48: 842 -> 750, most of it
+// the sort of 32 keys).
+// The order is total: higher score first, lower column first on equal
+// scores.
 //
 // Lists: one wave per (head, row), 64 columns per step, positions from a
 // ballot + popcount prefix (no sort, no atomics).
@@ -38,37 +43,20 @@ __device__ __forceinline__ uint32_t orderable(float v) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-template <int CTRL>
-__device__ __forceinline__ uint64_t dpp_u64(uint64_t v) {
-  const uint32_t lo = __builtin_amdgcn_update_dpp(0u, (uint32_t)v, CTRL, 0xF, 0xF, false);
-  const uint32_t hi = __builtin_amdgcn_update_dpp(0u, (uint32_t)(v >> 32), CTRL, 0xF, 0xF, false);
-  return ((uint64_t)hi << 32) | lo;
-}
-
-__device__ __forceinline__ uint64_t max_u64(uint64_t a, uint64_t b) { return a > b ? a : b; }
-
-// Max over the 64 lanes, wave-uniform. Within a 16-lane row: DPP exchanges
-// with lane ^ 1, lane ^ 2, the mirror inside 8 and the mirror inside 16;
-// across rows: a swizzle with lane ^ 16, then v_permlane32_swap with the
-// lane 32 positions away (it leaves {own, partner} in its two results, in
-// the same order for both halves of the key).
-__device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
-  v = max_u64(v, dpp_u64<0xB1>(v));   // quad_perm [1, 0, 3, 2]
-  v = max_u64(v, dpp_u64<0x4E>(v));   // quad_perm [2, 3, 0, 1]
-  v = max_u64(v, dpp_u64<0x141>(v));  // row_half_mirror
-  v = max_u64(v, dpp_u64<0x140>(v));  // row_mirror
-  {
-    const uint32_t lo = __builtin_amdgcn_ds_swizzle((uint32_t)v, 0x401F);
-    const uint32_t hi = __builtin_amdgcn_ds_swizzle((uint32_t)(v >> 32), 0x401F);
-    v = max_u64(v, ((uint64_t)hi << 32) | lo);
-  }
-  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
-  const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(v >> 32), (uint32_t)(v >> 32),
-                                                   false, false);
-  v = max_u64(((uint64_t)hi[0] << 32) | lo[0], ((uint64_t)hi[1] << 32) | lo[1]);
-  const uint32_t ulo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-  const uint32_t uhi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return ((uint64_t)uhi << 32) | ulo;
+// Max over the 64 lanes of a 32-bit key, wave-uniform. Within a 16-lane row:
+// DPP exchanges with lane ^ 1, lane ^ 2, the mirror inside 8 and the mirror
+// inside 16 (each folds into its v_max_u32); across rows: the row 16 lanes
+// away, then the lane 32 positions away (the swaps leave {own, partner} in
+// their two results, in either order).
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0u, v, 0xB1, 0xF, 0xF, false));   // quad_perm
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0u, v, 0x4E, 0xF, 0xF, false));   // quad_perm
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0u, v, 0x141, 0xF, 0xF, false));  // half mirror
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0u, v, 0x140, 0xF, 0xF, false));  // mirror
+  const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = max(a[0], a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)max(b[0], b[1]));
 }
 
 constexpr int kMaxCols = 2048;  // columns of one block (FA4's 2048-block cap)
@@ -129,23 +117,29 @@ __global__ void __launch_bounds__(256) select_topk_kernel(
 #pragma unroll
   for (int j = 0; j < N; ++j)
     if (j < per_lane) kv[j * 64 + lane] = k[j];
-  uint64_t best = k[0];
+  uint32_t best = (uint32_t)(k[0] >> 32);  // score key and column of this lane's head
+  uint32_t col = ~(uint32_t)k[0];
   int pos = 0;  // index of this lane's current head in its sorted list
   const bool has_extra = tile_id >= 0 && tile_id < n_extra && extra[tile_id] != 0;
   const int allowed = k_lo + (has_extra ? 1 : 0);
   int64_t* irow = index + h * osh + r * osr + col0;
   uint8_t* krow = keep + h * osh + r * osr + col0;
   for (int t = 0; t < k_hi; ++t) {
-    const uint64_t top = wave_max_u64(best);
-    const uint32_t c = ~(uint32_t)top;
-    const uint32_t vkey = (uint32_t)(top >> 32);
-    if ((int)(c & 63) == lane) {
-      irow[t] = block_start + (int64_t)c;
+    const uint32_t top = wave_max_u32(best);
+    uint64_t at = __ballot(best == top);
+    if (at & (at - 1)) {  // equal scores in several lanes: the lowest column (wave-uniform branch)
+      const uint32_t c = wave_max_u32(best == top ? ~col : 0u);
+      at = __ballot(best == top && ~col == c);
+    }
+    if (lane == __builtin_ctzll(at)) {
+      irow[t] = block_start + (int64_t)col;
       // kept: within the row's budget and `val > -inf` (False for NaN,
       // mask.py:251-284)
-      krow[t] = (t < allowed && vkey > kNegInfKey && vkey != kNaNKey) ? 1 : 0;
+      krow[t] = (t < allowed && top > kNegInfKey && top != kNaNKey) ? 1 : 0;
       ++pos;
-      best = pos < per_lane ? kv[pos * 64 + lane] : 0;
+      const uint64_t next = pos < per_lane ? kv[pos * 64 + lane] : 0;
+      best = (uint32_t)(next >> 32);
+      col = ~(uint32_t)next;
     }
   }
 }
