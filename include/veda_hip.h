@@ -94,7 +94,7 @@ int veda_gather_lse(const float* lse, int64_t lse_rows, int64_t lse_heads,
  * Top-k of one column block of the video quadrant (rule 'topk').
  * Replaces the per-block body of miowtion/veda/mask.py:251-284.
  *
- * For every head h and selection row r (video tile id rows[r]):
+ * For every head h and selection row r (video tile id rows[r]; rows NULL: r):
  *   s[c] = scores[h, r, block_start + c] for c in [0, n_cols),
  *   s[c] = -inf where kv_ok[block_start + c] == 0,
  *   s[rows[r] - block_start] = +inf when rows[r] lies in the block,
@@ -139,6 +139,33 @@ int veda_index_lists(const uint8_t* block_mask, int64_t n_heads,
                      const uint8_t* full_tile, int32_t* part_cnt,
                      int32_t* part_idx, int32_t* full_cnt, int32_t* full_idx,
                      void* stream);
+
+/*
+ * veda_index_lists of veda_dense_block_mask (global_rows) of a selection of
+ * all n_video video rows, without the mask: index / keep
+ * [n_heads, n_video, k_total] contiguous, n_tiles at most 4096; the lists of
+ * all n_tiles rows (miowtion/veda/mask.py:288-317, kernels/fa4.py:266-296).
+ */
+int veda_selection_lists(const int64_t* index, const uint8_t* keep,
+                         int64_t n_heads, int64_t n_video, int64_t k_total,
+                         const uint8_t* kv_ok, const uint8_t* full_tile,
+                         int64_t n_tiles, int32_t* part_cnt, int32_t* part_idx,
+                         int32_t* full_cnt, int32_t* full_idx, void* stream);
+
+/*
+ * The Q-direction lists of a block mask [n_heads, n_rows, n_tiles]
+ * (miowtion/kernels/fa4.py:282-296): row = key tile j, entries = the query
+ * tiles r with mask[h, r, j] & kv_ok[j], ascending, then the others; all in
+ * the full list where full_tile[j], else all in the partial one (the other
+ * list has count 0). *_cnt [n_heads, n_tiles], *_idx [n_heads, n_tiles,
+ * n_rows].
+ */
+int veda_index_lists_t(const uint8_t* block_mask, int64_t n_heads,
+                       int64_t n_rows, int64_t n_tiles, const uint8_t* kv_ok,
+                       const uint8_t* full_tile, int32_t* part_cnt,
+                       int32_t* part_idx, int32_t* full_cnt, int32_t* full_idx,
+                       void* stream);
+
 
 /*
  * Block-sparse attention forward on tile-ordered rows.

@@ -31,6 +31,8 @@ SIGNATURES: dict[str, list] = {
                          _I, _I, _I, _P],
     'veda_dense_block_mask': [_P, _P, _I, _I, _I, _P, _I, _I, _C, _P, _P],
     'veda_index_lists': [_P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P],
+    'veda_selection_lists': [_P, _P, _I, _I, _I, _P, _P, _I, _P, _P, _P, _P, _P],
+    'veda_index_lists_t': [_P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P],
     'veda_block_sparse_fwd': [_P, _I, _I, _P, _I, _I, _P, _I, _I, _I, _I, _I, _I,
                               _P, _P, _P, _P, _I, _P, _F, _P, _I, _I, _P, _I, _I, _I, _P],
     'veda_block_sparse_fwd_seq': [_P, _I, _I, _I, _I, _P, _P, _P, _P, _I, _P, _I, _I, _P, _I, _I,

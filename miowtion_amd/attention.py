@@ -243,18 +243,20 @@ class SparseStudent:
             logits = pred.layers[layer_index](feats_q, feats_k, heads, **extra)
             selection = veda_mask.select_video_blocks(
                 logits[:, :tile_layout.n_video_tiles], tile_layout, self.clip.blocks(tile_layout))
-            block_mask = veda_mask.dense_block_mask(selection, tile_layout)
-            lists = kernels.index_lists(block_mask, tile_layout)
             if compensated:
+                block_mask = veda_mask.dense_block_mask(selection, tile_layout)
+                lists = kernels.index_lists(block_mask, tile_layout)
                 # the lists already hold only kv_ok tiles (index_lists applies it)
                 o_tiles = kernels.compensated_attention(q_tiles, k_tiles, v_tiles, block_mask,
                                                         tile_layout, lists)
                 kernels.scatter_tiles_(out, o_tiles, tile_layout, heads)
-            elif kv_seq:
-                kernels.block_sparse_attention_seq_kv_(out, q, k, v, lists, tile_layout, heads)
             else:
-                kernels.block_sparse_attention_seq_(out, q, k_tiles, v_tiles, lists, tile_layout,
-                                                    heads)
+                lists = kernels.selection_lists(selection, tile_layout)
+                if kv_seq:
+                    kernels.block_sparse_attention_seq_kv_(out, q, k, v, lists, tile_layout, heads)
+                else:
+                    kernels.block_sparse_attention_seq_(out, q, k_tiles, v_tiles, lists,
+                                                        tile_layout, heads)
         self.last.setdefault('parts', []).append(
             dict(shape=tile_layout, heads=heads, selection=selection, lists=lists,
                  logits=logits))

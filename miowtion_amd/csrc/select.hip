@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(256) select_topk_kernel(
   const int64_t item = (int64_t)blockIdx.x * kSelWaves + wave;
   if (item >= n_heads * n_rows) return;  // whole wave exits together
   const int64_t h = item / n_rows, r = item % n_rows;
-  const int64_t tile_id = rows[r];
+  const int64_t tile_id = rows != nullptr ? rows[r] : r;
   const int64_t diag = tile_id - block_start;  // column of the own tile, if in block
   const float* srow = scores + h * ssh + r * ssr + block_start;
   const int per_lane = (n_cols + 63) / 64;
@@ -204,6 +204,172 @@ __device__ __forceinline__ void stage_classes(const uint8_t* __restrict__ m,
   counts = nf | (np << 16);  // both at most 4096
 }
 
+// The lists of one row whose classes are in `cls` (this wave's LDS row), NF
+// full and NP partial members.
+__device__ __forceinline__ void write_lists(const uint8_t* cls, int n_tiles, int lane, int NF,
+                                            int NP, int32_t* __restrict__ fi,
+                                            int32_t* __restrict__ pi) {
+  const uint64_t below = (1ull << lane) - 1ull;
+  int nf = 0, np = 0;  // members before the chunk
+  for (int c0 = 0; c0 < n_tiles; c0 += 64) {
+    const int c = c0 + lane;
+    const int k = c < n_tiles ? cls[c] : 0;
+    const uint64_t bf = __ballot(k == 1), bp = __ballot(k == 2);
+    const int rf = __popcll(bf & below), rp = __popcll(bp & below);
+    if (c < n_tiles) {
+      fi[k == 1 ? nf + rf : NF + (c0 - nf) + (lane - rf)] = c;
+      pi[k == 2 ? np + rp : NP + (c0 - np) + (lane - rp)] = c;
+    }
+    nf += __popcll(bf);
+    np += __popcll(bp);
+  }
+}
+
+// Orders this wave's LDS accesses before it against those after it.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// index_lists of dense_block_mask(selection) without the mask: one wave per
+// (head, row of all n_tiles tiles). A video row's members are its kept
+// columns and the global columns, a global row's every column, each where
+// kv_ok. Against the two kernels it saves writing and reading the mask and a
+// launch: 25 + 32 -> 35 us at 48 heads x 592 x 592, 95 + 284 -> 224 us at
+// 1,648 x 1,648 (4.7 TB/s of list entries written).
+__global__ void __launch_bounds__(64 * kListWaves) selection_lists_kernel(
+    const int64_t* __restrict__ index, const uint8_t* __restrict__ keep, int64_t n_items,
+    int64_t k_total, const uint8_t* __restrict__ kv_ok, const uint8_t* __restrict__ full_tile,
+    int n_tiles, int n_video, int32_t* __restrict__ part_cnt, int32_t* __restrict__ part_idx,
+    int32_t* __restrict__ full_cnt, int32_t* __restrict__ full_idx) {
+  __shared__ __align__(16) uint8_t cls_lds[kListWaves][kListCols];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int64_t item = (int64_t)blockIdx.x * kListWaves + wave;
+  if (item >= n_items) return;  // each wave uses only its own LDS row
+  const int64_t h = item / n_tiles, r = item % n_tiles;
+  const bool video_row = r < n_video;
+  uint8_t* cls = cls_lds[wave];
+  for (int c = lane; c < n_tiles; c += 64)
+    cls[c] = (!video_row || c >= n_video) && kv_ok[c] ? (full_tile[c] ? 1 : 2) : 0;
+  if (video_row) {
+    wave_lds_sync();
+    const int64_t base = (h * n_video + r) * k_total;
+    for (int64_t t = lane; t < k_total; t += 64) {
+      const int64_t c = index[base + t];
+      if (keep[base + t] && c >= 0 && c < n_tiles && kv_ok[c]) cls[c] = full_tile[c] ? 1 : 2;
+    }
+  }
+  wave_lds_sync();
+  int NF = 0, NP = 0;
+  for (int c0 = 0; c0 < n_tiles; c0 += 64) {
+    const int k = c0 + lane < n_tiles ? cls[c0 + lane] : 0;
+    NF += __popcll(__ballot(k == 1));
+    NP += __popcll(__ballot(k == 2));
+  }
+  write_lists(cls, n_tiles, lane, NF, NP, full_idx + item * n_tiles, part_idx + item * n_tiles);
+  if (lane == 0) {
+    full_cnt[item] = NF;
+    part_cnt[item] = NP;
+  }
+}
+
+// Transposed lists (row = key tile, entries = its query tiles; all members
+// in the full or all in the partial list, by the key tile's own fullness).
+// Workgroup = (head, 64 key tiles). The mask's 64 columns come in as one
+// 64-bit word per query row (a ballot over one coalesced 64-byte read), a
+// chunk of rows at a time in LDS; a ballot over 64 rows' words at one
+// column's bit then is that column's membership, from which every store of
+// a list row is 64 consecutive entries. One launch in place of a transposed
+// copy, a list kernel and four selects: at 48 heads x 592 x 592 about 195 us
+// in eight launches -> 64 us.
+constexpr int kTransThreads = 512;
+constexpr int kTransRows = 4096;  // rows staged at a time
+
+__global__ void __launch_bounds__(kTransThreads) index_lists_t_kernel(
+    const uint8_t* __restrict__ mask, int n_rows, int n_cols, const uint8_t* __restrict__ kv_ok,
+    const uint8_t* __restrict__ full_tile, int32_t* __restrict__ part_cnt,
+    int32_t* __restrict__ part_idx, int32_t* __restrict__ full_cnt,
+    int32_t* __restrict__ full_idx) {
+  __shared__ uint64_t words[kTransRows];
+  constexpr int kWaves = kTransThreads / 64, kColsPerWave = 64 / kWaves;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int groups = (n_cols + 63) / 64;
+  const int64_t h = blockIdx.x / groups;
+  const int c0 = (int)(blockIdx.x % groups) * 64;
+  const int c = c0 + lane;
+  const bool col_ok = c < n_cols && kv_ok[c];
+  const uint8_t* m = mask + h * n_rows * n_cols + c;
+  const int chunks = (n_rows + kTransRows - 1) / kTransRows;
+  // the words of rows [r0, r0 + kTransRows) (zero past the last row)
+  auto stage = [&](int r0) {
+    const int end = min(n_rows - r0, kTransRows), padded = (end + 63) & ~63;
+#pragma unroll 8
+    for (int r = wave; r < padded; r += kWaves) {
+      const bool in = r < end && col_ok && m[(int64_t)(r0 + r) * n_cols] != 0;
+      const uint64_t w = __ballot(in);
+      if (lane == 0) words[r] = w;
+    }
+    __syncthreads();
+  };
+  int total[kColsPerWave];
+#pragma unroll
+  for (int i = 0; i < kColsPerWave; ++i) total[i] = 0;
+  for (int k = 0; k < chunks; ++k) {
+    if (k > 0) __syncthreads();  // the previous chunk's words are read
+    stage(k * kTransRows);
+    for (int r = lane; r - lane < min(n_rows - k * kTransRows, kTransRows); r += 64) {
+      const uint64_t w = words[r];
+#pragma unroll
+      for (int i = 0; i < kColsPerWave; ++i)
+        total[i] += __popcll(__ballot((w >> (wave * kColsPerWave + i)) & 1));
+    }
+  }
+  int seen[kColsPerWave];
+#pragma unroll
+  for (int i = 0; i < kColsPerWave; ++i) seen[i] = 0;
+  const uint64_t below = (1ull << lane) - 1ull;
+  for (int k = 0; k < chunks; ++k) {
+    if (chunks > 1) {
+      __syncthreads();
+      stage(k * kTransRows);
+    }
+    const int r0 = k * kTransRows;
+    for (int r = lane; r - lane < min(n_rows - r0, kTransRows); r += 64) {
+      const uint64_t w = words[r];
+      const int at = r0 + r;
+#pragma unroll
+      for (int i = 0; i < kColsPerWave; ++i) {
+        const int col = c0 + wave * kColsPerWave + i;  // wave-uniform
+        if (col >= n_cols) break;
+        const bool in = (w >> (wave * kColsPerWave + i)) & 1;
+        const uint64_t b = __ballot(in);
+        const int64_t row = (h * n_cols + col) * n_rows;
+        const bool full = full_tile[col] != 0;
+        int32_t* list = (full ? full_idx : part_idx) + row;
+        int32_t* other = (full ? part_idx : full_idx) + row;
+        if (at < n_rows) {
+          const int before = seen[i] + __popcll(b & below);  // members before this row
+          list[in ? before : total[i] + at - before] = at;
+          other[at] = at;
+        }
+        seen[i] += __popcll(b);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kColsPerWave; ++i) {
+    const int col = c0 + wave * kColsPerWave + i;
+    if (col < n_cols && lane == 0) {
+      const bool full = full_tile[col] != 0;
+      full_cnt[h * n_cols + col] = full ? total[i] : 0;
+      part_cnt[h * n_cols + col] = full ? 0 : total[i];
+    }
+  }
+}
+
 __global__ void __launch_bounds__(64 * kListWaves) index_lists_kernel(
     const uint8_t* __restrict__ mask, int64_t n_items, int n_tiles, int vec,
     const uint8_t* __restrict__ kv_ok, const uint8_t* __restrict__ full_tile,
@@ -230,23 +396,8 @@ __global__ void __launch_bounds__(64 * kListWaves) index_lists_kernel(
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) counts += __shfl_xor(counts, off);
     const int NF = counts & 0xffff, NP = counts >> 16;
-    // the lanes' LDS stores are seen by the other lanes of this wave
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    int nf = 0, np = 0;  // members before the chunk
-    for (int c0 = 0; c0 < n_tiles; c0 += 64) {
-      const int c = c0 + lane;
-      const int k = c < n_tiles ? cls[c] : 0;
-      const uint64_t bf = __ballot(k == 1), bp = __ballot(k == 2);
-      const int rf = __popcll(bf & below), rp = __popcll(bp & below);
-      if (c < n_tiles) {
-        fi[k == 1 ? nf + rf : NF + (c0 - nf) + (lane - rf)] = c;
-        pi[k == 2 ? np + rp : NP + (c0 - np) + (lane - rp)] = c;
-      }
-      nf += __popcll(bf);
-      np += __popcll(bp);
-    }
+    wave_lds_sync();  // the lanes' LDS stores are seen by the other lanes of this wave
+    write_lists(cls, n_tiles, lane, NF, NP, fi, pi);
     if (lane == 0) {
       full_cnt[item] = NF;
       part_cnt[item] = NP;
@@ -361,4 +512,40 @@ extern "C" int veda_index_lists(const uint8_t* block_mask, int64_t n_heads, int6
                        s>>>(block_mask, items, (int)n_tiles, vec, kv_ok, full_tile, part_cnt,
                             part_idx, full_cnt, full_idx);
   return check_launch("veda_index_lists");
+}
+
+extern "C" int veda_selection_lists(const int64_t* index, const uint8_t* keep, int64_t n_heads,
+                                    int64_t n_video, int64_t k_total, const uint8_t* kv_ok,
+                                    const uint8_t* full_tile, int64_t n_tiles, int32_t* part_cnt,
+                                    int32_t* part_idx, int32_t* full_cnt, int32_t* full_idx,
+                                    void* stream) {
+  VEDA_REQUIRE(n_tiles >= 1 && n_tiles <= kListCols, "selection_lists: n_tiles %lld not in [1, %d]",
+               (long long)n_tiles, kListCols);
+  VEDA_REQUIRE(n_video >= 0 && n_video <= n_tiles, "selection_lists: n_video %lld outside [0, %lld]",
+               (long long)n_video, (long long)n_tiles);
+  VEDA_REQUIRE(n_heads >= 0 && k_total >= 0, "selection_lists: negative size");
+  const int64_t items = n_heads * n_tiles;
+  if (items == 0) return VEDA_OK;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  selection_lists_kernel<<<(unsigned)((items + kListWaves - 1) / kListWaves), 64 * kListWaves, 0,
+                           s>>>(index, keep, items, k_total, kv_ok, full_tile, (int)n_tiles,
+                                (int)n_video, part_cnt, part_idx, full_cnt, full_idx);
+  return check_launch("veda_selection_lists");
+}
+
+extern "C" int veda_index_lists_t(const uint8_t* block_mask, int64_t n_heads, int64_t n_rows,
+                                  int64_t n_tiles, const uint8_t* kv_ok, const uint8_t* full_tile,
+                                  int32_t* part_cnt, int32_t* part_idx, int32_t* full_cnt,
+                                  int32_t* full_idx, void* stream) {
+  VEDA_REQUIRE(n_tiles >= 1 && n_tiles < (1ll << 31) && n_rows >= 0 && n_rows < (1ll << 31) - 64 &&
+                   n_heads >= 0,
+               "index_lists_t: bad sizes");
+  const int64_t groups = n_heads * ((n_tiles + 63) / 64);
+  VEDA_REQUIRE(groups < (1ll << 31), "index_lists_t: too many heads x key tiles for one launch");
+  if (groups == 0) return VEDA_OK;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  index_lists_t_kernel<<<(unsigned)groups, kTransThreads, 0, s>>>(
+      block_mask, (int)n_rows, (int)n_tiles, kv_ok, full_tile, part_cnt, part_idx, full_cnt,
+      full_idx);
+  return check_launch("veda_index_lists_t");
 }

@@ -146,15 +146,19 @@ def index_lists(block_mask: torch.Tensor, layout: tiling.TileLayout,
         return tuple(ops.index_lists(block_mask, layout.kv_ok, layout.full_tile))
     if block_mask.shape[1] != layout.n_tiles:
         raise ValueError('transposed lists need the block mask of all query tiles')
-    mt = (block_mask & layout.kv_ok[None, None, :]).transpose(1, 2).contiguous()
-    ones = torch.ones(mt.shape[2], dtype=torch.bool, device=mt.device)
-    # with every column "full", each row's members land in the full list
-    empty_cnt, empty_idx, cnt, idx = ops.index_lists(mt, ones, ones)
-    full_row = layout.full_tile.to(mt.device)[None, None, :]
-    return (torch.where(full_row, empty_cnt, cnt),
-            torch.where(full_row[..., None], empty_idx, idx).contiguous(),
-            torch.where(full_row, cnt, empty_cnt),
-            torch.where(full_row[..., None], idx, empty_idx).contiguous())
+    return tuple(ops.index_lists_t(block_mask, layout.kv_ok, layout.full_tile))
+
+
+def selection_lists(selection, layout: tiling.TileLayout) -> tuple[torch.Tensor, ...]:
+    """index_lists(mask.dense_block_mask(selection, layout), layout) for a
+    selection of all video rows, without the mask where the kernel takes the
+    row length."""
+    if layout.n_tiles > ops.SELECTION_LISTS_MAX_TILES:
+        block_mask = ops.dense_block_mask(selection.index, selection.keep, layout.kv_ok,
+                                          layout.n_video_tiles, True)
+        return index_lists(block_mask, layout)
+    return tuple(ops.selection_lists(selection.index, selection.keep, layout.kv_ok,
+                                     layout.full_tile, layout.n_video_tiles))
 
 
 def _front_tiles(layout: tiling.TileLayout, rows: int) -> int:

@@ -131,9 +131,7 @@ def select_video_blocks(scores: torch.Tensor, layout: tiling.TileLayout,
     heads = scores.shape[0]
     n_video = layout.n_video_tiles
     device = scores.device
-    if rows is None:
-        rows = torch.arange(n_video, device=device)
-    num_rows = rows.numel()
+    num_rows = n_video if rows is None else rows.numel()
     if scores.shape[1] != num_rows:
         raise ValueError(f'scores has {scores.shape[1]} query rows but rows has {num_rows}; '
                          'index the query axis by `rows` before calling')
@@ -150,7 +148,8 @@ def select_video_blocks(scores: torch.Tensor, layout: tiling.TileLayout,
     scores32 = scores if scores.dtype == torch.float32 else scores.float()
     if scores32.stride(-1) != 1:
         scores32 = scores32.contiguous()
-    rows = rows.to(device=device, dtype=torch.int64).contiguous()
+    if rows is not None:
+        rows = rows.to(device=device, dtype=torch.int64).contiguous()
     col0 = 0
     for block, width in zip(blocks, widths):
         n_cols = block.stop - block.start

@@ -143,9 +143,10 @@ def _(lse, gather_index, slot_valid, heads):
 
 @torch.library.custom_op('veda::select_topk', mutates_args=('index', 'keep'))
 def select_topk(scores: torch.Tensor, block_start: int, n_cols: int, kv_ok: torch.Tensor,
-                rows: torch.Tensor, k_lo: int, k_hi: int, extra: torch.Tensor,
+                rows: torch.Tensor | None, k_lo: int, k_hi: int, extra: torch.Tensor,
                 index: torch.Tensor, keep: torch.Tensor, col0: int) -> None:
-    """One column block of the top-k; writes index/keep[:, :, col0:col0+k_hi]."""
+    """One column block of the top-k; writes index/keep[:, :, col0:col0+k_hi].
+    rows: the video tile of every score row; None: row r is tile r."""
     _require_gpu(scores, kv_ok, rows, extra, index, keep)
     if scores.dtype != torch.float32 or scores.stride(-1) != 1:
         raise ValueError('scores must be fp32 with contiguous columns')
@@ -155,7 +156,7 @@ def select_topk(scores: torch.Tensor, block_start: int, n_cols: int, kv_ok: torc
         raise ValueError('scores has fewer columns than the block needs')
     _native.call('veda_select_topk', scores.data_ptr(), scores.shape[0], scores.shape[1],
                  scores.stride(0), scores.stride(1), block_start, n_cols, kv_ok.data_ptr(),
-                 rows.data_ptr(), k_lo, k_hi, extra.data_ptr(), extra.numel(), index.data_ptr(),
+                 _p(rows), k_lo, k_hi, extra.data_ptr(), extra.numel(), index.data_ptr(),
                  keep.data_ptr(), index.stride(0), index.stride(1), col0, _stream(scores))
 
 
@@ -212,6 +213,69 @@ def _(block_mask, kv_ok, full_tile):
     c = block_mask.new_empty(1, h, r, dtype=torch.int32)
     i = block_mask.new_empty(1, h, r, n, dtype=torch.int32)
     return [c, i, c.clone(), i.clone()]
+
+
+def _empty_lists(heads: int, rows: int, cols: int, device) -> list[torch.Tensor]:
+    """Uninitialised [part_cnt, part_idx, full_cnt, full_idx]."""
+    cnt, idx = (1, heads, rows), (1, heads, rows, cols)
+    return [torch.empty(s, dtype=torch.int32, device=device) for s in (cnt, idx, cnt, idx)]
+
+
+@torch.library.custom_op('veda::index_lists_t', mutates_args=())
+def index_lists_t(block_mask: torch.Tensor, kv_ok: torch.Tensor,
+                  full_tile: torch.Tensor) -> list[torch.Tensor]:
+    """The Q-direction lists of a block mask [H', R, n] (fa4.py:282-296):
+    rows are key tiles, entries query tiles; cnt [1, H', n] and idx
+    [1, H', n, R] int32, in index_lists' order."""
+    _require_gpu(block_mask, kv_ok, full_tile)
+    if block_mask.dtype != torch.bool or block_mask.dim() != 3:
+        raise ValueError('block_mask must be bool [H\', R, n_tiles]')
+    heads, rows, n = block_mask.shape
+    if kv_ok.numel() != n or full_tile.numel() != n:
+        raise ValueError('kv_ok / full_tile do not match the mask columns')
+    bm = block_mask.contiguous()
+    pc, pi, fc, fi = _empty_lists(heads, n, rows, block_mask.device)
+    _native.call('veda_index_lists_t', bm.data_ptr(), heads, rows, n, kv_ok.data_ptr(),
+                 full_tile.data_ptr(), pc.data_ptr(), pi.data_ptr(), fc.data_ptr(),
+                 fi.data_ptr(), _stream(block_mask))
+    return [pc, pi, fc, fi]
+
+
+@index_lists_t.register_fake
+def _(block_mask, kv_ok, full_tile):
+    h, r, n = block_mask.shape
+    return _empty_lists(h, n, r, block_mask.device)
+
+
+# Row length up to which the lists come straight from a selection.
+SELECTION_LISTS_MAX_TILES = 4096
+
+
+@torch.library.custom_op('veda::selection_lists', mutates_args=())
+def selection_lists(index: torch.Tensor, keep: torch.Tensor, kv_ok: torch.Tensor,
+                    full_tile: torch.Tensor, n_video: int) -> list[torch.Tensor]:
+    """index_lists of dense_block_mask(index, keep, kv_ok, n_video,
+    global_rows=True) in one kernel, for at most SELECTION_LISTS_MAX_TILES
+    tiles."""
+    _require_gpu(index, keep, kv_ok, full_tile)
+    heads, n_sel, k_total = index.shape
+    n = kv_ok.numel()
+    if n_sel != n_video:
+        raise ValueError('selection_lists needs a selection of all video rows')
+    if full_tile.numel() != n:
+        raise ValueError('kv_ok and full_tile differ in length')
+    idx_c, keep_c = index.contiguous(), keep.contiguous()  # held until the launch
+    pc, pi, fc, fi = _empty_lists(heads, n, n, index.device)
+    _native.call('veda_selection_lists', idx_c.data_ptr(), keep_c.data_ptr(), heads, n_video,
+                 k_total, kv_ok.data_ptr(), full_tile.data_ptr(), n, pc.data_ptr(), pi.data_ptr(),
+                 fc.data_ptr(), fi.data_ptr(), _stream(index))
+    return [pc, pi, fc, fi]
+
+
+@selection_lists.register_fake
+def _(index, keep, kv_ok, full_tile, n_video):
+    n = kv_ok.numel()
+    return _empty_lists(index.shape[0], n, n, index.device)
 
 
 # --------------------------------------------------------------------------
