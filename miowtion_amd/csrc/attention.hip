@@ -2205,202 +2205,333 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
 // Teacher statistics pass (no dense output): the LSE of every query row over
 // all valid keys, and per (key tile, row) the block statistic of the heat.
 //
-// Workgroup = (head, group of four query items), 16 waves, so each K tile
-// fetched into LDS serves four query tiles. Wave w owns item w / 4 of the
-// group, rows 32 (w % 4) .. + 31 (Q^T in registers), and all 64 keys of every
-// step (two 32-key sub-blocks): the same online softmax as the sparse
-// forward's (log2 domain, reference max raised only past a slack of 8), with
-// the current key tile's partial (sum relative to the reference, or the raw
-// max) in a register, written as one log2 statistic per row at the tile's
-// last step. Steps are the 64-key halves of every key tile in tile order, a
-// tile's halves consecutive (an empty tile one step with no valid key, so
-// every tile gets its statistic), through a 4-slot K ring.
+// Workgroup = (head, group of four query items), 8 waves, one workgroup per
+// CU, so each K tile fetched into LDS serves four query tiles. Wave w owns
+// item w / 2 of the group, rows 64 (w % 2) .. + 63 as two groups of 32 (Q^T
+// of both in registers), so each K fragment read from LDS feeds two
+// products. The unit of the walk is a 32-key sub-block of a key tile (the
+// ragged ends of partial tiles cost what they hold, to 32 keys); an empty
+// tile is one sub-block with no valid key, so every tile gets its statistic.
+//
+// A wave's stage is software-pipelined over the sub-blocks: the 16 products
+// of sub-block n + 1 (into one set of score registers) with the
+// exponentials and sums of sub-block n (from the other set) written out
+// between them, so the matrix and vector units work at once inside the wave.
+// Before, a wave multiplied and then exponentiated, sixteen 32-row waves met
+// at a barrier every 64 keys, and the two phases of all four waves of a SIMD
+// fell together: 4,800 cycles per step at full clock against 2,048 of
+// products. TSTATSTABLE
+//
+// K goes through a ring of three 128-row slots (four sub-blocks, each wave
+// one 1 KB segment of each), two in flight while one is used, with one
+// barrier per slot, so the waves may drift a slot's work apart.
 
-constexpr int kStatThreads = 1024;
+constexpr int kStatThreads = 512;
 constexpr int kStatItems = 4;
+constexpr int kSubBytes = 32 * kD * 2;         // 8 KB: 32 K rows
+constexpr int kStatSubs = 4;                   // sub-blocks per ring slot
+constexpr uint32_t kSubLast = 1u << 31;        // entry flag: last sub-block of its key tile
 
 template <int HEAT>
-__global__ void __launch_bounds__(kStatThreads) tstats_kernel(FwdParams p) {
-  __shared__ __attribute__((aligned(1024))) uint8_t ring[4][kHalfBytes];
-  __shared__ uint16_t steps[2 * kMaxBlocks];  // (key tile << 2) | (half << 1) | last of tile
-  __shared__ uint8_t tvc[kMaxBlocks];
-  __shared__ int32_t step_total;
+__global__ void __launch_bounds__(kStatThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+tstats_kernel(FwdParams p) {
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[3][kStatSubs * kSubBytes];
+  // sub-blocks: first key row << 6 | valid keys | kSubLast, padded with
+  // empty ones (key row 0, no valid key) to whole slots
+  __shared__ __attribute__((aligned(16))) uint32_t subs[4 * kMaxBlocks + kStatSubs];
+  __shared__ int32_t sub_total;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int pick = wave >> 2, rg = wave & 3;
   const int li = lane & 31, hi = lane >> 5;
   const int64_t n_groups = (p.n_q_tiles + kStatItems - 1) / kStatItems;
   const int64_t head = blockIdx.x / n_groups;
-  const int64_t r = (blockIdx.x % n_groups) * kStatItems + pick;
+  const int64_t r = (blockIdx.x % n_groups) * kStatItems + (wave >> 1);
   const bool item_ok = r < p.n_q_tiles;
-  const int64_t qrow = r * kTile + 32 * rg + li;  // row of lse / part
+  const int row0 = 64 * (wave & 1) + li;          // row of the item: row0, row0 + 32
+  const int64_t qrow = r * kTile + row0;          // row of lse / part
   const int64_t qtile = item_ok ? (p.q_tiles != nullptr ? p.q_tiles[r] : r) : -1;
   const bool qtile_ok = qtile >= 0 && qtile < p.q_tiles_held;
-  const int64_t qsrc = (qtile_ok ? qtile : 0) * kTile + 32 * rg + li;
+  const int64_t qsrc = (qtile_ok ? qtile : 0) * kTile + row0;
   const int nk = (int)p.n_k_tiles;
 
-  for (int j = tid; j < nk; j += kStatThreads) tvc[j] = (uint8_t)min(max(p.valid_count[j], 0), kTile);
+  bf16x8 qf[2][8];
+  uint32_t any = 0;
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const u32x4 v = qtile_ok ? ld16(p.q + (qsrc + 32 * g) * p.qs + head * p.qh + 16 * s + 8 * hi)
+                               : u32x4{0, 0, 0, 0};
+      any |= v[0] | v[1] | v[2] | v[3];
+      qf[g][s] = as_bf16x8(v);
+    }
   if (wave == 0) {
     int n = 0;
     for (int j0 = 0; j0 < nk; j0 += 64) {
       const int j = j0 + lane;
-      const bool one = j < nk;
-      const bool two = one && p.valid_count[j] > kHalf;
-      const uint64_t b1 = __ballot(one), b2 = __ballot(two);
-      const int rank =
-          __builtin_amdgcn_mbcnt_hi((uint32_t)(b1 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b1, 0)) +
-          __builtin_amdgcn_mbcnt_hi((uint32_t)(b2 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b2, 0));
-      if (one) steps[n + rank] = (uint16_t)((j << 2) | (two ? 0 : 1));
-      if (two) steps[n + rank + 1] = (uint16_t)((j << 2) | 2 | 1);
-      n += __builtin_popcountll(b1) + __builtin_popcountll(b2);
+      const int vc = j < nk ? min(max(p.valid_count[j], 0), kTile) : 0;
+      const int cnt = j < nk ? max((vc + 31) >> 5, 1) : 0;  // 1 .. 4 sub-blocks
+      // exclusive prefix of the counts over the lanes, three ballots
+      int at = n, all = 0;
+#pragma unroll
+      for (int b = 0; b < 3; ++b) {
+        const uint64_t bal = __ballot((cnt >> b) & 1);
+        at += __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
+                                        __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0)) << b;
+        all += __builtin_popcountll(bal) << b;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i < cnt)
+          subs[at + i] = ((uint32_t)(j * kTile + 32 * i) << 6) | (uint32_t)min(max(vc - 32 * i, 0), 32) |
+                         (i == cnt - 1 ? kSubLast : 0u);
+      n += all;
     }
-    if (lane == 0) step_total = n;
-  }
-
-  WaveState w;
-#pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    const u32x4 v =
-        qtile_ok ? ld16(p.q + qsrc * p.qs + head * p.qh + 16 * s + 8 * hi) : u32x4{0, 0, 0, 0};
-    w.qf[s] = as_bf16x8(v);
+    if (lane < kStatSubs) subs[n + lane] = 0;
+    if (lane == 0) sub_total = n;
   }
 #pragma unroll
-  for (int s = 0; s < 8; ++s) asm volatile("" : : "v"(w.qf[s]));
-  w.m_run = -INFINITY;
-  w.l_run = 0.f;
-  w.mu = 0.f;
-  w.blk = HEAT == kHeatMax ? -INFINITY : 0.f;
-  __syncthreads();  // step list and valid counts ready
-  const int n_steps = __builtin_amdgcn_readfirstlane(step_total);
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int s = 0; s < 8; ++s) asm volatile("" : : "v"(qf[g][s]));
+  // a wave whose 64 query rows are all zero (padding): every score is 0
+  const bool q_zero = __ballot(any != 0) == 0;
+  __syncthreads();  // sub-block list ready
+  const int n_slots = (__builtin_amdgcn_readfirstlane(sub_total) + kStatSubs - 1) / kStatSubs;
 
   const float c = p.scale_log2;
-  const HFrag fa = hfrag_offsets(0, lane), fb = hfrag_offsets(1, lane);
-  // this wave's 1 KB K segment of a step: rows 4 wave + lane / 16, LDS chunk
-  // lane % 16 holding logical chunk (lane % 16) ^ (row & 15); a segment
-  // wholly past the valid count re-reads rows lane / 16
-  uint32_t koff, kskip;
+  // K fragment of product k: row li of the sub-block, logical chunk 2 k + hi
+  uint32_t kfo[8];
   {
-    const int lr = lane >> 4, pc = lane & 15, row = 4 * wave + lr;
-    const int kc = (pc ^ (row & 15)) << 3;
-    koff = (uint32_t)((row * p.ks + kc) * 2);
-    kskip = (uint32_t)((lr * p.ks + kc) * 2);
+    const uint32_t krow = li * 256, x = (hi ^ (li & 15)) << 4;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) kfo[k] = krow + (x ^ (k << 5));
+  }
+  // this wave's 1 KB segment of a sub-block: rows 4 wave + lane / 16, LDS
+  // chunk lane % 16 holding logical chunk (lane % 16) ^ (row & 15)
+  uint32_t koff;
+  {
+    const int pc = lane & 15, row = 4 * wave + (lane >> 4);
+    koff = (uint32_t)((row * p.ks + ((pc ^ (row & 15)) << 3)) * 2);
   }
   const uint16_t* kbase = p.k + head * p.kh;
-  auto entry = [&](int u) { return __builtin_amdgcn_readfirstlane((int)steps[u]); };
-  auto valid_of = [&](int e) {
-    const int vc = __builtin_amdgcn_readfirstlane((int)tvc[e >> 2]);
-    return (e & 2) ? vc - kHalf : min(vc, kHalf);
+  typedef const __attribute__((address_space(3))) u32x4* lds_u32x4;
+  struct Entries {
+    uint32_t e[kStatSubs];
   };
-  auto load_step = [&](int u, lds_u8* slot) {
-    const int e = entry(u);
-    const int64_t row0 = (int64_t)(e >> 2) * kTile + ((e >> 1) & 1) * kHalf;
-    const char* b = reinterpret_cast<const char*>(kbase + row0 * p.ks);
-    dma16(b, 4 * wave < valid_of(e) ? koff : kskip, slot + wave * 1024);
-  };
-  // One step over the step's vch valid keys (sub-block B only when vch > 32).
-  // 'sum': once a row has a reference, the step's probabilities are taken
-  // against it as it stands and kept unless their sum could lose range
-  // (2^64 or more, or not finite), so most steps skip the row max; such a
-  // step, a row's first one, and every 'max' step run the online softmax as
-  // the sparse forward does (reference raised past a slack of 8).
-  auto step = [&](const lds_u8* slot, int vch) {
-    const f32x16 sa = sub_scores(slot, fa, w, vch, hi);
-    f32x16 sb;
-    const bool two = vch > 32;
-    if (two) sb = sub_scores(slot, fb, w, vch - 32, hi);
-    if (HEAT == kHeatSum && __all(w.m_run != -INFINITY)) {
-      const float mu = w.mu;
-      float l4[4] = {0.f, 0.f, 0.f, 0.f};
+  auto entries = [&](int u) {
+    const u32x4 v = *reinterpret_cast<lds_u32x4>((const lds_u8*)&subs[kStatSubs * u]);
+    Entries x;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        l4[e >> 2] += __builtin_amdgcn_exp2f(fmaf(sa[e], c, -mu));
-        if (two) l4[e >> 2] += __builtin_amdgcn_exp2f(fmaf(sb[e], c, -mu));
-      }
-      const float lsum = (l4[0] + l4[1]) + (l4[2] + l4[3]);
-      if (__all(lsum < 0x1p64f)) {
-        w.l_run += lsum;
-        w.blk += lsum;
-        return;
-      }
+    for (int i = 0; i < kStatSubs; ++i) x.e[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)v[i]);
+    return x;
+  };
+  // rows past a sub-block's valid keys are the key tile's own padding rows
+  auto load_slot = [&](int u, lds_u8* slot) {
+    const Entries x = entries(u);
+#pragma unroll
+    for (int i = 0; i < kStatSubs; ++i) {
+      const int64_t row = (int64_t)((x.e[i] & ~kSubLast) >> 6);
+      dma16(reinterpret_cast<const char*>(kbase + row * p.ks), koff,
+            slot + i * kSubBytes + wave * 1024);
     }
+  };
+
+  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f}, mu[2] = {0.f, 0.f};
+  // the current key tile's partial: this lane's sum relative to mu, or its raw max
+  constexpr float kBlk0 = HEAT == kHeatMax ? -INFINITY : 0.f;
+  float blk[2] = {kBlk0, kBlk0};
+
+  // The online softmax over one sub-block's scores of row group g: the
+  // reference is raised past a slack of 8, sums move to it.
+  auto online = [&](int g, const f32x16& s) {
     float mloc = -INFINITY;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) mloc = fmaxf(mloc, two ? fmaxf(sa[e], sb[e]) : sa[e]);
-    const float mraw = half_swap_max(mloc);  // the row's raw max over the step's keys
-    mloc = mraw * c;
-    const float m_new = mloc > w.m_run + kRescaleSlack ? mloc : w.m_run;
-    const float mu = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = __builtin_amdgcn_exp2f(w.m_run - mu);
-    w.m_run = m_new;
-    w.mu = mu;
-    if (HEAT == kHeatMax) w.blk = fmaxf(w.blk, mraw);
+    for (int e = 0; e < 16; ++e) mloc = fmaxf(mloc, s[e]);
+    mloc = half_swap_max(mloc) * c;
+    const float m_new = mloc > m_run[g] + kRescaleSlack ? mloc : m_run[g];
+    const float mu_new = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = __builtin_amdgcn_exp2f(m_run[g] - mu_new);
+    m_run[g] = m_new;
+    mu[g] = mu_new;
     float l4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      l4[e >> 2] += __builtin_amdgcn_exp2f(fmaf(sa[e], c, -mu));
-      if (two) l4[e >> 2] += __builtin_amdgcn_exp2f(fmaf(sb[e], c, -mu));
-    }
+    for (int e = 0; e < 16; ++e) l4[e >> 2] += __builtin_amdgcn_exp2f(fmaf(s[e], c, -mu_new));
     const float lsum = (l4[0] + l4[1]) + (l4[2] + l4[3]);
-    w.l_run = fmaf(w.l_run, alpha, lsum);
-    if (HEAT == kHeatSum) w.blk = fmaf(w.blk, alpha, lsum);
+    l_run[g] = fmaf(l_run[g], alpha, lsum);
+    if (HEAT == kHeatSum) blk[g] = fmaf(blk[g], alpha, lsum);
   };
-  // At a tile's last step: its log2 statistic per row (log-sum-exp for
+  // At a tile's last sub-block: its log2 statistic per row (log-sum-exp for
   // 'sum', the bf16-rounded raw max times the scale for 'max', as the
   // reference's heat rounds scores to bf16 before scaling).
-  auto flush = [&](int j) {
-    float l;
-    if (HEAT == kHeatSum) {
-      const float tot = half_swap_sum(w.blk);
-      l = tot > 0.f ? __log2f(tot) + w.mu : -INFINITY;
-      w.blk = 0.f;
-    } else {
-      l = bf16_to_f32(f32_to_bf16(w.blk)) * c;
-      w.blk = -INFINITY;
+  float* const prow = p.part + head * p.part_sh + r * kTile;  // scalar; the lane adds row0
+  auto flush = [&](int64_t j) {
+    float* const dst = prow + j * p.part_st;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      float l;
+      if (HEAT == kHeatSum) {
+        const float tot = half_swap_sum(blk[g]);
+        l = tot > 0.f ? __log2f(tot) + mu[g] : -INFINITY;
+      } else {
+        l = bf16_to_f32(f32_to_bf16(half_swap_max(blk[g]))) * c;
+      }
+      blk[g] = kBlk0;
+      if (item_ok && hi == 0) dst[(uint32_t)(row0 + 32 * g)] = l;
     }
-    if (item_ok && hi == 0) p.part[head * p.part_sh + (int64_t)j * p.part_st + qrow] = l;
   };
-  auto compute_step = [&](int u, const lds_u8* slot) {
-    const int e = entry(u);
-    const int vch = valid_of(e);
-    if (vch > 0) step(slot, vch);
-    if (e & 1) flush(e >> 2);
+  bool have_ref = false;  // every row of the wave has a reference (wave-uniform)
+  // One stage: the products of the sub-block at `kb` into sn (PRODUCTS),
+  // and the softmax of the previous one's scores sp (entry `e`; VALUES).
+  // Probabilities are taken against the reference as it stands and kept
+  // unless their sum could lose range (2^64 or more, or not finite) or a row
+  // has no reference yet: then the sub-block runs the online softmax.
+  auto stage = [&](auto products, auto values, const lds_u8* kb, f32x16 (&sn)[2], f32x16 (&sp)[2],
+                   uint32_t e) __attribute__((always_inline)) {
+    constexpr bool P = decltype(products)::value, V = decltype(values)::value;
+    const int lim = (int)(e & 63u);
+    if (V && lim < 32) {
+      mask_scores(sp[0], lim, hi);
+      mask_scores(sp[1], lim, hi);
+    }
+    u32x4 kf[8];
+    float l4[2][4];
+    float mx[2] = {-INFINITY, -INFINITY};
+    if (P) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int x = 0; x < 16; ++x) sn[g][x] = 0.f;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) kf[k] = *reinterpret_cast<lds_u32x4>(kb + kfo[k]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (P) {
+        if (k + 3 < 8) kf[k + 3] = *reinterpret_cast<lds_u32x4>(kb + kfo[k + 3]);
+        sn[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kf[k]), qf[0][k], sn[0], 0, 0, 0);
+        sn[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kf[k]), qf[1][k], sn[1], 0, 0, 0);
+      }
+      if (V) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+#pragma unroll
+          for (int x = 2 * k; x < 2 * k + 2; ++x) {
+            const float pr = __builtin_amdgcn_exp2f(fmaf(sp[g][x], c, -mu[g]));
+            l4[g][x >> 2] = (x & 3) == 0 ? pr : l4[g][x >> 2] + pr;
+          }
+          if (HEAT == kHeatMax) mx[g] = fmaxf(mx[g], fmaxf(sp[g][2 * k], sp[g][2 * k + 1]));
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (V) {
+      const float l0 = (l4[0][0] + l4[0][1]) + (l4[0][2] + l4[0][3]);
+      const float l1 = (l4[1][0] + l4[1][1]) + (l4[1][2] + l4[1][3]);
+      if (HEAT == kHeatMax) {
+        blk[0] = fmaxf(blk[0], mx[0]);
+        blk[1] = fmaxf(blk[1], mx[1]);
+      }
+      // l0 + l1 below 2^64 (neither inf nor NaN) bounds both
+      if (__builtin_expect(have_ref && __ballot(l0 + l1 < 0x1p64f) == ~0ull, 1)) {
+        l_run[0] += l0;
+        l_run[1] += l1;
+        if (HEAT == kHeatSum) {
+          blk[0] += l0;
+          blk[1] += l1;
+        }
+      } else if (lim > 0) {
+        online(0, sp[0]);
+        online(1, sp[1]);
+        have_ref = __ballot(m_run[0] != -INFINITY && m_run[1] != -INFINITY) == ~0ull;
+      }
+      if (e & kSubLast) flush((int64_t)((e & ~kSubLast) >> 6) / kTile);
+    }
   };
-  lds_u8* K0 = (lds_u8*)ring[0];
-  lds_u8* K1 = (lds_u8*)ring[1];
-  lds_u8* K2 = (lds_u8*)ring[2];
-  lds_u8* K3 = (lds_u8*)ring[3];
-  // The ring: step u in slot u & 3; at the top of step u its own load is
-  // waited for (those of u+1, u+2 may stay in flight), then a bare barrier,
-  // then the slot step u-1 used is refilled with step u+3.
-  auto top = [&](int u) {
-    if (u + 2 < n_steps) VEDA_WAIT_VM(2);
-    else if (u + 1 < n_steps) VEDA_WAIT_VM(1);
+
+  lds_u8* R0 = (lds_u8*)ring[0];
+  lds_u8* R1 = (lds_u8*)ring[1];
+  lds_u8* R2 = (lds_u8*)ring[2];
+  // Slot u of the walk is ring slot u % 3. At its top its own loads are
+  // waited for (those of u + 1 may stay in flight), then a bare barrier (all
+  // waves' loads are in LDS, and all are done with slot u - 1's rows), then
+  // slot u + 2's loads go out into the place slot u - 1 left.
+  auto top = [&](int u, lds_u8* next) {
+    if (u + 1 < n_slots) VEDA_WAIT_VM(kStatSubs);
     else VEDA_WAIT_VM(0);
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");  // no LDS read of slot u above the barrier
+    if (u + 2 < n_slots) load_slot(u + 2, next);
   };
-  if (n_steps > 0) load_step(0, K0);
-  if (n_steps > 1) load_step(1, K1);
-  if (n_steps > 2) load_step(2, K2);
-  for (int u = 0; u < n_steps; u += 4) {
-    top(u);
-    if (u + 3 < n_steps) load_step(u + 3, K3);
-    compute_step(u, K0);
-    if (u + 1 >= n_steps) break;
-    top(u + 1);
-    if (u + 4 < n_steps) load_step(u + 4, K0);
-    compute_step(u + 1, K1);
-    if (u + 2 >= n_steps) break;
-    top(u + 2);
-    if (u + 5 < n_steps) load_step(u + 5, K1);
-    compute_step(u + 2, K2);
-    if (u + 3 >= n_steps) break;
-    top(u + 3);
-    if (u + 6 < n_steps) load_step(u + 6, K2);
-    compute_step(u + 3, K3);
+  f32x16 sa[2], sb[2];
+  uint32_t prev = 0;  // the entry whose scores are in sb
+  using T = std::true_type;
+  using F = std::false_type;
+  auto slot_work = [&](auto first, int u, const lds_u8* slot) __attribute__((always_inline)) {
+    const Entries x = entries(u);
+    if constexpr (decltype(first)::value)
+      stage(T{}, F{}, slot, sa, sb, 0u);
+    else
+      stage(T{}, T{}, slot, sa, sb, prev);
+    stage(T{}, T{}, slot + kSubBytes, sb, sa, x.e[0]);
+    stage(T{}, T{}, slot + 2 * kSubBytes, sa, sb, x.e[1]);
+    stage(T{}, T{}, slot + 3 * kSubBytes, sb, sa, x.e[2]);
+    prev = x.e[3];
+  };
+  // An all-zero wave: every valid key scores 0, so p is 1 and the reference
+  // 0; it loads and passes the barriers, and its statistics are counts.
+  auto slot_zero = [&](int u) {
+    const Entries x = entries(u);
+#pragma unroll
+    for (int i = 0; i < kStatSubs; ++i) {
+      const float n = (float)(x.e[i] & 63u);
+      if (n > 0.f) m_run[0] = m_run[1] = 0.f;
+      const float mine = hi == 0 ? n : 0.f;  // flush and the LSE add the two lane halves
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        l_run[g] += mine;
+        if (HEAT == kHeatSum) blk[g] += mine;
+        else if (n > 0.f) blk[g] = 0.f;
+      }
+      if (x.e[i] & kSubLast) flush((int64_t)((x.e[i] & ~kSubLast) >> 6) / kTile);
+    }
+  };
+  if (n_slots > 0) load_slot(0, R0);
+  if (n_slots > 1) load_slot(1, R1);
+  if (q_zero) {
+    for (int u = 0; u < n_slots; u += 3) {
+      top(u, R2);
+      slot_zero(u);
+      if (u + 1 >= n_slots) break;
+      top(u + 1, R0);
+      slot_zero(u + 1);
+      if (u + 2 >= n_slots) break;
+      top(u + 2, R1);
+      slot_zero(u + 2);
+    }
+  } else {
+    top(0, R2);
+    slot_work(T{}, 0, R0);
+    for (int u = 1; u < n_slots; u += 3) {
+      top(u, R0);
+      slot_work(F{}, u, R1);
+      if (u + 1 >= n_slots) break;
+      top(u + 1, R1);
+      slot_work(F{}, u + 1, R2);
+      if (u + 2 >= n_slots) break;
+      top(u + 2, R2);
+      slot_work(F{}, u + 2, R0);
+    }
+    stage(F{}, T{}, R0, sa, sb, prev);
   }
-  const float l = half_swap_sum(w.l_run);
-  if (item_ok && hi == 0)
-    p.lse[head * p.lse_sh + qrow * p.lse_ss] = l > 0.f ? (w.m_run + __log2f(l)) * kLn2 : -INFINITY;
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const float l = half_swap_sum(l_run[g]);
+    if (item_ok && hi == 0)
+      p.lse[head * p.lse_sh + (qrow + 32 * g) * p.lse_ss] =
+          l > 0.f ? (m_run[g] + __log2f(l)) * kLn2 : -INFINITY;
+  }
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
