@@ -45,7 +45,6 @@ namespace {
 
 constexpr int kD = 128;
 constexpr int kThreads = 512;
-constexpr int kTileBytes = kTile * kD * 2;       // 32 KB: one K or V tile
 constexpr int kMaxBlocks = 2048;                 // key tiles per row (FA4's cap)
 // LDS offset in ring slot 1 of the Q fragments a narrow walk hands from wave
 // 0 to wave 1 (8 KB, past the set-up's 12 KB step-list scratch)
@@ -550,10 +549,9 @@ constexpr uint16_t kPairStep = 0x8000;  // step entry flag: a pair of ragged hal
 constexpr int kSweepWorkgroups = 512;
 
 // Per-lane byte offsets of this wave's eight 1 KB segments of a step
-// (segments 4 w + u, u = 0..3, of K and of V: rows 4 seg + l / 16), and of
-// their redirect (rows l / 16) for segments wholly past the valid count.
+// (segments 4 w + u, u = 0..3, of K and of V: rows 4 seg + l / 16).
 struct SDma {
-  uint32_t k[4], v[4], k_skip[4], v_skip[4];
+  uint32_t k[4], v[4];
 };
 
 // Source offsets of wave `wave`'s four 1 KB segments (rows 16 wave .. + 15
@@ -571,8 +569,6 @@ __device__ __forceinline__ SDma sdma_offsets(int64_t ks, int64_t vs, int wave, i
     const int kc = (pc ^ (row & 15)) << 3, vc = (pc ^ ((row & 3) << 2)) << 3;
     d.k[u] = (uint32_t)((src * ks + kc) * 2);
     d.v[u] = (uint32_t)((src * vs + vc) * 2);
-    d.k_skip[u] = (uint32_t)((lr * ks + kc) * 2);
-    d.v_skip[u] = (uint32_t)((lr * vs + vc) * 2);
   }
   return d;
 }
@@ -605,66 +601,6 @@ __device__ __forceinline__ f32x16 sub_scores(const lds_u8* slot, const HFrag& f,
   return s;
 }
 
-// Scores of both 32-key sub-blocks of a step, as two interleaved MFMA
-// chains (each fragment read has the other chain's product to hide behind),
-// then the masks of sub-blocks with fewer than 32 valid keys.
-__device__ __forceinline__ void pair_scores(const lds_u8* slot, const HFrag& fa, const HFrag& fb,
-                                            const WaveState& w, int la, int lb, int hi,
-                                            f32x16& sa, f32x16& sb) {
-#pragma unroll
-  for (int e = 0; e < 16; ++e) sa[e] = sb[e] = 0.f;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const u32x4 ka = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(slot + fa.k[k]);
-    const u32x4 kb = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(slot + fb.k[k]);
-    sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(ka), w.qf[k], sa, 0, 0, 0);
-    sb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kb), w.qf[k], sb, 0, 0, 0);
-  }
-  // issue order: the reads of k + 2 before the products of k (more reads
-  // ahead than the compiler's own schedule keeps; all 16 ahead was slower)
-  __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-  }
-  __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-  mask_scores(sa, la, hi);
-  mask_scores(sb, lb, hi);
-}
-
-// The same products with hook(k) between them: the fragment reads of
-// product k + 2 are placed before product k and hook(k) before the reads of
-// k + 2, in program order (a hook that branches ends the scheduling region,
-// so the order is written out instead of left to scheduling hints).
-template <typename Hook>
-__device__ __forceinline__ void pair_scores_hooked(const lds_u8* slot, const HFrag& fa,
-                                                   const HFrag& fb, const WaveState& w, int la,
-                                                   int lb, int hi, f32x16& sa, f32x16& sb,
-                                                   Hook hook) {
-  typedef const __attribute__((address_space(3))) u32x4* lds_u32x4;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) sa[e] = sb[e] = 0.f;
-  u32x4 ka[8], kb[8];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    ka[k] = *reinterpret_cast<lds_u32x4>(slot + fa.k[k]);
-    kb[k] = *reinterpret_cast<lds_u32x4>(slot + fb.k[k]);
-  }
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    hook(k);
-    if (k + 2 < 8) {
-      ka[k + 2] = *reinterpret_cast<lds_u32x4>(slot + fa.k[k + 2]);
-      kb[k + 2] = *reinterpret_cast<lds_u32x4>(slot + fb.k[k + 2]);
-    }
-    sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(ka[k]), w.qf[k], sa, 0, 0, 0);
-    sb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kb[k]), w.qf[k], sb, 0, 0, 0);
-  }
-  mask_scores(sa, la, hi);
-  mask_scores(sb, lb, hi);
-}
-
 // The V^T fragment (A operand) of product (kk, dt) of a sub-block: two
 // transposed reads of its 16-key group kk.
 __device__ __forceinline__ bf16x8 vt_frag(const lds_u8* slot, const HFrag& f, int kk, int dt) {
@@ -691,74 +627,14 @@ __device__ __forceinline__ void pack_probs(const float (&ps)[16], u32x4 (&pk)[2]
     for (int m = 0; m < 4; ++m) pk[kk][m] = pack_bf16x2(ps[8 * kk + 2 * m], ps[8 * kk + 2 * m + 1]);
 }
 
-// One step of one wave over its two 32-key sub-blocks, la and lb valid keys
-// (as sub_scores' lim): the same online softmax as hstep, over 64 keys.
-// Both sub-blocks are always computed: one code path per step keeps the
-// accumulators in the same registers from step to step (a path that skips
-// sub-block b makes the compiler move O between register sets every step).
-// PAIR: the two sub-blocks' score products as interleaved chains with reads
-// ahead (pair_scores); the dense walk keeps them as two chains, which it
-// runs faster at long sequences (C5: 566 against 595 ms).
-// qk_hook(k) runs between the score products (pair_scores_hooked).
-template <bool PAIR = true, typename QKHook = NoHook>
-__device__ __forceinline__ void sstep(const lds_u8* slot, const HFrag& fa, const HFrag& fb,
-                                      float c, int la, int lb, int hi, WaveState& w,
-                                      QKHook qk_hook = {}) {
-  f32x16 sa, sb;
-  if constexpr (!std::is_same<QKHook, NoHook>::value) {
-    pair_scores_hooked(slot, fa, fb, w, la, lb, hi, sa, sb, qk_hook);
-  } else if constexpr (PAIR) {
-    pair_scores(slot, fa, fb, w, la, lb, hi, sa, sb);
-  } else {
-    sa = sub_scores(slot, fa, w, la, hi);
-    sb = sub_scores(slot, fb, w, lb, hi);
-  }
-
-  float mloc = -INFINITY;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) mloc = fmaxf(mloc, sa[e]);
-#pragma unroll
-  for (int e = 0; e < 16; ++e) mloc = fmaxf(mloc, sb[e]);
-  mloc = half_swap_max(mloc) * c;
-  const float m_new = mloc > w.m_run + kRescaleSlack ? mloc : w.m_run;
-  const float mu = m_new == -INFINITY ? 0.f : m_new;
-  const float alpha = __builtin_amdgcn_exp2f(w.m_run - mu);
-  w.m_run = m_new;
-  float pa[16], pb[16];
-#pragma unroll
-  for (int e = 0; e < 16; ++e) pa[e] = __builtin_amdgcn_exp2f(fmaf(sa[e], c, -mu));
-  float l4[4];
-#pragma unroll
-  for (int g = 0; g < 4; ++g) l4[g] = (pa[4 * g] + pa[4 * g + 1]) + (pa[4 * g + 2] + pa[4 * g + 3]);
-  float lsum = (l4[0] + l4[1]) + (l4[2] + l4[3]);
-#pragma unroll
-  for (int e = 0; e < 16; ++e) pb[e] = __builtin_amdgcn_exp2f(fmaf(sb[e], c, -mu));
-#pragma unroll
-  for (int g = 0; g < 4; ++g) l4[g] = (pb[4 * g] + pb[4 * g + 1]) + (pb[4 * g + 2] + pb[4 * g + 3]);
-  lsum += (l4[0] + l4[1]) + (l4[2] + l4[3]);
-  w.l_run = fmaf(w.l_run, alpha, lsum);
-  u32x4 ka[2], kb[2];
-  pack_probs(pa, ka);
-  pack_probs(pb, kb);
-  if (__any(alpha != 1.f)) {
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) w.o[dt][e] *= alpha;
-  }
-  sub_pv(slot, fa, ka, w);
-  sub_pv(slot, fb, kb, w);
-}
-
 // The step of a wave whose 32 query rows are all zero (the padding rows of
 // a partial query tile, whose gathered q is zero): every valid key scores
 // exactly 0, so P is 1 on the valid keys and 0 on the masked ones, the
 // running max is 0 from the first valid key on and the row sum counts the
 // valid keys. Only the P.V products remain; the result is bit-identical to
 // sstep's on the same rows (the same products of the same exact P).
-__device__ __forceinline__ void sstep_zero_q(const lds_u8* slot, const HFrag& fa,
-                                             const HFrag& fb, int la, int lb, int hi,
-                                             WaveState& w) {
+__device__ __forceinline__ void sstep_zero_q(const lds_u8* slot, const HFrag& f, int la, int lb,
+                                             int hi, WaveState& w) {
   if (la <= 0 && lb <= 0) return;  // no valid key: P is 0 everywhere
   w.m_run = 0.f;
   auto probs = [&](int lim, u32x4 (&pk)[2]) {
@@ -783,60 +659,15 @@ __device__ __forceinline__ void sstep_zero_q(const lds_u8* slot, const HFrag& fa
   u32x4 ka[2], kb[2];
   probs(la, ka);
   probs(lb, kb);
-  sub_pv(slot, fa, ka, w);
-  sub_pv(slot, fb, kb, w);
+  sub_pv(slot, f, ka, w);
+  sub_pv(slot + 8192, f, kb, w);
 }
 
 // Narrow walk (a query tile whose only real rows are its first 32): each
 // wave takes one 32-key sub-block of every step, so the tile's products
 // spread over all four SIMDs of the workgroup instead of one wave's chain.
-// sstep_half is one sub-block (lim valid keys) of sstep for the tile's real
-// rows, with hook(k) before the fragment reads of score product k + 2;
 // sstep_half_zero is one sub-block of sstep_zero_q. The two sub-blocks'
 // partial states are merged at the end of the walk.
-template <typename Hook>
-__device__ __forceinline__ void sstep_half(const lds_u8* slot, const HFrag& f, float c, int lim,
-                                           int hi, WaveState& w, Hook hook) {
-  typedef const __attribute__((address_space(3))) u32x4* lds_u32x4;
-  f32x16 s;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) s[e] = 0.f;
-  u32x4 kf[8];
-  kf[0] = *reinterpret_cast<lds_u32x4>(slot + f.k[0]);
-  kf[1] = *reinterpret_cast<lds_u32x4>(slot + f.k[1]);
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    hook(k);
-    if (k + 2 < 8) kf[k + 2] = *reinterpret_cast<lds_u32x4>(slot + f.k[k + 2]);
-    s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kf[k]), w.qf[k], s, 0, 0, 0);
-  }
-  mask_scores(s, lim, hi);
-  float mloc = -INFINITY;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) mloc = fmaxf(mloc, s[e]);
-  mloc = half_swap_max(mloc) * c;
-  const float m_new = mloc > w.m_run + kRescaleSlack ? mloc : w.m_run;
-  const float mu = m_new == -INFINITY ? 0.f : m_new;
-  const float alpha = __builtin_amdgcn_exp2f(w.m_run - mu);
-  w.m_run = m_new;
-  float ps[16];
-#pragma unroll
-  for (int e = 0; e < 16; ++e) ps[e] = __builtin_amdgcn_exp2f(fmaf(s[e], c, -mu));
-  float l4[4];
-#pragma unroll
-  for (int g = 0; g < 4; ++g) l4[g] = (ps[4 * g] + ps[4 * g + 1]) + (ps[4 * g + 2] + ps[4 * g + 3]);
-  w.l_run = fmaf(w.l_run, alpha, (l4[0] + l4[1]) + (l4[2] + l4[3]));
-  u32x4 pk[2];
-  pack_probs(ps, pk);
-  if (__any(alpha != 1.f)) {
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) w.o[dt][e] *= alpha;
-  }
-  sub_pv(slot, f, pk, w);
-}
-
 __device__ __forceinline__ void sstep_half_zero(const lds_u8* slot, const HFrag& f, int lim, int hi,
                                                 WaveState& w) {
   if (lim <= 0) return;  // no valid key: P is 0 everywhere
@@ -862,13 +693,125 @@ __device__ __forceinline__ void sstep_half_zero(const lds_u8* slot, const HFrag&
   sub_pv(slot, f, pk, w);
 }
 
-// The 16 weights of this lane's keys key0 + 8 g + 4 hi + m of a sub-block.
-__device__ __forceinline__ void sub_weights(const uint8_t* wt, int key0, int hi, float (&ww)[16]) {
+// ---------------------------------------------------------------------------
+// The pipelined step. A stage works on three consecutive 32-key sub-blocks at
+// once: the score products of sub-block n + 1 (QK: K rows at `kb` into sn),
+// the softmax of sub-block n (SM: scores sp, `lim` valid keys, into the
+// packed probabilities pn) and the P.V products of sub-block n - 1 (PV: V
+// rows at `vb`, probabilities pp). The three are independent, so they are
+// written out in turn, one product of each kind and the softmax of two keys
+// a piece, with scheduling fences between the pieces: a wave's vector and
+// matrix work run at once instead of one after the other. A stage is one
+// basic block: a branch inside it (a conditional load, O rescaled in place by
+// the softmax) makes the compiler move the softmax out of it or keep O in two
+// sets of registers, so loads are issued unconditionally and O's rescale is
+// left to the next stage's start (PipeState::alpha).
+//
+// Before, a step of 64 keys multiplied, took its softmax and multiplied
+// again, and on constant data (at full clock) took the sum of the two units'
+// times, the other wave of the SIMD filling little of it. 57,720 tokens x 48
+// heads, dense: 51.9 -> 44.8 ms on constant data (32.7 at the bf16 peak),
+// 72.2 -> 68.4 ms on random data, where the power limit lowers the clock
+// (the same board multiplies random bf16 matrices at 1.5 and zeros at 2.0
+// PFLOP/s). Sparse walks, where K and V come from beyond L2: sequence order
+// 6.08 -> 5.92 ms the whole layer (with the dead waves dropped), 14.64 ->
+// 14.12 at keep 0.2, tile order 5.58 -> 5.54 ms.
+//
+// The reference of a row is the maximum of its first sub-block; later
+// probabilities are taken against it as it stands, with no maximum taken,
+// unless a lane's 16 probabilities sum to kLazyLimit or more (or are not
+// finite), or a row has no reference yet: then the sub-block runs the online
+// softmax (raise_reference), which rescales O and l and takes the
+// probabilities again.
+constexpr float kLazyLimit = 4096.f;
+
+// The pipeline's state beside WaveState: the factor O is still to be scaled
+// by (the reference rose in the last softmax) and whether every row of the
+// wave has a reference.
+struct PipeState {
+  float alpha;
+  bool have_ref;
+};
+
+__device__ __forceinline__ void raise_reference(const f32x16& s, float c, u32x4 (&pk)[2],
+                                                WaveState& w, PipeState& ps) {
+  float mloc = -INFINITY;
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const uint32_t w4 = *reinterpret_cast<const uint32_t*>(wt + key0 + 8 * g + 4 * hi);
+  for (int e = 0; e < 16; ++e) mloc = fmaxf(mloc, s[e]);
+  mloc = half_swap_max(mloc) * c;
+  const float m_new = mloc > w.m_run + kRescaleSlack ? mloc : w.m_run;
+  const float mu = m_new == -INFINITY ? 0.f : m_new;
+  ps.alpha = __builtin_amdgcn_exp2f(w.m_run - mu);
+  w.m_run = m_new;
+  w.mu = mu;
+  float l4[4];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) ww[4 * g + m] = (float)((w4 >> (8 * m)) & 0xffu);
+  for (int j = 0; j < 8; ++j) {
+    const float a = __builtin_amdgcn_exp2f(fmaf(s[2 * j], c, -mu));
+    const float b = __builtin_amdgcn_exp2f(fmaf(s[2 * j + 1], c, -mu));
+    l4[j >> 1] = (j & 1) ? l4[j >> 1] + (a + b) : a + b;
+    pk[j >> 2][j & 3] = pack_bf16x2(a, b);
+  }
+  w.l_run = fmaf(w.l_run, ps.alpha, (l4[0] + l4[1]) + (l4[2] + l4[3]));
+  ps.have_ref = __ballot(m_new != -INFINITY) == ~0ull;
+}
+
+template <bool QK, bool SM, bool PV, typename Hook>
+__device__ __forceinline__ void pstage(const lds_u8* kb, const lds_u8* vb, const HFrag& f, float c,
+                                       int lim, int hi, f32x16& sn, f32x16& sp, u32x4 (&pn)[2],
+                                       const u32x4 (&pp)[2], WaveState& w, PipeState& ps, Hook hook) {
+  typedef const __attribute__((address_space(3))) u32x4* lds_u32x4;
+  if (SM) mask_scores(sp, lim, hi);
+  if (PV && __any(ps.alpha != 1.f)) {
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) w.o[dt][e] *= ps.alpha;
+  }
+  u32x4 kf[8];
+  bf16x8 va[8];
+  if (QK) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sn[e] = 0.f;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) kf[k] = *reinterpret_cast<lds_u32x4>(kb + f.k[k]);
+  }
+  if (PV) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) va[j] = vt_frag(vb, f, 0, j);
+  }
+  float l4[4];
+  const float mu = w.mu;
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    hook(j);
+    if (QK) {
+      if (j + 2 < 8) kf[j + 2] = *reinterpret_cast<lds_u32x4>(kb + f.k[j + 2]);
+      sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kf[j]), w.qf[j], sn, 0, 0, 0);
+    }
+    if (SM) {
+      const float a = __builtin_amdgcn_exp2f(fmaf(sp[2 * j], c, -mu));
+      const float b = __builtin_amdgcn_exp2f(fmaf(sp[2 * j + 1], c, -mu));
+      l4[j >> 1] = (j & 1) ? l4[j >> 1] + (a + b) : a + b;
+      uint32_t pk = pack_bf16x2(a, b);
+      asm volatile("" : "+v"(pk));  // kept here, not sunk to its use a stage later
+      pn[j >> 2][j & 3] = pk;
+    }
+    if (PV) {
+      if (j + 2 < 8) va[j + 2] = vt_frag(vb, f, (j + 2) >> 2, (j + 2) & 3);
+      w.o[j & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[j], as_bf16x8(pp[j >> 2]), w.o[j & 3],
+                                                           0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  ps.alpha = 1.f;
+  if (SM) {
+    const float lsum = (l4[0] + l4[1]) + (l4[2] + l4[3]);
+    if (__builtin_expect(ps.have_ref && __ballot(lsum < kLazyLimit) == ~0ull, 1))
+      w.l_run += lsum;
+    else if (lim > 0)
+      raise_reference(sp, c, pn, w, ps);
   }
 }
 
@@ -1174,11 +1117,14 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
   WaveState w;
   const uint16_t* qptr = p.q + qrow * p.qs + head * p.qh;
   bool q_live = !DENSE || qrow < p.used;
+  // sequence order: where the lane's output row goes (nowhere for padding)
+  uint16_t* orow_seq = nullptr;
   if (MODE == kSparse && p.seq_q != nullptr) {
-    const int64_t sh = p.seq_heads[head], src = p.seq_q[qrow];
-    q_live = p.slot_ok[qrow] != 0 && src >= 0 && src < p.seq_rows && sh >= 0 &&
-             sh < p.seq_heads_n;
+    const int64_t sh = p.seq_heads[head], src = p.seq_q[qrow], dst = p.seq_o[qrow];
+    const bool slot = p.slot_ok[qrow] != 0 && sh >= 0 && sh < p.seq_heads_n;
+    q_live = slot && src >= 0 && src < p.seq_rows;
     qptr = p.q + (q_live ? src : 0) * p.qs + (q_live ? sh : 0) * p.qh;
+    if (slot && dst >= 0 && dst < p.out_rows) orow_seq = p.out + dst * p.os + sh * p.oh;
   }
 #pragma unroll
   for (int s = 0; s < 8; ++s)
@@ -1399,6 +1345,9 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
 
 #pragma unroll
   for (int s = 0; s < 8; ++s) asm volatile("" : : "v"(w.qf[s]));
+  // a wave none of whose rows is stored (sequence order: all 32 slots are
+  // padding, whose rows the scatter drops)
+  const bool dead = MODE == kSparse && p.seq_q != nullptr && __ballot(orow_seq != nullptr) == 0;
   // a wave whose 32 query rows are all zero (padding rows) takes the
   // product-free step (wave-uniform)
   bool q_zero = false;
@@ -1410,7 +1359,8 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
       any |= x[0] | x[1] | x[2] | x[3];
     }
     q_zero = __ballot(any != 0) == 0;
-    if ((MODE == kSparse || MODE == kVirtualOnly) && lane == 0) zflag[wave] = q_zero ? 1 : 0;
+    if ((MODE == kSparse || MODE == kVirtualOnly) && lane == 0)
+      zflag[wave] = (q_zero ? 1 : 0) | (dead ? 2 : 0);
     // wave 0's Q fragments for wave 1 of a narrow walk (below), in ring
     // slot 1 past the step-list scratch; no load reaches slot 1 before the
     // walk's first barrier
@@ -1427,6 +1377,7 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
     for (int e = 0; e < 16; ++e) w.o[dt][e] = 0.f;
   w.m_run = -INFINITY;
   w.l_run = 0.f;
+  w.mu = 0.f;
   // compensation of a given output: the row's fixed reference (0 for a row
   // that kept nothing)
   const float ref2 =
@@ -1435,17 +1386,29 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
   // All-zero query groups of one tile have the same output and LSE (the
   // uniform average over the tile's valid kept keys, the same products in
   // the same order): the first such wave computes it, the others ("copy"
-  // waves) only load and pass the barriers, then store its staged rows.
+  // waves) only load and pass the barriers, then store its staged rows. A
+  // wave that stores nothing (dead) only loads; in a narrow walk, where waves
+  // 2 and 3 work for all all-zero rows, only if no such row is stored.
   int zero_src = 0;
   bool copy = false, has_copy = false;  // has_copy: workgroup-uniform
   bool narrow = false;                  // workgroup-uniform
+  bool drop = false;  // this wave only loads and passes the barriers, and stores nothing
+  uint32_t dbits = 0;
   if (MODE == kSparse) {
-    const uint32_t zbits = __builtin_amdgcn_readfirstlane(
-        (uint32_t)zflag[0] | ((uint32_t)zflag[1] << 1) | ((uint32_t)zflag[2] << 2) |
-        ((uint32_t)zflag[3] << 3));
-    zero_src = zbits ? __builtin_ctz(zbits) : 0;
-    copy = q_zero && wave != zero_src;
-    has_copy = __builtin_popcount(zbits) >= 2;
+    const uint32_t flags = __builtin_amdgcn_readfirstlane(
+        (uint32_t)zflag[0] | ((uint32_t)zflag[1] << 2) | ((uint32_t)zflag[2] << 4) |
+        ((uint32_t)zflag[3] << 6));
+    uint32_t zbits = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      zbits |= ((flags >> (2 * i)) & 1u) << i;
+      dbits |= ((flags >> (2 * i + 1)) & 1u) << i;
+    }
+    const uint32_t live = zbits & ~dbits;  // all-zero groups with a row to store
+    zero_src = live ? __builtin_ctz(live) : 0;
+    drop = dead;
+    copy = q_zero && !dead && wave != zero_src;
+    has_copy = __builtin_popcount(live) >= 2;
     narrow = zbits == 0xEu;
   }
   const int n_lsteps = __builtin_amdgcn_readfirstlane(step_total);
@@ -1457,8 +1420,11 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
   // output and waves 1 and 3 copy it.
   narrow = narrow && n_lsteps > 0;
   if (narrow) {
+    const bool none = (dbits & 0xEu) == 0xEu;  // no all-zero row is stored
     zero_src = 2;
-    copy = (wave & 1) != 0;
+    copy = !none && (wave & 1) != 0;
+    has_copy = !none;
+    drop = none && wave >= 2;
     if (wave == 1) {
 #pragma unroll
       for (int s = 0; s < 8; ++s)
@@ -1494,76 +1460,18 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
     }
   }
 
-  // Step u of the virtual and dense walks (the list walk decodes its own
-  // steps): sub-block a is key rows row0 .. + 31 with la valid keys, sub-block
-  // b rows rowb .. + 31 with lb (as sub_scores' lim). Steps n_lsteps .. are
-  // virtual.
-  auto decode = [&](int u, int64_t& row0, int& la, int64_t& rowb, int& lb) {
-    if (VKEYS && u >= n_lsteps) {
-      const int v = u - n_lsteps;
-      row0 = (int64_t)v * kHalf;
-      la = min(nk - v * kHalf, kHalf);
-    } else if (DENSE) {
-      row0 = (int64_t)u * kHalf;
-      la = (int)min(p.used - row0, (int64_t)kHalf);
-    } else {
-      row0 = 0;
-      la = 0;
-    }
-    rowb = row0 + 32;
-    lb = la - 32;
-  };
   const uint16_t* kbase = p.k + head * p.kh;
   const uint16_t* vbase = p.v + head * p.vh;
   const float c = p.scale_log2;
   const SDma dma = sdma_offsets(p.ks, p.vs, wave, lane);
   const HFrag fa = hfrag_offsets(0, lane), fb = hfrag_offsets(1, lane);
-  const HFrag fh = hfrag_offsets(wave & 1, lane);  // a narrow walk's sub-block
-  auto load_step = [&](int u, lds_u8* slot) {
-    int64_t row0, rowb;
-    int vch, lb;
-    decode(u, row0, vch, rowb, lb);
-    if (VKEYS && u >= n_lsteps) {
-      load_virtual(u - n_lsteps, slot);
-      return;
-    }
-    if (DENSE && vch < kHalf) {
-      const char* kb = reinterpret_cast<const char*>(kbase + row0 * p.ks);
-      const char* vb = reinterpret_cast<const char*>(vbase + row0 * p.vs);
-      // the last dense step: rows past `used` may not exist, so every lane
-      // reads a row below vch (masked keys)
-      const int lr = lane >> 4, pc = lane & 15;
-#pragma unroll
-      for (int u4 = 0; u4 < 4; ++u4) {
-        const int seg = 4 * wave + u4, row = 4 * seg + lr, src = min(row, vch - 1);
-        const uint32_t ko = (uint32_t)((src * p.ks + ((pc ^ (row & 15)) << 3)) * 2);
-        const uint32_t vo = (uint32_t)((src * p.vs + ((pc ^ ((row & 3) << 2)) << 3)) * 2);
-        dma16(kb, ko, slot + seg * 1024);
-        dma16(vb, vo, slot + kHalfBytes + seg * 1024);
-      }
-      return;
-    }
-    // waves 0, 1: sub-block a from row0; waves 2, 3: sub-block b from rowb.
-    // Segments past a sub-block's valid keys reload its first rows (not
-    // read: masked), so every wave issues the same loads.
-    const bool wa = wave < 2;
-    const int64_t base = wa ? row0 : rowb;
-    const int lim = wa ? vch : lb + 32;
-    const char* kb = reinterpret_cast<const char*>(kbase + base * p.ks);
-    const char* vb = reinterpret_cast<const char*>(vbase + base * p.vs);
-#pragma unroll
-    for (int u4 = 0; u4 < 4; ++u4) {
-      const int seg = 4 * wave + u4;
-      const bool live = 4 * seg < lim;
-      dma16(kb, live ? dma.k[u4] : dma.k_skip[u4], slot + seg * 1024);
-      dma16(vb, live ? dma.v[u4] : dma.v_skip[u4], slot + kHalfBytes + seg * 1024);
-    }
-  };
+  const HFrag fh = hfrag_offsets(wave & 1, lane);  // a narrow compensation's sub-block
   lds_u8* s0 = (lds_u8*)ring[0];
   lds_u8* s1 = (lds_u8*)ring[1];
-  // Step u: wait for its own loads (the only ones in flight), barrier (all
+  // The virtual steps (the list and dense walks have their own): step u waits
+  // for its own loads (the only ones in flight), then the barrier (all
   // waves' loads of step u are in LDS and all are done reading the other
-  // slot), issue step u + 1 into the other slot, compute step u.
+  // slot), issues step u + 1 into the other slot and computes step u.
   // Compensation of a given output: o_kept's rows go to LDS as whole rows
   // during the last step (into the slot the epilogue stages the output in,
   // each wave its own 8 KB, with the output's layout) when every row start
@@ -1583,7 +1491,7 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
     VEDA_WAIT_VM(0);
     __builtin_amdgcn_s_barrier();
     if (u + 1 < n_steps)
-      load_step(u + 1, nxt);
+      load_virtual(u + 1 - n_lsteps, nxt);
     else if (kept_lds)
       load_kept(nxt);
   };
@@ -1649,240 +1557,220 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
       ra = (uint32_t)__builtin_amdgcn_readlane((int)win_a, u & 63);
       rb = (uint32_t)__builtin_amdgcn_readlane((int)win_b, u & 63);
     };
-    // A step's loads: waves 0, 1 load sub-block a, waves 2, 3 sub-block b,
-    // rows 16 (wave & 1) .. + 15 of it as four 1 KB segments of K and four of
-    // V, with no branch. Segments past the sub-block's valid keys load the
-    // key tile's own padding rows, as the reference's kernel reads them (they
-    // are masked: the scores become -inf, the probabilities exactly 0); at
-    // C2 they are 0.5 % of the segments.
-    auto rec_base = [&](uint32_t ra, uint32_t rb, const char*& kb, const char*& vb) {
-      const int64_t base = (int64_t)((wave < 2 ? ra : rb) >> 6);
-      kb = reinterpret_cast<const char*>(kbase + base * p.ks);
-      vb = reinterpret_cast<const char*>(vbase + base * p.vs);
+    // The walk. K and V of step u have their halves of slot u % 2, and V runs
+    // one step behind K: iteration u multiplies K of step u + 1 and V of step
+    // u, and issues K of step u + 2 (into the half every wave was done with
+    // at the iteration's barrier: K of step u) and V of step u + 1. So a load
+    // has the whole iteration to arrive, as long as when a step's K and V are
+    // loaded together. Past the last step the last one's rows are loaded
+    // again, so every iteration issues the same eight loads per wave with no
+    // branch (a branch between the products would split the stage, and the
+    // compiler then moves the softmax out of it).
+    //
+    // Waves 0, 1 load sub-block a, waves 2, 3 sub-block b, rows 16 (wave & 1)
+    // .. + 15 of it as four 1 KB segments of K and four of V. Segments past
+    // the sub-block's valid keys load the key tile's own padding rows, as the
+    // reference's kernel reads them (they are masked: the scores become -inf,
+    // the probabilities exactly 0); at C2 they are 0.5 % of the segments.
+    //
+    // Sequence-order k / v (SEQKV): segment u4's row of lane l is slot row
+    // 16 (wave & 1) + 4 u4 + l / 16 of the sub-block; it is read from the row
+    // its slot gathers (the low word of the int64 gather index), and a row
+    // past the sub-block's valid keys (padding, masked) from the sub-block's
+    // first row, a real row of the same key tile (so a non-finite value there
+    // reaches only query tiles that keep the block, as in the tiled form).
+    // The rows are looked up an iteration before their K loads are issued.
+    struct Rec {
+      uint32_t a, b;  // records of sub-blocks a and b
     };
-    // load j of a step: K segment j (j < 4) or V segment j - 4, into the
-    // slot whose segment 4 wave (this wave's first) is at LDS address lds
-    auto issue = [&](const char* kb, const char* vb, int j, uint32_t lds) {
-      const int u4 = j & 3;
-      if (j < 4)
-        dma16_m0(kb, dma.k[u4], lds + u4 * 1024);
-      else
-        dma16_m0(vb, dma.v[u4], lds + kHalfBytes + u4 * 1024);
+    auto fetch_rec = [&](int u, Rec last) {
+      Rec r = last;
+      if (u < n_lsteps) fetch(u, r.a, r.b);
+      return r;
     };
     // this wave's first segment of each slot, as LDS addresses
     const uint32_t lds_s0 = __builtin_amdgcn_readfirstlane(
         (uint32_t)(uintptr_t)(s0 + 4 * wave * 1024));
     const uint32_t lds_s1 = __builtin_amdgcn_readfirstlane(
         (uint32_t)(uintptr_t)(s1 + 4 * wave * 1024));
-    // Step (ra, rb) from `cur`, with the loads of step (na, nb) into `nxt`
-    // (unless it is the last step) issued between its products, so a load
-    // that waits for the CU's load path waits beside this wave's own running
-    // products. Issued in one burst after the barrier, the loads of all
-    // eight waves of a CU queue at the load path together and each wave
-    // stalls on them.
-    // kind: 0 a wave with a real query row, 1 the wave that computes the
-    // all-zero groups' output, 2 a copy wave (loads only); in a narrow
-    // walk, 3 a wave with the tile's real rows over one sub-block and 4 the
-    // all-zero rows over one sub-block
-    // Compensated attention: the last list step loads the first virtual
-    // step (the tile summaries) instead.
-    const bool virt_next = MODE == kSparseComp && n_virt > 0;
-    auto step = [&](auto kind, bool more, uint32_t ra, uint32_t rb, const lds_u8* cur,
-                    uint32_t na, uint32_t nb, uint32_t nxt, lds_u8* nxt_slot)
-        __attribute__((always_inline)) {
-      const int la = (int)(ra & 63u), lb = (int)(rb & 63u);
-      const char *kb, *vb;
-      rec_base(na, nb, kb, vb);
-      if constexpr (decltype(kind)::value == 3) {
-        sstep_half(cur, fh, c, (wave & 1) ? lb : la, hi, w, [&](int k) {
-          if (more) issue(kb, vb, k, nxt);
-        });
-      } else if constexpr (decltype(kind)::value != 0) {
-        if (more) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) issue(kb, vb, j, nxt);
-        } else if (virt_next) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) virtual_seg(0, nxt_slot, j);
-        }
-        if constexpr (decltype(kind)::value == 1) sstep_zero_q(cur, fa, fb, la, lb, hi, w);
-        if constexpr (decltype(kind)::value == 4) sstep_half_zero(cur, fh, (wave & 1) ? lb : la, hi, w);
-      } else {
-        sstep(cur, fa, fb, c, la, lb, hi, w, [&](int k) {
-          if (more) issue(kb, vb, k, nxt);
-          else if (virt_next) virtual_seg(0, nxt_slot, k);
-        });
-      }
-    };
-    // A copy of the walk per kind of wave (same loads and barriers), so
-    // each keeps O in one set of registers. Step u computes from slot u % 2
-    // and loads step u + 1 into the other.
-    auto walk = [&](auto zero) __attribute__((always_inline)) {
-      uint32_t ca = 0, cb = 0;
-      if (n_lsteps > 0) {
-        fetch(0, ca, cb);
-        const char *kb, *vb;
-        rec_base(ca, cb, kb, vb);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) issue(kb, vb, j, lds_s0);
-      } else if (virt_next) {
-        load_virtual(0, s0);
-      }
-      for (int u = 0; u < n_lsteps; u += 2) {
-        uint32_t na = 0, nb = 0;
-        VEDA_WAIT_VM(0);
-        __builtin_amdgcn_s_barrier();
-        const bool more1 = u + 1 < n_lsteps;
-        if (more1) fetch(u + 1, na, nb);
-        step(zero, more1, ca, cb, s0, na, nb, lds_s1, s1);
-        if (!more1) break;
-        VEDA_WAIT_VM(0);
-        __builtin_amdgcn_s_barrier();
-        const bool more2 = u + 2 < n_lsteps;
-        if (more2) fetch(u + 2, ca, cb);
-        step(zero, more2, na, nb, s1, ca, cb, lds_s0, s0);
-      }
-    };
-    // Sequence-order k / v: this wave's four segments of a step are rows
-    // 16 (wave & 1) + 4 u4 + lane / 16 of its sub-block; each is read from
-    // the row its slot gathers (the low word of the int64 gather index),
-    // and a row past the sub-block's valid keys (padding, masked) from the
-    // sub-block's first row, a real row of the same key tile (so a
-    // non-finite value there reaches only query tiles that keep the block,
-    // as in the tiled form). The rows of step u + 2 are looked up during
-    // step u, so the step's loads wait for no lookup.
     const int32_t* tok_of = reinterpret_cast<const int32_t*>(p.seq_q);
     const int kv_head = SEQKV ? (int)min(max(p.seq_heads[head], (int64_t)0), p.seq_heads_n - 1) : 0;
     const char* kseq = reinterpret_cast<const char*>(p.k + (int64_t)kv_head * p.kh);
     const char* vseq = reinterpret_cast<const char*>(p.v + (int64_t)kv_head * p.vh);
-    auto tokens = [&](uint32_t ra, uint32_t rb, int32_t (&t)[4]) {
-      const uint32_t rec = wave < 2 ? ra : rb;
-      const int64_t base = (int64_t)(rec >> 6);
-      const int lim = (int)(rec & 63u);
+    struct Rows {
+      uint32_t r[4];  // sequence row (looked up), then its byte offset
+    };
+    auto lookup = [&](Rec rec) {
+      Rows t;
+      const uint32_t x = wave < 2 ? rec.a : rec.b;
+      const int64_t base = (int64_t)(x >> 6);
+      const int lim = (int)(x & 63u);
 #pragma unroll
       for (int u4 = 0; u4 < 4; ++u4) {
         const int src = 16 * (wave & 1) + 4 * u4 + (lane >> 4);
-        t[u4] = tok_of[2 * (base + (src < lim ? src : 0))];
+        t.r[u4] = (uint32_t)tok_of[2 * (base + (src < lim ? src : 0))];
       }
+      return t;
     };
     // byte offset of a row: row * (2 stride_s) fits 32 bits (the launcher
-    // checks), k and v share the stride; the chunk swizzles of the slot rows
-    // are per-lane constants
+    // checks), k and v share the stride
     const uint32_t row_bytes = (uint32_t)(2 * p.ks);
     const uint32_t n_rows = (uint32_t)p.seq_rows;
-    uint32_t kswz[4], vswz[4];
+    auto bytes = [&](const Rows& t) {
+      Rows o;
 #pragma unroll
-    for (int u4 = 0; u4 < 4; ++u4) {
-      const int pc = lane & 15, row = 4 * (4 * wave + u4) + (lane >> 4);  // slot row
-      kswz[u4] = (uint32_t)((pc ^ (row & 15)) << 4);
-      vswz[u4] = (uint32_t)((pc ^ ((row & 3) << 2)) << 4);
-    }
-    auto offsets = [&](const int32_t (&t)[4], uint32_t (&ok)[4], uint32_t (&ov)[4]) {
-#pragma unroll
-      for (int u4 = 0; u4 < 4; ++u4) {
-        const uint32_t tk = (uint32_t)t[u4] < n_rows ? (uint32_t)t[u4] : 0u;
-        const uint32_t b = tk * row_bytes;
-        ok[u4] = b + kswz[u4];
-        ov[u4] = b + vswz[u4];
-      }
+      for (int u4 = 0; u4 < 4; ++u4) o.r[u4] = (t.r[u4] < n_rows ? t.r[u4] : 0u) * row_bytes;
+      return o;
     };
-    auto issue_kv = [&](const uint32_t (&ok)[4], const uint32_t (&ov)[4], int j, uint32_t lds) {
+    // chunk swizzle of slot row 16 wave + 4 u4 + l / 16: K's is kswz0 with u4
+    // xored into its bits 2, 3 (of the chunk), V's does not depend on u4
+    const uint32_t kswz0 = (uint32_t)(((lane & 15) ^ (lane >> 4)) << 4);
+    const uint32_t vswz = (uint32_t)(((lane & 15) ^ ((lane >> 4) << 2)) << 4);
+    // load j of an iteration: K segment j of step u + 2 (j < 4), V segment
+    // j - 4 of step u + 1, from base kb / vb (tile order) or rows ok / ov
+    auto issue = [&](const char* kb, const char* vb, const Rows& ok, const Rows& ov, int j,
+                     uint32_t lk, uint32_t lv) {
       const int u4 = j & 3;
-      if (j < 4)
-        dma16_m0(kseq, ok[u4], lds + u4 * 1024);
-      else
-        dma16_m0(vseq, ov[u4], lds + kHalfBytes + u4 * 1024);
-    };
-    auto step_kv = [&](auto kind, bool more, uint32_t ra, uint32_t rb, const lds_u8* cur,
-                       const uint32_t (&ok)[4], const uint32_t (&ov)[4], uint32_t nxt)
-        __attribute__((always_inline)) {
-      const int la = (int)(ra & 63u), lb = (int)(rb & 63u);
-      if constexpr (decltype(kind)::value == 3) {
-        sstep_half(cur, fh, c, (wave & 1) ? lb : la, hi, w, [&](int k) {
-          if (more) issue_kv(ok, ov, k, nxt);
-        });
-      } else if constexpr (decltype(kind)::value != 0) {
-        if (more) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) issue_kv(ok, ov, j, nxt);
-        }
-        if constexpr (decltype(kind)::value == 1) sstep_zero_q(cur, fa, fb, la, lb, hi, w);
-        if constexpr (decltype(kind)::value == 4) sstep_half_zero(cur, fh, (wave & 1) ? lb : la, hi, w);
+      if (SEQKV) {
+        if (j < 4)
+          dma16_m0(kseq, ok.r[u4] + (kswz0 ^ (uint32_t)(u4 << 6)), lk + u4 * 1024);
+        else
+          dma16_m0(vseq, ov.r[u4] + vswz, lv + kHalfBytes + u4 * 1024);
       } else {
-        sstep(cur, fa, fb, c, la, lb, hi, w, [&](int k) {
-          if (more) issue_kv(ok, ov, k, nxt);
-        });
+        if (j < 4)
+          dma16_m0(kb, dma.k[u4], lk + u4 * 1024);
+        else
+          dma16_m0(vb, dma.v[u4], lv + kHalfBytes + u4 * 1024);
       }
     };
-    // the walk above with sequence-order k / v; (ra0, rb0) and (ra1, rb1)
-    // are the records of steps u and u + 1, tk the rows of the next step
-    // whose loads are not issued yet
-    auto walk_kv = [&](auto zero) __attribute__((always_inline)) {
-      uint32_t ra0 = 0, rb0 = 0, ra1 = 0, rb1 = 0;
-      int32_t tk[4] = {0, 0, 0, 0};
-      uint32_t ok[4], ov[4];
-      if (n_lsteps > 0) {
-        fetch(0, ra0, rb0);
-        tokens(ra0, rb0, tk);
-        offsets(tk, ok, ov);
+    auto k_base = [&](Rec r) {
+      const int64_t row = (int64_t)((wave < 2 ? r.a : r.b) >> 6);
+      return reinterpret_cast<const char*>(kbase + row * p.ks);
+    };
+    auto v_base = [&](Rec r) {
+      const int64_t row = (int64_t)((wave < 2 ? r.a : r.b) >> 6);
+      return reinterpret_cast<const char*>(vbase + row * p.vs);
+    };
+    auto sync = [&]() {
+      VEDA_WAIT_VM(0);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");  // no LDS read of the new step above the barrier
+    };
+    // A copy of the walk per kind of wave (same loads and barriers), so each
+    // keeps O in one set of registers. Kind: 0 a wave with a real query row,
+    // 1 the wave that computes the all-zero groups' output, 2 a copy wave
+    // (loads only); in a narrow walk, 3 a wave with the tile's real rows over
+    // one sub-block and 4 the all-zero rows over one sub-block.
+    const bool virt_next = MODE == kSparseComp && n_virt > 0;
+    auto walk = [&](auto kind) __attribute__((always_inline)) {
+      constexpr int K = decltype(kind)::value;
+      if (n_lsteps == 0) {
+        if (virt_next) load_virtual(0, s0);
+        return;
+      }
+      Rec r0 = fetch_rec(0, Rec{0, 0}), r1 = fetch_rec(1, r0), r2;
+      Rows o1{}, t2{};  // V offsets of step u + 1, rows of step u + 2
+      {
+        Rows o0{};
+        if (SEQKV) {
+          const Rows t0 = lookup(r0), t1 = lookup(r1);
+          o0 = bytes(t0);
+          o1 = bytes(t1);
+        }
+        const char *k0 = k_base(r0), *k1 = k_base(r1), *v0 = v_base(r0);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) issue_kv(ok, ov, j, lds_s0);
-      }
-      if (n_lsteps > 1) {
-        fetch(1, ra1, rb1);
-        tokens(ra1, rb1, tk);
-      }
-      for (int u = 0; u < n_lsteps; u += 2) {
-        VEDA_WAIT_VM(0);
+        for (int j = 0; j < 4; ++j) issue(k0, v0, o0, o0, j, lds_s0, lds_s0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) issue(k1, v0, o1, o0, j, lds_s1, lds_s0);
+#pragma unroll
+        for (int j = 4; j < 8; ++j) issue(k1, v0, o1, o0, j, lds_s1, lds_s0);
+        r2 = fetch_rec(2, r1);
+        VEDA_WAIT_VM(8);  // K of step 0; K of step 1 and V of step 0 may be in flight
         __builtin_amdgcn_s_barrier();
-        const bool more1 = u + 1 < n_lsteps;
-        uint32_t ra2 = 0, rb2 = 0;
-        if (more1) offsets(tk, ok, ov);  // step u + 1
-        if (u + 2 < n_lsteps) {
-          fetch(u + 2, ra2, rb2);
-          tokens(ra2, rb2, tk);
+        asm volatile("" ::: "memory");
+        if (SEQKV) t2 = lookup(r2);
+      }
+      f32x16 sa, sb;
+      u32x4 pa[2], pb[2];
+      PipeState ps{1.f, false};
+      const lds_u8* const kz = s0;  // unused operands of partial stages
+      const int h = 8192 * (wave & 1);  // a narrow wave's sub-block
+      if constexpr (K == 0) {
+        pstage<true, false, false>(s0, kz, fa, c, 32, hi, sa, sb, pb, pa, w, ps, NoHook{});
+        pstage<true, true, false>(s0 + 8192, kz, fa, c, (int)(r0.a & 63u), hi, sb, sa, pa, pb, w, ps,
+                                  NoHook{});
+      } else if constexpr (K == 3) {
+        pstage<true, false, false>(s0 + h, kz, fa, c, 32, hi, sa, sb, pb, pa, w, ps, NoHook{});
+      }
+      // iteration u < n - 1: K of step u + 1 in nxt, V of step u in cur
+      auto iter = [&](lds_u8* cur, lds_u8* nxt, uint32_t lcur, uint32_t lnxt, int u)
+          __attribute__((always_inline)) {
+        // addresses and records first: after the barrier every wave goes
+        // straight to its fragment reads
+        const Rec r3 = fetch_rec(u + 3, r2);
+        const char *kb = k_base(r2), *vb = v_base(r1);
+        Rows o2{};
+        if (SEQKV) o2 = bytes(t2);
+        const Rows ov = o1;
+        sync();
+        if (SEQKV) t2 = lookup(r3);
+        auto hook = [&](int j) { issue(kb, vb, o2, ov, j, lcur, lnxt); };
+        const int la0 = (int)(r0.a & 63u), lb0 = (int)(r0.b & 63u), la1 = (int)(r1.a & 63u);
+        if constexpr (K == 0) {
+          pstage<true, true, true>(nxt, cur, fa, c, lb0, hi, sa, sb, pb, pa, w, ps, hook);
+          pstage<true, true, true>(nxt + 8192, cur + 8192, fa, c, la1, hi, sb, sa, pa, pb, w, ps,
+                                   NoHook{});
+        } else if constexpr (K == 3) {
+          pstage<true, true, false>(nxt + h, kz, fa, c, (wave & 1) ? lb0 : la0, hi, sb, sa, pa, pb, w,
+                                    ps, hook);
+          pstage<false, false, true>(kz, cur + h, fa, c, 32, hi, sb, sa, pb, pa, w, ps, NoHook{});
+          sa = sb;
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) hook(j);
+          if constexpr (K == 1) sstep_zero_q(cur, fa, la0, lb0, hi, w);
+          if constexpr (K == 4) sstep_half_zero(cur + h, fa, (wave & 1) ? lb0 : la0, hi, w);
         }
-        step_kv(zero, more1, ra0, rb0, s0, ok, ov, lds_s1);
-        if (!more1) break;
-        VEDA_WAIT_VM(0);
-        __builtin_amdgcn_s_barrier();
-        const bool more2 = u + 2 < n_lsteps;
-        uint32_t ra3 = 0, rb3 = 0;
-        if (more2) offsets(tk, ok, ov);  // step u + 2
-        if (u + 3 < n_lsteps) {
-          fetch(u + 3, ra3, rb3);
-          tokens(ra3, rb3, tk);
-        }
-        step_kv(zero, more2, ra1, rb1, s1, ok, ov, lds_s0);
-        ra0 = ra2;
-        rb0 = rb2;
-        ra1 = ra3;
-        rb1 = rb3;
+        r0 = r1;
+        r1 = r2;
+        r2 = r3;
+        o1 = o2;
+      };
+      int u = 0;
+      for (; u + 2 < n_lsteps; u += 2) {
+        iter(s0, s1, lds_s0, lds_s1, u);
+        iter(s1, s0, lds_s1, lds_s0, u + 1);
+      }
+      if (u + 1 < n_lsteps) iter(s0, s1, lds_s0, lds_s1, u);
+      // the last iteration: V of the last step in its slot
+      lds_u8* const cur = s0 + ((n_lsteps - 1) & 1) * kSlotBytes;
+      sync();
+      if (virt_next) load_virtual(0, s0 + (n_lsteps & 1) * kSlotBytes);
+      const int la0 = (int)(r0.a & 63u), lb0 = (int)(r0.b & 63u);
+      if constexpr (K == 0) {
+        pstage<false, true, true>(kz, cur, fa, c, lb0, hi, sa, sb, pb, pa, w, ps, NoHook{});
+        pstage<false, false, true>(kz, cur + 8192, fa, c, 32, hi, sb, sa, pa, pb, w, ps, NoHook{});
+      } else if constexpr (K == 3) {
+        pstage<false, true, false>(kz, kz, fa, c, (wave & 1) ? lb0 : la0, hi, sb, sa, pa, pb, w, ps,
+                                   NoHook{});
+        pstage<false, false, true>(kz, cur + h, fa, c, 32, hi, sb, sa, pb, pa, w, ps, NoHook{});
+      } else {
+        if constexpr (K == 1) sstep_zero_q(cur, fa, la0, lb0, hi, w);
+        if constexpr (K == 4) sstep_half_zero(cur + h, fa, (wave & 1) ? lb0 : la0, hi, w);
       }
     };
-    if constexpr (SEQKV) {
-      if (narrow && wave < 2)
-        walk_kv(std::integral_constant<int, 3>{});
-      else if (narrow)
-        walk_kv(std::integral_constant<int, 4>{});
-      else if (copy)
-        walk_kv(std::integral_constant<int, 2>{});
-      else if (q_zero)
-        walk_kv(std::integral_constant<int, 1>{});
-      else
-        walk_kv(std::integral_constant<int, 0>{});
-    } else {
-      if (narrow && wave < 2)
-        walk(std::integral_constant<int, 3>{});
-      else if (narrow)
-        walk(std::integral_constant<int, 4>{});
-      else if (copy)
-        walk(std::integral_constant<int, 2>{});
-      else if (q_zero)
-        walk(std::integral_constant<int, 1>{});
-      else
-        walk(std::integral_constant<int, 0>{});
-    }
+    if (narrow && wave < 2)
+      walk(std::integral_constant<int, 3>{});
+    else if (drop)
+      walk(std::integral_constant<int, 2>{});
+    else if (narrow)
+      walk(std::integral_constant<int, 4>{});
+    else if (copy)
+      walk(std::integral_constant<int, 2>{});
+    else if (q_zero)
+      walk(std::integral_constant<int, 1>{});
+    else
+      walk(std::integral_constant<int, 0>{});
     if constexpr (MODE == kSparseComp) {
       // a row that kept nothing: the reference's unit mass at reference 0
       // (a select, not a branch: the condition is per row)
@@ -1911,46 +1799,115 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
       }
     }
   } else {
-  if (n_steps > 0 && MODE != kVirtualOnly) load_step(0, s0);  // kVirtualOnly: issued at set-up
   if constexpr (DENSE) {
-    // Dense walk: step u is key rows 64 u .. of the used rows, from slot
-    // u % 2. It waits for its own loads and passes the barrier, then issues
-    // step u + 1's loads between its score products (as the sparse walk
-    // does), the last step's rows clamped to the used ones.
-    auto dstep = [&](int u, const lds_u8* cur, lds_u8* nxt) {
+    // Dense walk, the list walk's pipeline over key rows: step u is rows
+    // 64 u .. + 63 of the used rows, the last step the last 64 of them with
+    // the keys of the step before it masked (fewer than 64 rows in all: one
+    // step whose loads are clamped to them).
+    const int rem = (int)(p.used - (int64_t)(n_steps - 1) * kHalf);  // keys of the last step
+    const bool clamp = n_steps == 1 && rem < kHalf;
+    const int lr = lane >> 4, pc = lane & 15;
+    const uint32_t lds_s0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(s0 + 4096 * wave));
+    const uint32_t lds_s1 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(s1 + 4096 * wave));
+    // first row of step u for this wave's loads (its offsets count from row
+    // 0 of the step for waves 0, 1 and from row 32 for waves 2, 3); past the
+    // last step the last one again
+    auto row_of = [&](int u) {
+      const int64_t row = min((int64_t)u * kHalf, max(p.used - kHalf, (int64_t)0));
+      return row + (wave >= 2 ? 32 : 0);
+    };
+    auto k_base = [&](int u) { return reinterpret_cast<const char*>(kbase + row_of(u) * p.ks); };
+    auto v_base = [&](int u) { return reinterpret_cast<const char*>(vbase + row_of(u) * p.vs); };
+    // load j of an iteration: K segment j (j < 4) or V segment j - 4
+    auto issue = [&](const char* kb, const char* vb, int j, uint32_t lk, uint32_t lv) {
+      if (j < 4)
+        dma16_m0(kb, dma.k[j], lk + j * 1024);
+      else
+        dma16_m0(vb, dma.v[j - 4], lv + kHalfBytes + (j - 4) * 1024);
+    };
+    // keys 32 sub .. of step u: the count from the front that is masked (the
+    // last step holds `rem` new keys, at its end), or for the clamped step
+    // the count that is valid
+    auto mask_front = [&](f32x16& s, int u, int sub) {
+      if (u != n_steps - 1 || rem == kHalf) return;
+      if (clamp) {
+        mask_scores(s, rem - 32 * sub, hi);
+        return;
+      }
+      const int l = kHalf - rem - 32 * sub - 4 * hi;
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (8 * (e >> 2) + (e & 3) < l) s[e] = -INFINITY;
+    };
+    f32x16 sa, sb;
+    u32x4 pa[2], pb[2];
+    PipeState ps{1.f, false};
+    auto sync = [&]() {
       VEDA_WAIT_VM(0);
       __builtin_amdgcn_s_barrier();
-      const bool more = u + 1 < n_steps;
-      const int64_t row0 = (int64_t)u * kHalf;
-      const int vch = (int)min(p.used - row0, (int64_t)kHalf);
-      const int64_t nrow0 = row0 + kHalf;
-      const int nvch = more ? (int)min(p.used - nrow0, (int64_t)kHalf) : 0;
-      // waves 0, 1 load sub-block a, waves 2, 3 sub-block b (rows from 32)
-      const int64_t nbase = nvch == kHalf && wave >= 2 ? nrow0 + 32 : nrow0;
-      const char* kb = reinterpret_cast<const char*>(kbase + nbase * p.ks);
-      const char* vb = reinterpret_cast<const char*>(vbase + nbase * p.vs);
-      const int lr = lane >> 4, pc = lane & 15;
-      auto hook = [&](int j) {
-        if (!more) return;
-        const int u4 = j & 3, seg = 4 * wave + u4;
-        lds_u8* dst = nxt + (j < 4 ? 0 : kHalfBytes) + seg * 1024;
-        if (nvch == kHalf) {
-          dma16(j < 4 ? kb : vb, j < 4 ? dma.k[u4] : dma.v[u4], dst);
-        } else {
-          // the last step: rows past `used` may not exist, so every lane
-          // reads a row below nvch (masked keys)
-          const int row = 4 * seg + lr, src = min(row, nvch - 1);
-          const uint32_t off = j < 4 ? (uint32_t)((src * p.ks + ((pc ^ (row & 15)) << 3)) * 2)
-                                     : (uint32_t)((src * p.vs + ((pc ^ ((row & 3) << 2)) << 3)) * 2);
-          dma16(j < 4 ? kb : vb, off, dst);
-        }
-      };
-      sstep(cur, fa, fb, c, vch, vch - 32, hi, w, hook);
+      asm volatile("" ::: "memory");
     };
-    for (int u = 0; u < n_steps; u += 2) {
-      dstep(u, s0, s1);
-      if (u + 1 >= n_steps) break;
-      dstep(u + 1, s1, s0);
+    const int64_t k_step = 2 * kHalf * p.ks, v_step = 2 * kHalf * p.vs;
+    const char *kp = k_base(2), *vp = v_base(1);
+    auto iter = [&](auto masked, int u, lds_u8* cur, lds_u8* nxt, uint32_t lcur, uint32_t lnxt)
+        __attribute__((always_inline)) {
+      // M: step u + 2 may be the last one; otherwise its rows follow the
+      // previous step's, and kp / vp walk along
+      constexpr bool M = decltype(masked)::value;
+      const char* kb = M ? k_base(u + 2) : kp;
+      const char* vb = M ? v_base(u + 1) : vp;
+      kp += k_step;
+      vp += v_step;
+      sync();
+      pstage<true, true, true>(nxt, cur, fa, c, 32, hi, sa, sb, pb, pa, w, ps,
+                               [&](int j) { issue(kb, vb, j, lcur, lnxt); });
+      if (M) mask_front(sa, u + 1, 0);
+      pstage<true, true, true>(nxt + 8192, cur + 8192, fa, c, 32, hi, sb, sa, pa, pb, w, ps,
+                               NoHook{});
+      if (M) mask_front(sb, u + 1, 1);
+    };
+    if (n_steps > 0) {
+      if (clamp) {
+#pragma unroll
+        for (int u4 = 0; u4 < 4; ++u4) {
+          const int row = 4 * (4 * wave + u4) + lr, src = min(row, rem - 1);
+          dma16(reinterpret_cast<const char*>(kbase),
+                (uint32_t)((src * p.ks + ((pc ^ (row & 15)) << 3)) * 2), s0 + (4 * wave + u4) * 1024);
+          dma16(reinterpret_cast<const char*>(vbase),
+                (uint32_t)((src * p.vs + ((pc ^ ((row & 3) << 2)) << 3)) * 2),
+                s0 + kHalfBytes + (4 * wave + u4) * 1024);
+        }
+        VEDA_WAIT_VM(0);
+      } else {
+        // K of step 0, then K of step 1 and V of step 0 in flight
+        const char *k0 = k_base(0), *k1 = k_base(1), *v0 = v_base(0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) issue(k0, v0, j, lds_s0, lds_s0);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) issue(k1, v0, j, lds_s1, lds_s0);
+        VEDA_WAIT_VM(8);
+      }
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      pstage<true, false, false>(s0, s0, fa, c, 32, hi, sa, sb, pb, pa, w, ps, NoHook{});
+      mask_front(sa, 0, 0);
+      pstage<true, true, false>(s0 + 8192, s0, fa, c, 32, hi, sb, sa, pa, pb, w, ps, NoHook{});
+      mask_front(sb, 0, 1);
+      int u = 0;
+      for (; u + 4 < n_steps; u += 2) {
+        iter(std::false_type{}, u, s0, s1, lds_s0, lds_s1);
+        iter(std::false_type{}, u + 1, s1, s0, lds_s1, lds_s0);
+      }
+#pragma unroll 1
+      for (; u + 1 < n_steps; ++u) {
+        const int o = (u & 1) * kSlotBytes;
+        iter(std::true_type{}, u, s0 + o, s0 + (kSlotBytes - o), lds_s0 + o,
+             lds_s0 + (kSlotBytes - o));
+      }
+      lds_u8* const cur = s0 + ((n_steps - 1) & 1) * kSlotBytes;
+      sync();
+      pstage<false, true, true>(s0, cur, fa, c, 32, hi, sa, sb, pb, pa, w, ps, NoHook{});
+      pstage<false, false, true>(s0, cur + 8192, fa, c, 32, hi, sb, sa, pa, pb, w, ps, NoHook{});
     }
   } else {
     // compensation of a given output: the virtual steps, step u in slot
@@ -2098,10 +2055,8 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
   uint16_t* orow = p.out + (row_exists ? qrow : 0) * p.os + head * p.oh;
   bool o_live = row_exists;
   if (MODE == kSparse && p.seq_o != nullptr) {
-    const int64_t sh = p.seq_heads[head], dst = p.seq_o[qrow];
-    o_live = p.slot_ok[qrow] != 0 && dst >= 0 && dst < p.out_rows && sh >= 0 &&
-             sh < p.seq_heads_n;
-    orow = p.out + (o_live ? dst : 0) * p.os + (o_live ? sh : 0) * p.oh;
+    o_live = orow_seq != nullptr;
+    orow = orow_seq;
   }
   const uint16_t* krow = MODE == kVirtualOnly ? p.o_kept + qrow * p.oks + head * p.okh : nullptr;
   // The output goes out as whole rows: each wave writes its 32 rows (bf16)
