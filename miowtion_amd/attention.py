@@ -135,6 +135,19 @@ def _chunk_heads(tile_layout: tiling.TileLayout, collect_bytes: int) -> int:
     return max(1, collect_bytes // (tile_layout.num_slots * _HEAD_DIM_BYTES))
 
 
+def _zeroed(out: torch.Tensor, groups, used: int) -> torch.Tensor:
+    """The [S + 1, H, D] scatter buffer with zeros wherever no kernel writes.
+    The reference zero-fills all of it (attention.py:732). When the plan's
+    groups hold every head, every (real row, head) is written (each real row
+    is one valid slot of every layout), so only rows [used, S] need the zeros;
+    the scatter never writes those."""
+    if sum(g.heads.numel() for g in groups) == out.shape[1]:
+        out[used:].zero_()
+    else:
+        out.zero_()
+    return out
+
+
 def _require_kernels(device: torch.device, who: str) -> None:
     if device.type != 'cuda':
         raise RuntimeError(f'{who} needs the HIP block-sparse kernels on a GPU, not {device}; '
@@ -176,24 +189,13 @@ class SparseStudent:
         self.calls['sparse'] += 1
         seq_len = q.shape[0]
         groups = self.plan.head_groups(layer_index, self.clip.device)
-        # The reference zero-fills the [S + 1, H, D] buffer (attention.py:732).
-        # When the plan's groups hold every head, every (real row, head) is
-        # written below (each real row is one valid slot of every layout), so
-        # only rows [used, S] need the zeros; the result is the same.
-        out = self._output_buffer(q, seq_len + 1)
-        if sum(g.heads.numel() for g in groups) == q.shape[1]:
-            out[used:].zero_()
-        else:
-            out.zero_()
+        out = _zeroed(self._output_buffer(q, seq_len + 1), groups, used)
         self.last = {}
         for group in groups:
             tile_layout = self.clip.get(group.shape)
             for heads in group.heads.split(_chunk_heads(tile_layout, self.clip.config.collect_bytes)):
                 self._attend(q, k, v, layer_index, tile_layout, heads, out)
-        out = out[:seq_len]
-        if used < seq_len:
-            out[used:] = 0
-        return out
+        return out[:seq_len]
 
     def _output_buffer(self, q: torch.Tensor, rows: int) -> torch.Tensor:
         """The [rows, H, D] scatter buffer, uninitialised (every row the
@@ -296,16 +298,14 @@ class OracleStudent:
             with torch.no_grad():
                 _, lse = kernels.dense_attention(q, k, v, used, return_lse=True)
         seq_len = q.shape[0]
-        out = q.new_zeros(seq_len + 1, *q.shape[1:])
+        groups = self.plan.head_groups(layer_index, self.clip.device)
+        out = _zeroed(q.new_empty(seq_len + 1, *q.shape[1:]), groups, used)
         self.last = {'lse': lse}
-        for group in self.plan.head_groups(layer_index, self.clip.device):
+        for group in groups:
             tile_layout = self.clip.get(group.shape)
             for heads in group.heads.split(_chunk_heads(tile_layout, self.clip.config.collect_bytes)):
                 self._attend(q, k, v, lse, tile_layout, heads, out)
-        out = out[:seq_len]
-        if used < seq_len:
-            out[used:] = 0
-        return out
+        return out[:seq_len]
 
     def _attend(self, q, k, v, lse, tile_layout: tiling.TileLayout, heads, out) -> None:
         q_tiles = kernels.gather_tiles(q, tile_layout, heads)

@@ -21,6 +21,60 @@ from miowtion_amd import _native
 TILE = 128
 
 
+def _ordinary(args) -> bool:
+    """Whether a call with these arguments may run its launch code directly:
+    nothing of what the dispatcher adds for the op is in play. That is: plain
+    GPU tensors, none of which autograd would have to follow; no dispatch or
+    function mode (fake tensors, a device context, a profiling mode); no
+    functorch transform, forward-mode level or tracing; not under compile."""
+    if (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()):
+        return False
+    grad = torch.is_grad_enabled()
+    for a in args:
+        if isinstance(a, torch.Tensor) and (type(a) is not torch.Tensor or not a.is_cuda
+                                            or (grad and a.requires_grad)):
+            return False
+    return True
+
+
+class _Op:
+    """A `veda::` custom op whose ordinary calls skip the dispatcher.
+
+    A custom op's way through the dispatcher costs about 24 us of host time, a
+    direct call 5: a layer makes nine, which at a four-frame preview's sizes
+    is more than its kernels take (200 us of host work for 84 us of kernels).
+    Every other call (gradients, modes, transforms, tracing, tensors that are
+    not on the GPU) goes through the registered op, torch.ops.veda.*, as
+    before. Arguments written in place have their version raised either way.
+    """
+
+    def __init__(self, fn, name: str, mutates_args):
+        self._fn = fn
+        self._op = torch.library.custom_op(name, mutates_args=mutates_args)(fn)
+        code = fn.__code__
+        names = code.co_varnames[:code.co_argcount]
+        self._mutated = tuple(names.index(a) for a in mutates_args)
+        self.__doc__ = fn.__doc__
+
+    def __call__(self, *args, **kwargs):
+        if kwargs or not _ordinary(args):
+            return self._op(*args, **kwargs)
+        out = self._fn(*args)
+        for i in self._mutated:
+            torch.autograd.graph.increment_version(args[i])
+        return out
+
+    def __getattr__(self, name):
+        return getattr(self._op, name)
+
+
+def _custom_op(name: str, mutates_args=()):
+    return lambda fn: _Op(fn, name, mutates_args)
+
+
 def _require_gpu(*tensors: torch.Tensor) -> None:
     for t in tensors:
         if t is not None and not t.is_cuda:
@@ -48,7 +102,7 @@ def _check_rows(name: str, t: torch.Tensor) -> None:
 # gather / pool / scatter (miowtion/kernels/tile_gather_triton.py:156-224)
 
 
-@torch.library.custom_op('veda::gather', mutates_args=())
+@_custom_op('veda::gather', mutates_args=())
 def gather(x: torch.Tensor, gather_index: torch.Tensor, slot_valid: torch.Tensor,
            valid_count: torch.Tensor, heads: torch.Tensor, write_rows: bool, pool: bool,
            second: bool) -> list[torch.Tensor]:
@@ -99,7 +153,7 @@ def _(x, gather_index, slot_valid, valid_count, heads, write_rows, pool, second)
     return res
 
 
-@torch.library.custom_op('veda::scatter_', mutates_args=('out',))
+@_custom_op('veda::scatter_', mutates_args=('out',))
 def scatter_(out: torch.Tensor, tiled: torch.Tensor, scatter_index: torch.Tensor,
              slot_valid: torch.Tensor, heads: torch.Tensor) -> None:
     _require_gpu(out, tiled, scatter_index, slot_valid, heads)
@@ -117,7 +171,7 @@ def scatter_(out: torch.Tensor, tiled: torch.Tensor, scatter_index: torch.Tensor
                  out.shape[0], out.shape[1], out.stride(0), out.stride(1), _stream(out))
 
 
-@torch.library.custom_op('veda::gather_lse', mutates_args=())
+@_custom_op('veda::gather_lse', mutates_args=())
 def gather_lse(lse: torch.Tensor, gather_index: torch.Tensor, slot_valid: torch.Tensor,
                heads: torch.Tensor) -> torch.Tensor:
     _require_gpu(lse, gather_index, slot_valid, heads)
@@ -141,7 +195,7 @@ def _(lse, gather_index, slot_valid, heads):
 # selection, block mask, lists (miowtion/veda/mask.py, miowtion/kernels/fa4.py)
 
 
-@torch.library.custom_op('veda::select_topk', mutates_args=('index', 'keep'))
+@_custom_op('veda::select_topk', mutates_args=('index', 'keep'))
 def select_topk(scores: torch.Tensor, block_start: int, n_cols: int, kv_ok: torch.Tensor,
                 rows: torch.Tensor | None, k_lo: int, k_hi: int, extra: torch.Tensor,
                 index: torch.Tensor, keep: torch.Tensor, col0: int) -> None:
@@ -160,7 +214,7 @@ def select_topk(scores: torch.Tensor, block_start: int, n_cols: int, kv_ok: torc
                  keep.data_ptr(), index.stride(0), index.stride(1), col0, _stream(scores))
 
 
-@torch.library.custom_op('veda::dense_block_mask', mutates_args=())
+@_custom_op('veda::dense_block_mask', mutates_args=())
 def dense_block_mask(index: torch.Tensor, keep: torch.Tensor, kv_ok: torch.Tensor,
                      n_video: int, global_rows: bool) -> torch.Tensor:
     _require_gpu(index, keep, kv_ok)
@@ -184,7 +238,7 @@ def _(index, keep, kv_ok, n_video, global_rows):
     return index.new_empty(heads, n if global_rows else n_sel, n, dtype=torch.bool)
 
 
-@torch.library.custom_op('veda::index_lists', mutates_args=())
+@_custom_op('veda::index_lists', mutates_args=())
 def index_lists(block_mask: torch.Tensor, kv_ok: torch.Tensor,
                 full_tile: torch.Tensor) -> list[torch.Tensor]:
     """-> [part_cnt, part_idx, full_cnt, full_idx], cnt [1, H', R] and idx
@@ -221,7 +275,7 @@ def _empty_lists(heads: int, rows: int, cols: int, device) -> list[torch.Tensor]
     return [torch.empty(s, dtype=torch.int32, device=device) for s in (cnt, idx, cnt, idx)]
 
 
-@torch.library.custom_op('veda::index_lists_t', mutates_args=())
+@_custom_op('veda::index_lists_t', mutates_args=())
 def index_lists_t(block_mask: torch.Tensor, kv_ok: torch.Tensor,
                   full_tile: torch.Tensor) -> list[torch.Tensor]:
     """The Q-direction lists of a block mask [H', R, n] (fa4.py:282-296):
@@ -251,7 +305,7 @@ def _(block_mask, kv_ok, full_tile):
 SELECTION_LISTS_MAX_TILES = 4096
 
 
-@torch.library.custom_op('veda::selection_lists', mutates_args=())
+@_custom_op('veda::selection_lists', mutates_args=())
 def selection_lists(index: torch.Tensor, keep: torch.Tensor, kv_ok: torch.Tensor,
                     full_tile: torch.Tensor, n_video: int) -> list[torch.Tensor]:
     """index_lists of dense_block_mask(index, keep, kv_ok, n_video,
@@ -282,7 +336,7 @@ def _(index, keep, kv_ok, full_tile, n_video):
 # attention (miowtion/kernels/fa4.py:299-377, miowtion/h3/attention.py:28-102)
 
 
-@torch.library.custom_op('veda::block_sparse_fwd', mutates_args=())
+@_custom_op('veda::block_sparse_fwd', mutates_args=())
 def block_sparse_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                      part_cnt: torch.Tensor, part_idx: torch.Tensor, full_cnt: torch.Tensor,
                      full_idx: torch.Tensor, valid_count: torch.Tensor,
@@ -328,7 +382,7 @@ def _(q, k, v, part_cnt, part_idx, full_cnt, full_idx, valid_count, return_lse, 
     return [out]
 
 
-@torch.library.custom_op('veda::block_sparse_fwd_seq_', mutates_args=('out',))
+@_custom_op('veda::block_sparse_fwd_seq_', mutates_args=('out',))
 def block_sparse_fwd_seq_(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                           gather_index: torch.Tensor, scatter_index: torch.Tensor,
                           slot_valid: torch.Tensor, heads: torch.Tensor, part_cnt: torch.Tensor,
@@ -371,7 +425,7 @@ def block_sparse_fwd_seq_(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v
                  out.stride(1), front_tiles, _stream(q))
 
 
-@torch.library.custom_op('veda::block_sparse_fwd_seq_kv_', mutates_args=('out',))
+@_custom_op('veda::block_sparse_fwd_seq_kv_', mutates_args=('out',))
 def block_sparse_fwd_seq_kv_(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor,
                              v: torch.Tensor, gather_index: torch.Tensor,
                              scatter_index: torch.Tensor, slot_valid: torch.Tensor,
@@ -425,7 +479,7 @@ def _check_lists(name: str, cnt: torch.Tensor, idx: torch.Tensor, heads: int, ro
         raise ValueError(f'{name} count must be contiguous int32 [1, {heads}, {rows}]')
 
 
-@torch.library.custom_op('veda::block_sparse_bwd', mutates_args=())
+@_custom_op('veda::block_sparse_bwd', mutates_args=())
 def block_sparse_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor,
                      dout: torch.Tensor, lse: torch.Tensor, dlse: torch.Tensor | None,
                      part_cnt: torch.Tensor, part_idx: torch.Tensor, full_cnt: torch.Tensor,
@@ -483,7 +537,7 @@ def _(q, k, v, out, dout, lse, dlse, part_cnt, part_idx, full_cnt, full_idx, par
     return [torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)]
 
 
-@torch.library.custom_op('veda::dense_fwd', mutates_args=())
+@_custom_op('veda::dense_fwd', mutates_args=())
 def dense_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, used: int,
               return_lse: bool) -> list[torch.Tensor]:
     """Dense attention of rows [0, used) of packed [S, H, D]; -> [out] or
@@ -517,7 +571,7 @@ def _(q, k, v, used, return_lse):
 # teacher heat (miowtion/kernels/block_heat_triton.py:141-173)
 
 
-@torch.library.custom_op('veda::block_heat', mutates_args=())
+@_custom_op('veda::block_heat', mutates_args=())
 def block_heat(q: torch.Tensor, k: torch.Tensor, lse: torch.Tensor, valid_count: torch.Tensor,
                q_tiles: torch.Tensor, reduce: str) -> torch.Tensor:
     """[H', R, n_tiles] fp32 block heat; the real rows of tile t are its first
@@ -558,7 +612,7 @@ def _(q, k, lse, slot_valid, q_tiles, reduce):
 HEAT_WORKSPACE_BYTES = 4 * 2 ** 30
 
 
-@torch.library.custom_op('veda::dense_heat', mutates_args=())
+@_custom_op('veda::dense_heat', mutates_args=())
 def dense_heat(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor | None,
                valid_count: torch.Tensor, q_tiles: torch.Tensor, reduce: str,
                workspace_bytes: int = HEAT_WORKSPACE_BYTES) -> list[torch.Tensor]:
@@ -630,7 +684,7 @@ def _(q, k, v, valid_count, q_tiles, reduce, workspace_bytes=HEAT_WORKSPACE_BYTE
 # miowtion/kernels/compensation_triton.py:80-258)
 
 
-@torch.library.custom_op('veda::tile_summaries', mutates_args=())
+@_custom_op('veda::tile_summaries', mutates_args=())
 def tile_summaries(k: torch.Tensor, v: torch.Tensor, valid_count: torch.Tensor) -> list[torch.Tensor]:
     """[kc, vc], both [n, H', D] bf16: mean of K and sum of V over each key
     tile's real rows (compensation_triton.py:80-99)."""
@@ -657,7 +711,7 @@ def _(k, v, valid_count):
     return [kc, torch.empty_like(kc)]
 
 
-@torch.library.custom_op('veda::zero_order_compensation', mutates_args=())
+@_custom_op('veda::zero_order_compensation', mutates_args=())
 def zero_order_compensation(o_kept: torch.Tensor, lse_kept: torch.Tensor, q: torch.Tensor,
                             kc: torch.Tensor, vc: torch.Tensor, block_mask: torch.Tensor,
                             valid_count: torch.Tensor) -> torch.Tensor:
@@ -695,7 +749,7 @@ def _(o_kept, lse_kept, q, kc, vc, block_mask, valid_count):
     return torch.empty_like(o_kept)
 
 
-@torch.library.custom_op('veda::compensated_attention', mutates_args=())
+@_custom_op('veda::compensated_attention', mutates_args=())
 def compensated_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                           part_cnt: torch.Tensor, part_idx: torch.Tensor, full_cnt: torch.Tensor,
                           full_idx: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor,
@@ -749,7 +803,7 @@ def _(q, k, v, part_cnt, part_idx, full_cnt, full_idx, kc, vc, block_mask, valid
 W_BF16, W_FP32, W_E4M3 = 0, 1, 2
 
 
-@torch.library.custom_op('veda::predictor_embed', mutates_args=())
+@_custom_op('veda::predictor_embed', mutates_args=())
 def predictor_embed(feats: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor | None,
                     heads: torch.Tensor, residual: bool) -> torch.Tensor:
     _require_gpu(feats, weight, weight_scale, heads)
@@ -785,7 +839,7 @@ def _(feats, weight, weight_scale, heads, residual):
     return feats.new_empty(feats.shape[0], feats.shape[1], weight.shape[2])
 
 
-@torch.library.custom_op('veda::predictor_logits', mutates_args=())
+@_custom_op('veda::predictor_logits', mutates_args=())
 def predictor_logits(a: torch.Tensor, b: torch.Tensor, scale: float, gain: torch.Tensor | None,
                      heads: torch.Tensor | None, log_count: torch.Tensor | None,
                      base: torch.Tensor | None) -> torch.Tensor:
