@@ -65,6 +65,19 @@ int veda_gather_tiles(const void* x, int64_t x_rows, int64_t x_heads,
                       float* feats, float* sq, float* var, void* stream);
 
 /*
+ * The pooling of veda_gather_tiles (feats, or feats, sq and var) of two
+ * tensors of the same shape and strides in one launch, without the rows:
+ * what the predictor reads of q and k (miowtion/veda/attention.py:745-757).
+ */
+int veda_pool_pair(const void* x, const void* x2, int64_t x_rows,
+                   int64_t x_heads, int64_t x_stride_s, int64_t x_stride_h,
+                   const int64_t* gather_index, const int32_t* slot_valid,
+                   const int32_t* valid_count, int64_t n_tiles,
+                   const int64_t* heads, int64_t n_heads, int64_t head_dim,
+                   float* feats, float* sq, float* var, float* feats2,
+                   float* sq2, float* var2, void* stream);
+
+/*
  * Write tile-ordered rows back: out[scatter_index[s], heads[h'], :] =
  * tiled[s, h', :] for every slot with slot_valid[s] != 0 (padding slots are
  * dropped, so the result on rows [0, S) equals the reference's index write
@@ -490,6 +503,18 @@ int veda_predictor_embed(const float* feats, int64_t n_heads, int64_t n_tiles,
                          const float* w_scale, int64_t w_heads,
                          const int64_t* heads, int64_t n_out, int residual,
                          float* out, void* stream);
+
+/*
+ * Two veda_predictor_embed calls of the same sizes, weight format and heads
+ * (the query and key projections) in one launch.
+ */
+int veda_predictor_embed_pair(const float* feats, const float* feats2,
+                              int64_t n_heads, int64_t n_tiles, int64_t k_dim,
+                              const void* w, const void* w2, int w_dtype,
+                              const float* w_scale, const float* w_scale2,
+                              int64_t w_heads, const int64_t* heads,
+                              int64_t n_out, int residual, float* out,
+                              float* out2, void* stream);
 
 /*
  * Predictor block logits, miowtion/veda/predictor.py:325-338:

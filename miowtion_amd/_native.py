@@ -25,6 +25,8 @@ _C = ctypes.c_int
 SIGNATURES: dict[str, list] = {
     'veda_gather_tiles': [_P, _I, _I, _I, _I, _P, _P, _P, _I, _P, _I, _I, _P, _I, _I,
                           _P, _P, _P, _P],
+    'veda_pool_pair': [_P, _P, _I, _I, _I, _I, _P, _P, _P, _I, _P, _I, _I, _P, _P, _P, _P, _P, _P,
+                       _P],
     'veda_scatter_tiles': [_P, _I, _I, _P, _P, _I, _P, _I, _I, _P, _I, _I, _I, _I, _P],
     'veda_gather_lse': [_P, _I, _I, _I, _I, _P, _P, _I, _P, _I, _P, _P],
     'veda_select_topk': [_P, _I, _I, _I, _I, _I, _I, _P, _P, _I, _I, _P, _I, _P, _P,
@@ -62,6 +64,8 @@ SIGNATURES: dict[str, list] = {
                                    _P, _P, _P, _P, _I, _P, _P, _I, _I, _P, _P, _F,
                                    _P, _I, _I, _I, _P],
     'veda_predictor_embed': [_P, _I, _I, _I, _P, _C, _P, _I, _P, _I, _C, _P, _P],
+    'veda_predictor_embed_pair': [_P, _P, _I, _I, _I, _P, _P, _C, _P, _P, _I, _P, _I, _C, _P, _P,
+                                  _P],
     'veda_predictor_logits': [_P, _P, _I, _I, _I, _I, _F, _P, _P, _P, _C, _P, _P],
 }
 

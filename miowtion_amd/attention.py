@@ -212,30 +212,20 @@ class SparseStudent:
         # and scatters its rows itself, so q is only pooled, not permuted;
         # when k and v are laid out as q it gathers their key tiles itself
         # too, so they are only pooled (k) or not touched (v) here.
-        q_tiles = None
-        if compensated:
-            q_res = kernels.gather_and_pool(q, tile_layout, heads, second=bool(want))
-            q_tiles, q_res = q_res[0], q_res[1:]
-        else:
-            q_res = kernels.pool_seq(q, tile_layout, heads, second=bool(want))
         kv_seq = not compensated and _seq_kv_ok(q, k, v)
-        k_tiles = v_tiles = None
-        if want:
-            feats_q, sq_q, _ = q_res
-            if kv_seq:
-                feats_k, _, var_k = kernels.pool_seq(k, tile_layout, heads, second=True)
-            else:
-                k_tiles, feats_k, _, var_k = kernels.gather_and_pool(k, tile_layout, heads,
-                                                                     second=True)
+        q_tiles = k_tiles = v_tiles = None
+        if kv_seq:
+            q_res, k_res = kernels.pool_seq_pair(q, k, tile_layout, heads, second=bool(want))
         else:
-            (feats_q,) = q_res
-            if kv_seq:
-                (feats_k,) = kernels.pool_seq(k, tile_layout, heads)
+            if compensated:
+                q_res = kernels.gather_and_pool(q, tile_layout, heads, second=bool(want))
+                q_tiles, q_res = q_res[0], q_res[1:]
             else:
-                k_tiles, feats_k = kernels.gather_and_pool(k, tile_layout, heads)
-            sq_q = var_k = None
-        if not kv_seq:
+                q_res = kernels.pool_seq(q, tile_layout, heads, second=bool(want))
+            k_tiles, *k_res = kernels.gather_and_pool(k, tile_layout, heads, second=bool(want))
             v_tiles = kernels.gather_tiles(v, tile_layout, heads)
+        feats_q, feats_k = q_res[0], k_res[0]
+        sq_q, var_k = (q_res[1], k_res[2]) if want else (None, None)
         with torch.no_grad():
             extra = {}
             if pred.count_term:

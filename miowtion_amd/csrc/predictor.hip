@@ -172,6 +172,13 @@ struct PGemm {
   const float* log_count;
   int accumulate;
   float* out;
+  // embed: the second product of a pair (same sizes and weight format) in
+  // workgroups z >= n_heads
+  int64_t n_heads;
+  const float* a2;
+  const void* w2;
+  const float* w_scale2;
+  float* out2;
 };
 
 constexpr int kKB = 32;  // k per staged block
@@ -249,7 +256,14 @@ __global__ void __launch_bounds__(256) pgemm_kernel(PGemm p) {
   __shared__ __attribute__((aligned(16))) float Bs[2][kBN][kKB];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int li = lane & 31, g = lane >> 5;
-  const int64_t hp = blockIdx.z;
+  int64_t hp = blockIdx.z;
+  if (EMBED && hp >= p.n_heads) {
+    hp -= p.n_heads;
+    p.a = p.a2;
+    p.w = p.w2;
+    p.w_scale = p.w_scale2;
+    p.out = p.out2;
+  }
   const int64_t mb = (int64_t)blockIdx.y * kBM, nb = (int64_t)blockIdx.x * kBN;
   const int wm = 32 * (wave >> 1), wn = 32 * (wave & 1);
   int64_t head = 0;
@@ -380,34 +394,68 @@ __global__ void __launch_bounds__(256) pgemm_kernel(PGemm p) {
 
 using namespace veda;
 
-extern "C" int veda_predictor_embed(const float* feats, int64_t n_heads, int64_t n_tiles,
-                                    int64_t k_dim, const void* w, int w_dtype,
-                                    const float* w_scale, int64_t w_heads, const int64_t* heads,
-                                    int64_t n_out, int residual, float* out, void* stream) {
+// One product, or a pair of the same sizes (feats2 / w2 / ... not NULL): a
+// pair is one launch of twice the workgroups where the matrix form takes it.
+static int embed_launch(const float* feats, const float* feats2, int64_t n_heads, int64_t n_tiles,
+                        int64_t k_dim, const void* w, const void* w2, int w_dtype,
+                        const float* w_scale, const float* w_scale2, int64_t w_heads,
+                        const int64_t* heads, int64_t n_out, int residual, float* out, float* out2,
+                        hipStream_t s) {
   VEDA_REQUIRE(w_dtype >= 0 && w_dtype <= 2, "predictor_embed: unknown weight dtype %d", w_dtype);
-  VEDA_REQUIRE(w_dtype != 2 || w_scale != nullptr, "predictor_embed: e4m3 needs a scale");
+  VEDA_REQUIRE(w_dtype != 2 || (w_scale != nullptr && (w2 == nullptr || w_scale2 != nullptr)),
+               "predictor_embed: e4m3 needs a scale");
   VEDA_REQUIRE(!residual || k_dim >= n_out, "predictor_embed: residual needs k_dim >= n_out");
   VEDA_REQUIRE(n_heads >= 0 && n_tiles >= 0 && k_dim >= 1 && n_out >= 1,
                "predictor_embed: bad sizes");
   if (n_heads == 0 || n_tiles == 0) return VEDA_OK;
+  const bool pair = feats2 != nullptr;
   dim3 grid((unsigned)((n_out + kBN - 1) / kBN), (unsigned)((n_tiles + kBM - 1) / kBM),
             (unsigned)n_heads);
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (k_dim % 4 == 0 && (reinterpret_cast<uintptr_t>(feats) & 15) == 0) {
+  auto at = [](const void* x) { return reinterpret_cast<uintptr_t>(x); };
+  if (k_dim % 4 == 0 && ((at(feats) | at(feats2)) & 15) == 0) {
     PGemm p{};
     p.a = feats; p.w = w; p.w_dtype = w_dtype; p.w_scale = w_scale; p.w_heads = w_heads;
     p.heads = heads; p.m = n_tiles; p.n = n_out; p.k = k_dim; p.residual = residual;
     p.out = out;
+    p.n_heads = n_heads;
+    p.a2 = feats2; p.w2 = w2; p.w_scale2 = w_scale2; p.out2 = out2;
+    if (pair) grid.z *= 2;
     // whole groups of eight columns, each as one aligned load
-    if (n_out % 8 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0)
+    if (n_out % 8 == 0 && ((at(w) | at(w2)) & 15) == 0)
       pgemm_kernel<true, true><<<grid, 256, 0, s>>>(p);
     else
       pgemm_kernel<true, false><<<grid, 256, 0, s>>>(p);
   } else {
     embed_kernel<<<grid, 256, 0, s>>>(feats, n_tiles, k_dim, w, w_dtype, w_scale, w_heads, heads,
                                       n_out, residual, out);
+    if (pair)
+      embed_kernel<<<grid, 256, 0, s>>>(feats2, n_tiles, k_dim, w2, w_dtype, w_scale2, w_heads,
+                                        heads, n_out, residual, out2);
   }
   return check_launch("veda_predictor_embed");
+}
+
+extern "C" int veda_predictor_embed(const float* feats, int64_t n_heads, int64_t n_tiles,
+                                    int64_t k_dim, const void* w, int w_dtype,
+                                    const float* w_scale, int64_t w_heads, const int64_t* heads,
+                                    int64_t n_out, int residual, float* out, void* stream) {
+  return embed_launch(feats, nullptr, n_heads, n_tiles, k_dim, w, nullptr, w_dtype, w_scale,
+                      nullptr, w_heads, heads, n_out, residual, out, nullptr,
+                      reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int veda_predictor_embed_pair(const float* feats, const float* feats2, int64_t n_heads,
+                                         int64_t n_tiles, int64_t k_dim, const void* w,
+                                         const void* w2, int w_dtype, const float* w_scale,
+                                         const float* w_scale2, int64_t w_heads,
+                                         const int64_t* heads, int64_t n_out, int residual,
+                                         float* out, float* out2, void* stream) {
+  VEDA_REQUIRE(feats2 != nullptr && w2 != nullptr && out2 != nullptr,
+               "predictor_embed_pair: the second product's operands are required");
+  VEDA_REQUIRE(n_heads < 32768, "predictor_embed_pair: too many heads for one launch");
+  return embed_launch(feats, feats2, n_heads, n_tiles, k_dim, w, w2, w_dtype, w_scale, w_scale2,
+                      w_heads, heads, n_out, residual, out, out2,
+                      reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int veda_predictor_logits(const float* a, const float* b, int64_t n_heads, int64_t n_q,

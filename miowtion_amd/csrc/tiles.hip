@@ -85,6 +85,16 @@ __device__ __forceinline__ float elem(const Row8& r, int e) {
   return bf16_to_f32((e & 1) ? (w >> 16) : (w & 0xffffu));
 }
 
+// The second tensor of a pooled pair (same shape, strides and layout as the
+// first) and its outputs: grid.y = 2, so two small launches and the gap
+// between them are one.
+struct Second2 {
+  const uint16_t* x;
+  float* feats;
+  float* sq;
+  float* var;
+};
+
 // Gather. Workgroup = (tile, group of heads) with WAVES waves, each on
 // 128 / WAVES consecutive slots; lane = (head, 16-byte chunk). More waves
 // per tile put more rows in flight per workgroup: the plain copy runs with
@@ -98,7 +108,13 @@ __global__ void __launch_bounds__(64 * WAVES) gather_kernel(
     const int32_t* __restrict__ valid_count, int64_t n_tiles,
     const int64_t* __restrict__ heads, int64_t n_heads,
     uint16_t* __restrict__ out, int64_t os, int64_t oh,
-    float* __restrict__ feats, float* __restrict__ sq, float* __restrict__ var) {
+    float* __restrict__ feats, float* __restrict__ sq, float* __restrict__ var, Second2 two) {
+  if (blockIdx.y) {  // the pair's second tensor (pooling only)
+    x = two.x;
+    feats = two.feats;
+    sq = two.sq;
+    var = two.var;
+  }
   constexpr int kChunks = D / 8;          // 16-byte chunks per head row
   constexpr int kHeadsPerGroup = 64 / kChunks;
   const int n_groups = (int)((n_heads + kHeadsPerGroup - 1) / kHeadsPerGroup);
@@ -289,7 +305,11 @@ __global__ void __launch_bounds__(SPLIT == 1 ? 64 * kWaves : 64 * SPLIT,
     const int32_t* __restrict__ slot_valid,
     const int32_t* __restrict__ valid_count, int64_t n_tiles,
     const int64_t* __restrict__ heads, int64_t n_heads,
-    uint16_t* __restrict__ out, int64_t os, int64_t oh, float* __restrict__ feats) {
+    uint16_t* __restrict__ out, int64_t os, int64_t oh, float* __restrict__ feats, Second2 two) {
+  if (blockIdx.y) {  // the pair's second tensor (pooling only)
+    x = two.x;
+    feats = two.feats;
+  }
   constexpr int kChunks = D / 8;
   constexpr int kHeadsPerGroup = 64 / kChunks;
   constexpr int kGroup = kTile / kPoolSplit;  // slots per partial sum
@@ -537,13 +557,13 @@ extern "C" const char* veda_last_error(void) { return g_error.c_str(); }
 
 extern "C" int veda_abi_version(void) { return 5; }
 
-extern "C" int veda_gather_tiles(const void* x, int64_t x_rows, int64_t x_heads,
+static int gather_launch(const void* x, int64_t x_rows, int64_t x_heads,
                                  int64_t x_stride_s, int64_t x_stride_h,
                                  const int64_t* gather_index, const int32_t* slot_valid,
                                  const int32_t* valid_count, int64_t n_tiles,
                                  const int64_t* heads, int64_t n_heads, int64_t head_dim,
                                  void* out, int64_t out_stride_s, int64_t out_stride_h,
-                                 float* feats, float* sq, float* var, void* stream) {
+                                 float* feats, float* sq, float* var, const Second2& two, void* stream) {
   VEDA_REQUIRE(head_dim == 64 || head_dim == 128, "gather: head_dim must be 64 or 128, got %lld",
                (long long)head_dim);
   VEDA_REQUIRE(n_tiles >= 0 && n_heads >= 0, "gather: negative size");
@@ -558,21 +578,22 @@ extern "C" int veda_gather_tiles(const void* x, int64_t x_rows, int64_t x_heads,
   const int64_t n_wg = n_tiles * ((n_heads + hpg - 1) / hpg);
   VEDA_REQUIRE(n_wg <= INT32_MAX, "gather: %lld tiles x head groups exceed one launch",
                (long long)n_wg);
-  dim3 grid((unsigned)n_wg);
+  const unsigned gy = two.x != nullptr ? 2 : 1;
+  dim3 grid((unsigned)n_wg, gy);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   auto xx = static_cast<const uint16_t*>(x);
   auto oo = static_cast<uint16_t*>(out);
 #define VEDA_GATHER(D, P, S2, W)                                                              \
   gather_kernel<D, P, S2, W><<<grid, 64 * W, 0, s>>>(                                          \
       xx, x_rows, x_heads, x_stride_s, x_stride_h, gather_index, slot_valid, valid_count,      \
-      n_tiles, heads, n_heads, oo, out_stride_s, out_stride_h, feats, sq, var)
+      n_tiles, heads, n_heads, oo, out_stride_s, out_stride_h, feats, sq, var, two)
 #define VEDA_POOL_FORM(D, SPLIT, GRID, THREADS)                                               \
-  pool_gather_kernel<D, SPLIT><<<(unsigned)(GRID), THREADS, 0, s>>>(                           \
+  pool_gather_kernel<D, SPLIT><<<dim3((unsigned)(GRID), gy), THREADS, 0, s>>>(                 \
       xx, x_rows, x_heads, x_stride_s, x_stride_h, gather_index, slot_valid, valid_count,      \
-      n_tiles, heads, n_heads, oo, out_stride_s, out_stride_h, feats)
+      n_tiles, heads, n_heads, oo, out_stride_s, out_stride_h, feats, two)
 #define VEDA_POOL_GATHER(D)                                                                   \
   do {                                                                                        \
-    if (out != nullptr || n_wg < kPoolSplitItems)                                             \
+    if (out != nullptr || n_wg * gy < kPoolSplitItems)                                             \
       VEDA_POOL_FORM(D, kPoolSplit, n_wg, 64 * kPoolSplit);                                   \
     else                                                                                      \
       VEDA_POOL_FORM(D, 1, (n_wg + kWaves - 1) / kWaves, 64 * kWaves);                        \
@@ -590,6 +611,33 @@ extern "C" int veda_gather_tiles(const void* x, int64_t x_rows, int64_t x_heads,
 #undef VEDA_POOL_GATHER
 #undef VEDA_POOL_FORM
   return check_launch("veda_gather_tiles");
+}
+
+extern "C" int veda_gather_tiles(const void* x, int64_t x_rows, int64_t x_heads,
+                                 int64_t x_stride_s, int64_t x_stride_h,
+                                 const int64_t* gather_index, const int32_t* slot_valid,
+                                 const int32_t* valid_count, int64_t n_tiles,
+                                 const int64_t* heads, int64_t n_heads, int64_t head_dim,
+                                 void* out, int64_t out_stride_s, int64_t out_stride_h,
+                                 float* feats, float* sq, float* var, void* stream) {
+  return gather_launch(x, x_rows, x_heads, x_stride_s, x_stride_h, gather_index, slot_valid,
+                       valid_count, n_tiles, heads, n_heads, head_dim, out, out_stride_s,
+                       out_stride_h, feats, sq, var, Second2{}, stream);
+}
+
+extern "C" int veda_pool_pair(const void* x, const void* x2, int64_t x_rows, int64_t x_heads,
+                              int64_t x_stride_s, int64_t x_stride_h, const int64_t* gather_index,
+                              const int32_t* slot_valid, const int32_t* valid_count,
+                              int64_t n_tiles, const int64_t* heads, int64_t n_heads,
+                              int64_t head_dim, float* feats, float* sq, float* var,
+                              float* feats2, float* sq2, float* var2, void* stream) {
+  VEDA_REQUIRE(x2 != nullptr && aligned16(x2), "pool_pair: rows must be 16-byte aligned");
+  VEDA_REQUIRE(feats != nullptr && feats2 != nullptr, "pool_pair: both feature outputs are required");
+  VEDA_REQUIRE((sq == nullptr) == (sq2 == nullptr) && (var == nullptr) == (var2 == nullptr),
+               "pool_pair: second moments of both tensors or of neither");
+  return gather_launch(x, x_rows, x_heads, x_stride_s, x_stride_h, gather_index, slot_valid,
+                       valid_count, n_tiles, heads, n_heads, head_dim, nullptr, 0, 0, feats, sq,
+                       var, Second2{static_cast<const uint16_t*>(x2), feats2, sq2, var2}, stream);
 }
 
 extern "C" int veda_scatter_tiles(const void* tiled, int64_t tiled_stride_s,

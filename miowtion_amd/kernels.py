@@ -98,6 +98,16 @@ def pool_seq(x: torch.Tensor, layout: tiling.TileLayout, heads: torch.Tensor | N
     return tuple(res[1:])
 
 
+def pool_seq_pair(x: torch.Tensor, x2: torch.Tensor, layout: tiling.TileLayout,
+                  heads: torch.Tensor | None, second: bool = False) -> tuple[tuple, tuple]:
+    """(pool_seq(x), pool_seq(x2)) of two tensors laid out alike, in one
+    launch."""
+    res = ops.pool_pair(x, x2, layout.gather_index, layout.slot_valid, layout.valid_count,
+                        _heads(x, heads), second)
+    half = len(res) // 2
+    return tuple(res[:half]), tuple(res[half:])
+
+
 def pool_tiles(x: torch.Tensor, layout: tiling.TileLayout, second: str | None = None) -> torch.Tensor:
     """Pooling of already tile-ordered rows [N, H', D] (predictor.py:82-130):
     [H', n, 3D] fp32 [mean | max | min], or [H', n, D] E[x^2] ('raw') /

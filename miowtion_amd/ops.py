@@ -21,21 +21,30 @@ from miowtion_amd import _native
 TILE = 128
 
 
+# bound once: these run on every call
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_modes = torch._C._len_torch_function_stack
+_transforms = torch._C._functorch.peek_interpreter_stack
+_tracing = torch._C._get_tracing_state
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 def _ordinary(args) -> bool:
     """Whether a call with these arguments may run its launch code directly:
     nothing of what the dispatcher adds for the op is in play. That is: plain
     GPU tensors, none of which autograd would have to follow; no dispatch or
     function mode (fake tensors, a device context, a profiling mode); no
     functorch transform, forward-mode level or tracing; not under compile."""
-    if (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-            or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch.autograd.forward_ad._current_level >= 0
-            or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()):
+    if (torch.compiler.is_compiling() or _dispatch_modes() or _function_modes()
+            or _transforms() is not None or torch.autograd.forward_ad._current_level >= 0
+            or _tracing() is not None):
         return False
     grad = torch.is_grad_enabled()
     for a in args:
-        if isinstance(a, torch.Tensor) and (type(a) is not torch.Tensor or not a.is_cuda
-                                            or (grad and a.requires_grad)):
+        if type(a) is torch.Tensor:
+            if not a.is_cuda or (grad and a.requires_grad):
+                return False
+        elif isinstance(a, torch.Tensor):  # a subclass
             return False
     return True
 
@@ -84,7 +93,7 @@ def _require_gpu(*tensors: torch.Tensor) -> None:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.device.index)  # the current stream of the tensor's device
 
 
 def _p(t: torch.Tensor | None):
@@ -151,6 +160,40 @@ def _(x, gather_index, slot_valid, valid_count, heads, write_rows, pool, second)
         if second:
             res += [x.new_empty(hp, n_tiles, d, dtype=torch.float32) for _ in range(2)]
     return res
+
+
+@_custom_op('veda::pool_pair', mutates_args=())
+def pool_pair(x: torch.Tensor, x2: torch.Tensor, gather_index: torch.Tensor,
+              slot_valid: torch.Tensor, valid_count: torch.Tensor, heads: torch.Tensor,
+              second: bool) -> list[torch.Tensor]:
+    """The pooling of two tensors laid out alike in one launch: [feats,
+    feats2], or [feats, sq, var, feats2, sq2, var2] with `second`."""
+    _require_gpu(x, x2, gather_index, slot_valid, valid_count, heads)
+    _check_rows('x', x)
+    _check_rows('x2', x2)
+    if x2.shape != x.shape or x2.stride() != x.stride():
+        raise ValueError('x2 must be laid out as x')
+    n_slots = gather_index.numel()
+    if n_slots % TILE:
+        raise ValueError('gather_index must hold n_tiles * 128 slots')
+    n_tiles, d, hp = n_slots // TILE, x.shape[-1], heads.numel()
+    if d not in (64, 128):
+        raise ValueError('tile kernels need contiguous head_dim 64 or 128')
+    sizes = (3 * d, d, d) if second else (3 * d,)
+    res = [torch.empty(hp, n_tiles, n, dtype=torch.float32, device=x.device) for n in sizes * 2]
+    p = [t.data_ptr() for t in res]
+    a, b = (p[:3], p[3:]) if second else ([p[0], None, None], [p[1], None, None])
+    _native.call('veda_pool_pair', x.data_ptr(), x2.data_ptr(), x.shape[0], x.shape[1],
+                 x.stride(0), x.stride(1), gather_index.data_ptr(), slot_valid.data_ptr(),
+                 valid_count.data_ptr(), n_tiles, heads.data_ptr(), hp, d, *a, *b, _stream(x))
+    return res
+
+
+@pool_pair.register_fake
+def _(x, x2, gather_index, slot_valid, valid_count, heads, second):
+    hp, n_tiles, d = heads.numel(), gather_index.numel() // TILE, x.shape[-1]
+    return [x.new_empty(hp, n_tiles, n, dtype=torch.float32)
+            for n in ((3 * d, d, d) if second else (3 * d,)) * 2]
 
 
 @_custom_op('veda::scatter_', mutates_args=('out',))
@@ -803,17 +846,14 @@ def _(q, k, v, part_cnt, part_idx, full_cnt, full_idx, kc, vc, block_mask, valid
 W_BF16, W_FP32, W_E4M3 = 0, 1, 2
 
 
-@_custom_op('veda::predictor_embed', mutates_args=())
-def predictor_embed(feats: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor | None,
-                    heads: torch.Tensor, residual: bool) -> torch.Tensor:
-    _require_gpu(feats, weight, weight_scale, heads)
+def _embed_args(feats, weight, weight_scale, residual):
+    """(contiguous feats, contiguous weight, weight format) of a checked embedding."""
     if feats.dtype != torch.float32 or feats.dim() != 3:
         raise ValueError('feats must be fp32 [H\', n, K]')
-    hp, n, kd = feats.shape
+    kd = feats.shape[2]
     if weight.dim() != 3 or weight.shape[1] != kd:
         raise ValueError(f'weight {tuple(weight.shape)} does not take {kd} features')
-    n_out = weight.shape[2]
-    if residual and kd < n_out:
+    if residual and kd < weight.shape[2]:
         raise ValueError('residual needs at least n_out features')
     if weight.dtype == torch.bfloat16:
         wd = W_BF16
@@ -825,8 +865,16 @@ def predictor_embed(feats: torch.Tensor, weight: torch.Tensor, weight_scale: tor
             raise ValueError('e4m3 weights need a per-head fp32 scale')
     else:
         raise ValueError(f'unsupported weight dtype {weight.dtype}')
-    f = feats.contiguous()
-    w = weight.contiguous()
+    return feats.contiguous(), weight.contiguous(), wd
+
+
+@_custom_op('veda::predictor_embed', mutates_args=())
+def predictor_embed(feats: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor | None,
+                    heads: torch.Tensor, residual: bool) -> torch.Tensor:
+    _require_gpu(feats, weight, weight_scale, heads)
+    f, w, wd = _embed_args(feats, weight, weight_scale, residual)
+    hp, n, kd = f.shape
+    n_out = w.shape[2]
     out = torch.empty(hp, n, n_out, dtype=torch.float32, device=feats.device)
     _native.call('veda_predictor_embed', f.data_ptr(), hp, n, kd, w.data_ptr(), wd,
                  _p(weight_scale), weight.shape[0], heads.data_ptr(), n_out, int(residual),
@@ -837,6 +885,33 @@ def predictor_embed(feats: torch.Tensor, weight: torch.Tensor, weight_scale: tor
 @predictor_embed.register_fake
 def _(feats, weight, weight_scale, heads, residual):
     return feats.new_empty(feats.shape[0], feats.shape[1], weight.shape[2])
+
+
+@_custom_op('veda::predictor_embed_pair', mutates_args=())
+def predictor_embed_pair(feats: torch.Tensor, feats2: torch.Tensor, weight: torch.Tensor,
+                         weight2: torch.Tensor, weight_scale: torch.Tensor | None,
+                         weight_scale2: torch.Tensor | None, heads: torch.Tensor,
+                         residual: bool) -> list[torch.Tensor]:
+    """Two predictor_embed of the same shapes and weight format in one launch."""
+    _require_gpu(feats, feats2, weight, weight2, weight_scale, weight_scale2, heads)
+    f, w, wd = _embed_args(feats, weight, weight_scale, residual)
+    f2, w2, wd2 = _embed_args(feats2, weight2, weight_scale2, residual)
+    if f2.shape != f.shape or w2.shape != w.shape or wd2 != wd:
+        raise ValueError('the two embeddings of a pair must have the same shapes and weight dtype')
+    hp, n, kd = f.shape
+    n_out = w.shape[2]
+    out, out2 = (torch.empty(hp, n, n_out, dtype=torch.float32, device=feats.device)
+                 for _ in range(2))
+    _native.call('veda_predictor_embed_pair', f.data_ptr(), f2.data_ptr(), hp, n, kd,
+                 w.data_ptr(), w2.data_ptr(), wd, _p(weight_scale), _p(weight_scale2),
+                 weight.shape[0], heads.data_ptr(), n_out, int(residual), out.data_ptr(),
+                 out2.data_ptr(), _stream(feats))
+    return [out, out2]
+
+
+@predictor_embed_pair.register_fake
+def _(feats, feats2, weight, weight2, weight_scale, weight_scale2, heads, residual):
+    return [feats.new_empty(feats.shape[0], feats.shape[1], weight.shape[2]) for _ in range(2)]
 
 
 @_custom_op('veda::predictor_logits', mutates_args=())

@@ -60,6 +60,16 @@ class ProjWeight:
         return self.values.shape
 
 
+def _embed_two(x, y, px: ProjWeight, py: ProjWeight, heads: torch.Tensor, residual: bool):
+    """The embeddings of x with px and of y with py, as one launch when their
+    shapes and weight formats agree."""
+    if x.shape == y.shape and px.shape == py.shape and px.values.dtype == py.values.dtype:
+        return ops.predictor_embed_pair(x, y, px.values, py.values, px.scale, py.scale, heads,
+                                        residual)
+    return (ops.predictor_embed(x, px.values, px.scale, heads, residual),
+            ops.predictor_embed(y, py.values, py.scale, heads, residual))
+
+
 class LayerPredictor:
     """Projections of one layer: proj_q, proj_k [num_heads, 3D, D]; with
     second_order_rank > 0 also so_q, so_k [num_heads, D, rank]; with
@@ -107,15 +117,13 @@ class LayerPredictor:
             raise ValueError('log_count and count_term must be set together')
         if bool(self.second_order_rank) != (sq_q is not None and var_k is not None):
             raise ValueError('second-order features and second_order_rank must be set together')
-        q_hat = self.embed(feats_q, heads, self.proj_q)
-        k_hat = self.embed(feats_k, heads, self.proj_k)
+        q_hat, k_hat = _embed_two(feats_q, feats_k, self.proj_q, self.proj_k, heads, True)
         logits = ops.predictor_logits(q_hat, k_hat, 1.0 / math.sqrt(self.head_dim),
                                       self.count_gain, heads if log_count is not None else None,
                                       log_count, None)
         if not self.second_order_rank:
             return logits
-        u = ops.predictor_embed(sq_q, self.so_q.values, self.so_q.scale, heads, False)
-        w = ops.predictor_embed(var_k, self.so_k.values, self.so_k.scale, heads, False)
+        u, w = _embed_two(sq_q, var_k, self.so_q, self.so_k, heads, False)
         return ops.predictor_logits(u, w, 1.0, None, None, None, logits)
 
 

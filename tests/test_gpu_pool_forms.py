@@ -45,3 +45,19 @@ def test_head_chunks_keep_the_bits():
     parts = torch.cat([kernels.pool_seq(x, lay, h)[0] for h in heads.split(4)])
     assert torch.equal(whole, parts)
     assert torch.equal(whole, kernels.gather_and_pool(x, lay, heads)[1])
+
+
+@pytest.mark.parametrize('dim', [64, 128])
+@pytest.mark.parametrize('second', [False, True])
+def test_a_pair_pools_as_its_tensors_alone(dim, second):
+    lay = helpers.product_layout(*helpers.small_layout(), device='cuda')
+    x, y = (t.cuda() for t in helpers.qkv(lay.seq_len, 5, dim, seed=9, n=2))
+    heads = torch.tensor([4, 0, 2, 3, 1], device='cuda')
+    for pair in ((x, y), (x[:, 1:], y[:, 1:])):  # whole tensors, and strided views of them
+        h = heads if pair[0].shape[1] == 5 else heads[:3] % 4
+        got = kernels.pool_seq_pair(*pair, lay, h, second)
+        for g, t in zip(got, pair):
+            for a, b in zip(g, kernels.pool_seq(t, lay, h, second)):
+                assert torch.equal(a, b)
+    with pytest.raises(ValueError, match='laid out'):
+        kernels.pool_seq_pair(x, y[:, 1:], lay, heads)

@@ -52,3 +52,15 @@ def test_embedding_matches_float64(fmt, m, k, n, offset):
         size = size + feats[..., :n].double().abs()
     # k + 1 roundings of fp32 sums, each at most 2^-24 of the sum of magnitudes
     assert ((got - want).abs() <= (k + 1) * 2.0 ** -24 * size + 1e-30).all()
+
+
+@pytest.mark.parametrize('fmt', ['fp8', 'bf16', 'fp32'])
+@pytest.mark.parametrize('m,k,n', [(70, 384, 128), (9, 64, 16), (5, 30, 8), (5, 32, 12)])
+def test_a_pair_embeds_as_its_products_alone(fmt, m, k, n):
+    g = torch.Generator().manual_seed(m + k)
+    feats = [torch.randn(3, m, k, generator=g).cuda() for _ in range(2)]
+    (wa, sa, _), (wb, sb, _) = (_weights(fmt, 4, k, n, 0, g) for _ in range(2))
+    heads = torch.tensor([3, 0, 7], device='cuda')
+    got = ops.predictor_embed_pair(*feats, wa, wb, sa, sb, heads, k >= n)
+    assert torch.equal(got[0], ops.predictor_embed(feats[0], wa, sa, heads, k >= n))
+    assert torch.equal(got[1], ops.predictor_embed(feats[1], wb, sb, heads, k >= n))
