@@ -415,6 +415,36 @@ int veda_compensated_attention(const void* q, int64_t q_stride_s, int64_t q_stri
                                int64_t front_tiles, void* stream);
 
 /*
+ * veda_compensated_attention with the permutation of q and out fused in, as
+ * veda_block_sparse_fwd_seq has it (the gather of q, compensation_triton.
+ * attention and the scatter of miowtion/veda/attention.py:760-794).
+ */
+int veda_compensated_attention_seq(
+    const void* q, int64_t q_rows, int64_t seq_heads, int64_t q_stride_s,
+    int64_t q_stride_h, const int64_t* gather_index,
+    const int64_t* scatter_index, const int32_t* slot_valid,
+    const int64_t* heads, int64_t n_heads, const void* k, int64_t k_stride_s,
+    int64_t k_stride_h, const void* v, int64_t v_stride_s, int64_t v_stride_h,
+    int64_t head_dim, int64_t n_q_tiles, int64_t n_k_tiles,
+    const int32_t* full_cnt, const int32_t* full_idx, const int32_t* part_cnt,
+    const int32_t* part_idx, int64_t list_ld, const void* kc, const void* vc,
+    int64_t c_stride_s, int64_t c_stride_h, const uint8_t* keep,
+    const int32_t* valid_count, float scale, void* out, int64_t out_rows,
+    int64_t o_stride_s, int64_t o_stride_h, int64_t front_tiles, void* stream);
+
+/*
+ * veda_tile_summaries from the pooled features [n_heads, n_tiles, 3 D] of
+ * tile-ordered K and V (mean first): kc = mean K, vc = mean V * valid_count,
+ * bf16 (miowtion/kernels/compensation_triton.py:80-99).
+ */
+int veda_summaries_from_means(const float* feats_k, const float* feats_v,
+                              const int32_t* valid_count, int64_t n_tiles,
+                              int64_t n_heads, int64_t head_dim, void* kc,
+                              void* vc, int64_t c_stride_s, int64_t c_stride_h,
+                              void* stream);
+
+
+/*
  * Block-sparse attention backward: the gradients of veda_block_sparse_fwd
  * (FA4's backward with the Q-direction lists, reached through
  * miowtion/kernels/fa4.py:340-373 -> fa4_sm8x/interface.py:3722-3790

@@ -63,6 +63,10 @@ SIGNATURES: dict[str, list] = {
     'veda_compensated_attention': [_P, _I, _I, _P, _I, _I, _P, _I, _I, _I, _I, _I, _I,
                                    _P, _P, _P, _P, _I, _P, _P, _I, _I, _P, _P, _F,
                                    _P, _I, _I, _I, _P],
+    'veda_compensated_attention_seq': [_P, _I, _I, _I, _I, _P, _P, _P, _P, _I, _P, _I, _I, _P, _I, _I,
+                                       _I, _I, _I, _P, _P, _P, _P, _I, _P, _P, _I, _I, _P, _P, _F,
+                                       _P, _I, _I, _I, _I, _P],
+    'veda_summaries_from_means': [_P, _P, _P, _I, _I, _I, _P, _P, _I, _I, _P],
     'veda_predictor_embed': [_P, _I, _I, _I, _P, _C, _P, _I, _P, _I, _C, _P, _P],
     'veda_predictor_embed_pair': [_P, _P, _I, _I, _I, _P, _P, _C, _P, _P, _I, _P, _I, _C, _P, _P,
                                   _P],

@@ -208,22 +208,22 @@ class SparseStudent:
         want = pred.second_order_rank
         cfg = self.clip.config
         compensated = cfg.zero_order_compensation or cfg.triton_compensation
-        # Without compensation the attention kernel reads q in sequence order
-        # and scatters its rows itself, so q is only pooled, not permuted;
-        # when k and v are laid out as q it gathers their key tiles itself
-        # too, so they are only pooled (k) or not touched (v) here.
+        # The attention kernel reads q in sequence order and scatters its rows
+        # itself, so q is only pooled, not permuted; without compensation and
+        # with k and v laid out as q it gathers their key tiles itself too, so
+        # they are only pooled (k) or not touched (v) here. Compensation takes
+        # the tile summaries from the pooled k and v.
         kv_seq = not compensated and _seq_kv_ok(q, k, v)
-        q_tiles = k_tiles = v_tiles = None
+        k_tiles = v_tiles = feats_v = None
         if kv_seq:
             q_res, k_res = kernels.pool_seq_pair(q, k, tile_layout, heads, second=bool(want))
         else:
-            if compensated:
-                q_res = kernels.gather_and_pool(q, tile_layout, heads, second=bool(want))
-                q_tiles, q_res = q_res[0], q_res[1:]
-            else:
-                q_res = kernels.pool_seq(q, tile_layout, heads, second=bool(want))
+            q_res = kernels.pool_seq(q, tile_layout, heads, second=bool(want))
             k_tiles, *k_res = kernels.gather_and_pool(k, tile_layout, heads, second=bool(want))
-            v_tiles = kernels.gather_tiles(v, tile_layout, heads)
+            if compensated:
+                v_tiles, feats_v = kernels.gather_and_pool(v, tile_layout, heads)
+            else:
+                v_tiles = kernels.gather_tiles(v, tile_layout, heads)
         feats_q, feats_k = q_res[0], k_res[0]
         sq_q, var_k = (q_res[1], k_res[2]) if want else (None, None)
         with torch.no_grad():
@@ -238,10 +238,9 @@ class SparseStudent:
             if compensated:
                 block_mask = veda_mask.dense_block_mask(selection, tile_layout)
                 lists = kernels.index_lists(block_mask, tile_layout)
-                # the lists already hold only kv_ok tiles (index_lists applies it)
-                o_tiles = kernels.compensated_attention(q_tiles, k_tiles, v_tiles, block_mask,
-                                                        tile_layout, lists)
-                kernels.scatter_tiles_(out, o_tiles, tile_layout, heads)
+                kernels.compensated_attention_seq_(
+                    out, q, k_tiles, v_tiles, feats_k, feats_v,
+                    block_mask & tile_layout.kv_ok[None, None, :], lists, tile_layout, heads)
             else:
                 lists = kernels.selection_lists(selection, tile_layout)
                 if kv_seq:

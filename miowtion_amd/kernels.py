@@ -367,3 +367,19 @@ def compensated_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     kc, vc = tile_summaries(k, v, layout)
     return ops.compensated_attention(q, k, v, *lists, kc, vc, kept, layout.valid_count,
                                      _front_tiles(layout, q.shape[0] // 128))
+
+
+def compensated_attention_seq_(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor,
+                               v: torch.Tensor, feats_k: torch.Tensor, feats_v: torch.Tensor,
+                               block_mask: torch.Tensor, lists, layout: tiling.TileLayout,
+                               heads: torch.Tensor | None) -> None:
+    """scatter_tiles_(out, compensated_attention(gather_tiles(q), k, v, ...))
+    with q [S, H, D] in sequence order and out the [S + 1, H, D] scatter
+    buffer, in one kernel, and the tile summaries from the pooled features of
+    k and v (gather_and_pool) instead of a pass over k and v. block_mask: the
+    kept blocks with kv_ok applied; lists: its index_lists."""
+    kc, vc = ops.summaries_from_means(feats_k, feats_v, layout.valid_count)
+    ops.compensated_attention_seq_(out, q, k, v, layout.gather_index, layout.scatter_index,
+                                   layout.slot_valid, _heads(q, heads), *lists, kc, vc, block_mask,
+                                   layout.valid_count,
+                                   _front_tiles(layout, layout.gather_index.numel() // 128))

@@ -840,6 +840,83 @@ def _(q, k, v, part_cnt, part_idx, full_cnt, full_idx, kc, vc, block_mask, valid
     return torch.empty_like(q)
 
 
+@_custom_op('veda::summaries_from_means', mutates_args=())
+def summaries_from_means(feats_k: torch.Tensor, feats_v: torch.Tensor,
+                         valid_count: torch.Tensor) -> list[torch.Tensor]:
+    """tile_summaries' [kc, vc] from the pooled features [H', n, 3D] of K and V."""
+    _require_gpu(feats_k, feats_v, valid_count)
+    for name, t in (('feats_k', feats_k), ('feats_v', feats_v)):
+        if t.dtype != torch.float32 or t.dim() != 3 or not t.is_contiguous():
+            raise ValueError(f"{name} must be contiguous fp32 [H', n, 3D]")
+    if feats_k.shape != feats_v.shape or feats_k.shape[2] not in (192, 384):
+        raise ValueError('feats_k and feats_v must have equal shapes, of head_dim 64 or 128')
+    heads, n, d = feats_k.shape[0], feats_k.shape[1], feats_k.shape[2] // 3
+    if valid_count.numel() != n or valid_count.dtype != torch.int32:
+        raise ValueError(f'valid_count must be int32 [{n}]')
+    kc = torch.empty(n, heads, d, dtype=torch.bfloat16, device=feats_k.device)
+    vc = torch.empty_like(kc)
+    _native.call('veda_summaries_from_means', feats_k.data_ptr(), feats_v.data_ptr(),
+                 valid_count.contiguous().data_ptr(), n, heads, d, kc.data_ptr(), vc.data_ptr(),
+                 kc.stride(0), kc.stride(1), _stream(feats_k))
+    return [kc, vc]
+
+
+@summaries_from_means.register_fake
+def _(feats_k, feats_v, valid_count):
+    return [feats_k.new_empty(feats_k.shape[1], feats_k.shape[0], feats_k.shape[2] // 3,
+                              dtype=torch.bfloat16) for _ in range(2)]
+
+
+@_custom_op('veda::compensated_attention_seq_', mutates_args=('out',))
+def compensated_attention_seq_(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor,
+                               v: torch.Tensor, gather_index: torch.Tensor,
+                               scatter_index: torch.Tensor, slot_valid: torch.Tensor,
+                               heads: torch.Tensor, part_cnt: torch.Tensor,
+                               part_idx: torch.Tensor, full_cnt: torch.Tensor,
+                               full_idx: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor,
+                               block_mask: torch.Tensor, valid_count: torch.Tensor,
+                               front_tiles: int = 0) -> None:
+    """compensated_attention with q [S, H, D] in sequence order, read through
+    gather_index, and its rows written into out [S + 1, H, D] through
+    scatter_index; k / v tile-ordered. heads maps the H' heads of k, v and the
+    lists to heads of q and out."""
+    _require_gpu(out, q, k, v, gather_index, scatter_index, slot_valid, heads, part_cnt, part_idx,
+                 full_cnt, full_idx, kc, vc, block_mask, valid_count)
+    for name, t in (('out', out), ('q', q), ('k', k), ('v', v), ('kc', kc), ('vc', vc)):
+        _check_rows(name, t)
+    if q.shape[-1] != 128 or out.shape[1:] != q.shape[1:] or out.dtype != q.dtype:
+        raise ValueError(f'q {tuple(q.shape)} and out {tuple(out.shape)} must be [*, H, 128] alike')
+    n_slots, hp = gather_index.numel(), heads.numel()
+    if (n_slots % TILE or scatter_index.numel() != n_slots or slot_valid.numel() != n_slots
+            or gather_index.dtype != torch.int64 or scatter_index.dtype != torch.int64
+            or slot_valid.dtype != torch.int32 or heads.dtype != torch.int64):
+        raise ValueError('gather_index / scatter_index int64 and slot_valid int32 of n_tiles * 128 '
+                         'slots, heads int64')
+    if k.shape != v.shape or k.shape[0] % TILE or k.shape[1] != hp or k.shape[2] != 128:
+        raise ValueError(f'k {tuple(k.shape)} / v {tuple(v.shape)} must be [n * 128, {hp}, 128]')
+    r_tiles, n = n_slots // TILE, k.shape[0] // TILE
+    _check_lists('part', part_cnt, part_idx, hp, r_tiles, n)
+    _check_lists('full', full_cnt, full_idx, hp, r_tiles, n)
+    if part_idx.shape[3] != full_idx.shape[3]:
+        raise ValueError('the part and full lists must have equal rows')
+    if vc.shape != kc.shape or tuple(kc.shape) != (n, hp, 128) or vc.stride() != kc.stride():
+        raise ValueError(f'kc / vc must be [{n}, {hp}, 128] alike')
+    if block_mask.dtype != torch.bool or tuple(block_mask.shape) != (hp, r_tiles, n):
+        raise ValueError(f'block_mask must be bool [{hp}, {r_tiles}, {n}]')
+    if valid_count.numel() != n or valid_count.dtype != torch.int32:
+        raise ValueError(f'valid_count must be int32 [{n}]')
+    keep = block_mask.contiguous()  # held until the launch
+    _native.call('veda_compensated_attention_seq', q.data_ptr(), q.shape[0], q.shape[1],
+                 q.stride(0), q.stride(1), gather_index.data_ptr(), scatter_index.data_ptr(),
+                 slot_valid.data_ptr(), heads.data_ptr(), hp, k.data_ptr(), k.stride(0),
+                 k.stride(1), v.data_ptr(), v.stride(0), v.stride(1), 128, r_tiles, n,
+                 full_cnt.data_ptr(), full_idx.data_ptr(), part_cnt.data_ptr(),
+                 part_idx.data_ptr(), part_idx.shape[3], kc.data_ptr(), vc.data_ptr(),
+                 kc.stride(0), kc.stride(1), keep.data_ptr(), valid_count.contiguous().data_ptr(),
+                 1.0 / math.sqrt(128), out.data_ptr(), out.shape[0], out.stride(0), out.stride(1),
+                 front_tiles, _stream(q))
+
+
 # --------------------------------------------------------------------------
 # predictor (miowtion/veda/predictor.py:251-338)
 
