@@ -49,6 +49,7 @@ int veda_abi_version(void);
  *   sq[h', t, :]  = E[x^2],  var[h', t, :] = centred Var(x) (two-pass form)
  *
  * x: bf16 [x_rows, H, D] with strides (x_stride_s, x_stride_h, 1).
+ * heads NULL: the first n_heads heads in order (pool_pair and scatter too).
  * out: bf16 [n_tiles*128, n_heads, D], strides (out_stride_s, out_stride_h, 1),
  *   or NULL to pool only (x is then usually already tile-ordered).
  * feats: fp32 [n_heads, n_tiles, 3D] contiguous, or NULL (no pooling).

@@ -126,7 +126,7 @@ __global__ void __launch_bounds__(64 * WAVES) gather_kernel(
   const int chunk = lane % kChunks;
   const int64_t hp = (int64_t)group * kHeadsPerGroup + hl;  // h'
   const bool head_ok = hp < n_heads;
-  const int64_t head = head_ok ? heads[hp] : 0;
+  const int64_t head = !head_ok ? 0 : heads != nullptr ? heads[hp] : hp;
   const bool src_head_ok = head_ok && head >= 0 && head < x_heads;
   constexpr int kSlots = kTile / WAVES;  // slots per wave
   static_assert(!SECOND || WAVES == kWaves, "the variance pass runs on kWaves waves");
@@ -325,7 +325,7 @@ __global__ void __launch_bounds__(SPLIT == 1 ? 64 * kWaves : 64 * SPLIT,
   const int chunk = lane % kChunks;
   const int64_t hp = (int64_t)group * kHeadsPerGroup + lane / kChunks;
   const bool head_ok = hp < n_heads;
-  const int64_t head = head_ok ? heads[hp] : 0;
+  const int64_t head = !head_ok ? 0 : heads != nullptr ? heads[hp] : hp;
   const bool src_head_ok = head_ok && head >= 0 && head < x_heads;
   // lanes of a missing head read head 0 of the row and keep zeros
   const int64_t lane_off = (src_head_ok ? head : 0) * xh + chunk * 8;
@@ -457,7 +457,7 @@ __global__ void __launch_bounds__(64 * WAVES) scatter_kernel(
   const int64_t hp = (int64_t)(blockIdx.x % n_groups) * kHeadsPerGroup + lane / kChunks;
   const int chunk = lane % kChunks;
   if (hp >= n_heads) return;
-  const int64_t head = heads[hp];
+  const int64_t head = heads != nullptr ? heads[hp] : hp;
   if (head < 0 || head >= out_heads) return;
   constexpr int kSlots = kTile / WAVES;
   const int64_t slot0 = (int64_t)tile * kTile + wave * kSlots;

@@ -74,7 +74,7 @@ def gather_tiles(x: torch.Tensor, layout: tiling.TileLayout,
                  heads: torch.Tensor | None) -> torch.Tensor:
     """[S, H, D] -> [N, H', D] tile order, padding slots zero."""
     return ops.gather(x, layout.gather_index, layout.slot_valid, layout.valid_count,
-                      _heads(x, heads), True, False, False)[0]
+                      heads, True, False, False)[0]
 
 
 def gather_and_pool(x: torch.Tensor, layout: tiling.TileLayout,
@@ -85,7 +85,7 @@ def gather_and_pool(x: torch.Tensor, layout: tiling.TileLayout,
     (E[x^2], Var(x)) [H', n, D] fp32 when `second`.
     """
     res = ops.gather(x, layout.gather_index, layout.slot_valid, layout.valid_count,
-                     _heads(x, heads), True, True, second)
+                     heads, True, True, second)
     return tuple(res)
 
 
@@ -94,7 +94,7 @@ def pool_seq(x: torch.Tensor, layout: tiling.TileLayout, heads: torch.Tensor | N
     """The pooling of gather_and_pool without writing the tile-ordered rows
     (one read of x): (feats,) or (feats, E[x^2], Var(x))."""
     res = ops.gather(x, layout.gather_index, layout.slot_valid, layout.valid_count,
-                     _heads(x, heads), False, True, second)
+                     heads, False, True, second)
     return tuple(res[1:])
 
 
@@ -103,7 +103,7 @@ def pool_seq_pair(x: torch.Tensor, x2: torch.Tensor, layout: tiling.TileLayout,
     """(pool_seq(x), pool_seq(x2)) of two tensors laid out alike, in one
     launch."""
     res = ops.pool_pair(x, x2, layout.gather_index, layout.slot_valid, layout.valid_count,
-                        _heads(x, heads), second)
+                        heads, second)
     half = len(res) // 2
     return tuple(res[:half]), tuple(res[half:])
 
@@ -116,7 +116,7 @@ def pool_tiles(x: torch.Tensor, layout: tiling.TileLayout, second: str | None = 
         raise ValueError(f'unknown second moment {second!r}')
     ident = _identity(layout)
     res = ops.gather(x, ident, layout.slot_valid, layout.valid_count,
-                     torch.arange(x.shape[1], device=x.device), False, True, second is not None)
+                     None, False, True, second is not None)
     if second is None:
         return res[1]
     return res[2] if second == SECOND_RAW else res[3]
@@ -134,7 +134,7 @@ def scatter_tiles_(out: torch.Tensor, tiled: torch.Tensor, layout: tiling.TileLa
     """Writes tile-ordered rows into out[S + 1, H, D] (padding slots dropped)."""
     if out.shape[0] != layout.seq_len + 1:
         raise ValueError(f'scatter buffer needs {layout.seq_len + 1} rows')
-    ops.scatter_(out, tiled, layout.scatter_index, layout.slot_valid, _heads(out, heads))
+    ops.scatter_(out, tiled, layout.scatter_index, layout.slot_valid, heads)
 
 
 def gather_lse(lse: torch.Tensor, layout: tiling.TileLayout, heads: torch.Tensor) -> torch.Tensor:

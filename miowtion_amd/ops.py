@@ -96,6 +96,10 @@ def _stream(t: torch.Tensor) -> int:
     return _raw_stream(t.device.index)  # the current stream of the tensor's device
 
 
+def _n_heads(x: torch.Tensor, heads: torch.Tensor | None) -> int:
+    return x.shape[1] if heads is None else heads.numel()
+
+
 def _p(t: torch.Tensor | None):
     return None if t is None else t.data_ptr()
 
@@ -113,10 +117,11 @@ def _check_rows(name: str, t: torch.Tensor) -> None:
 
 @_custom_op('veda::gather', mutates_args=())
 def gather(x: torch.Tensor, gather_index: torch.Tensor, slot_valid: torch.Tensor,
-           valid_count: torch.Tensor, heads: torch.Tensor, write_rows: bool, pool: bool,
+           valid_count: torch.Tensor, heads: torch.Tensor | None, write_rows: bool, pool: bool,
            second: bool) -> list[torch.Tensor]:
     """Returns [tiles] or [tiles, feats] or [tiles, feats, sq, var]; `tiles`
-    is an empty tensor when write_rows is False (pool-only)."""
+    is an empty tensor when write_rows is False (pool-only). heads None: every
+    head of x in order."""
     _require_gpu(x, gather_index, slot_valid, valid_count, heads)
     _check_rows('x', x)
     n_slots = gather_index.numel()
@@ -126,7 +131,7 @@ def gather(x: torch.Tensor, gather_index: torch.Tensor, slot_valid: torch.Tensor
     d = x.shape[-1]
     if d not in (64, 128):
         raise ValueError('tile kernels need contiguous head_dim 64 or 128')
-    hp = heads.numel()
+    hp = _n_heads(x, heads)
     dev = x.device
     out = (torch.empty(n_slots, hp, d, dtype=x.dtype, device=dev) if write_rows
            else torch.empty(0, dtype=x.dtype, device=dev))
@@ -138,7 +143,7 @@ def gather(x: torch.Tensor, gather_index: torch.Tensor, slot_valid: torch.Tensor
             var = torch.empty(hp, n_tiles, d, dtype=torch.float32, device=dev)
     _native.call('veda_gather_tiles', x.data_ptr(), x.shape[0], x.shape[1], x.stride(0),
                  x.stride(1), gather_index.data_ptr(), slot_valid.data_ptr(),
-                 valid_count.data_ptr(), n_tiles, heads.data_ptr(), hp, d,
+                 valid_count.data_ptr(), n_tiles, _p(heads), hp, d,
                  out.data_ptr() if write_rows else None,
                  out.stride(0) if write_rows else 0, out.stride(1) if write_rows else 0,
                  _p(feats), _p(sq), _p(var), _stream(x))
@@ -152,7 +157,7 @@ def gather(x: torch.Tensor, gather_index: torch.Tensor, slot_valid: torch.Tensor
 
 @gather.register_fake
 def _(x, gather_index, slot_valid, valid_count, heads, write_rows, pool, second):
-    n_slots, hp, d = gather_index.numel(), heads.numel(), x.shape[-1]
+    n_slots, hp, d = gather_index.numel(), _n_heads(x, heads), x.shape[-1]
     n_tiles = n_slots // TILE
     res = [x.new_empty(n_slots, hp, d) if write_rows else x.new_empty(0)]
     if pool:
@@ -164,7 +169,7 @@ def _(x, gather_index, slot_valid, valid_count, heads, write_rows, pool, second)
 
 @_custom_op('veda::pool_pair', mutates_args=())
 def pool_pair(x: torch.Tensor, x2: torch.Tensor, gather_index: torch.Tensor,
-              slot_valid: torch.Tensor, valid_count: torch.Tensor, heads: torch.Tensor,
+              slot_valid: torch.Tensor, valid_count: torch.Tensor, heads: torch.Tensor | None,
               second: bool) -> list[torch.Tensor]:
     """The pooling of two tensors laid out alike in one launch: [feats,
     feats2], or [feats, sq, var, feats2, sq2, var2] with `second`."""
@@ -176,7 +181,7 @@ def pool_pair(x: torch.Tensor, x2: torch.Tensor, gather_index: torch.Tensor,
     n_slots = gather_index.numel()
     if n_slots % TILE:
         raise ValueError('gather_index must hold n_tiles * 128 slots')
-    n_tiles, d, hp = n_slots // TILE, x.shape[-1], heads.numel()
+    n_tiles, d, hp = n_slots // TILE, x.shape[-1], _n_heads(x, heads)
     if d not in (64, 128):
         raise ValueError('tile kernels need contiguous head_dim 64 or 128')
     sizes = (3 * d, d, d) if second else (3 * d,)
@@ -185,32 +190,31 @@ def pool_pair(x: torch.Tensor, x2: torch.Tensor, gather_index: torch.Tensor,
     a, b = (p[:3], p[3:]) if second else ([p[0], None, None], [p[1], None, None])
     _native.call('veda_pool_pair', x.data_ptr(), x2.data_ptr(), x.shape[0], x.shape[1],
                  x.stride(0), x.stride(1), gather_index.data_ptr(), slot_valid.data_ptr(),
-                 valid_count.data_ptr(), n_tiles, heads.data_ptr(), hp, d, *a, *b, _stream(x))
+                 valid_count.data_ptr(), n_tiles, _p(heads), hp, d, *a, *b, _stream(x))
     return res
 
 
 @pool_pair.register_fake
 def _(x, x2, gather_index, slot_valid, valid_count, heads, second):
-    hp, n_tiles, d = heads.numel(), gather_index.numel() // TILE, x.shape[-1]
+    hp, n_tiles, d = _n_heads(x, heads), gather_index.numel() // TILE, x.shape[-1]
     return [x.new_empty(hp, n_tiles, n, dtype=torch.float32)
             for n in ((3 * d, d, d) if second else (3 * d,)) * 2]
 
 
 @_custom_op('veda::scatter_', mutates_args=('out',))
 def scatter_(out: torch.Tensor, tiled: torch.Tensor, scatter_index: torch.Tensor,
-             slot_valid: torch.Tensor, heads: torch.Tensor) -> None:
+             slot_valid: torch.Tensor, heads: torch.Tensor | None) -> None:
     _require_gpu(out, tiled, scatter_index, slot_valid, heads)
     _check_rows('out', out)
     _check_rows('tiled', tiled)
-    n_slots = scatter_index.numel()
-    if tiled.shape[0] != n_slots or tiled.shape[1] != heads.numel():
-        raise ValueError(f'tiled {tuple(tiled.shape)} does not match {n_slots} slots x '
-                         f'{heads.numel()} heads')
+    n_slots, hp = scatter_index.numel(), _n_heads(out, heads)
+    if tiled.shape[0] != n_slots or tiled.shape[1] != hp:
+        raise ValueError(f'tiled {tuple(tiled.shape)} does not match {n_slots} slots x {hp} heads')
     if tiled.dtype != out.dtype or tiled.shape[-1] != out.shape[-1]:
         raise ValueError('tiled and out differ in dtype or head_dim')
     _native.call('veda_scatter_tiles', tiled.data_ptr(), tiled.stride(0), tiled.stride(1),
                  scatter_index.data_ptr(), slot_valid.data_ptr(), n_slots // TILE,
-                 heads.data_ptr(), heads.numel(), out.shape[-1], out.data_ptr(),
+                 _p(heads), hp, out.shape[-1], out.data_ptr(),
                  out.shape[0], out.shape[1], out.stride(0), out.stride(1), _stream(out))
 
 

@@ -223,18 +223,12 @@ def build_tile_layout(spans: Sequence[TiledSpan], used: int, seq_len: int,
         slot_valid=dev((perm >= 0).astype(np.int32)))
 
 
-def _heads(x: torch.Tensor, heads: torch.Tensor | None) -> torch.Tensor:
-    if heads is None:
-        return torch.arange(x.shape[1], device=x.device)
-    return heads
-
-
 def gather_tiles(x: torch.Tensor, layout: TileLayout, heads: torch.Tensor | None) -> torch.Tensor:
     """[S, H, D] -> [N, H', D] in tile order, padding slots zero
     (tiling.py:278-297); the HIP gather kernel."""
     from miowtion_amd import ops
     return ops.gather(x, layout.gather_index, layout.slot_valid, layout.valid_count,
-                      _heads(x, heads), True, False, False)[0]
+                      heads, True, False, False)[0]
 
 
 def scatter_tiles_(out: torch.Tensor, tiled: torch.Tensor, layout: TileLayout,
@@ -244,4 +238,4 @@ def scatter_tiles_(out: torch.Tensor, tiled: torch.Tensor, layout: TileLayout,
     from miowtion_amd import ops
     if out.shape[0] != layout.seq_len + 1:
         raise ValueError(f'scatter buffer needs {layout.seq_len + 1} rows')
-    ops.scatter_(out, tiled, layout.scatter_index, layout.slot_valid, _heads(out, heads))
+    ops.scatter_(out, tiled, layout.scatter_index, layout.slot_valid, heads)

@@ -61,3 +61,21 @@ def test_a_pair_pools_as_its_tensors_alone(dim, second):
                 assert torch.equal(a, b)
     with pytest.raises(ValueError, match='laid out'):
         kernels.pool_seq_pair(x, y[:, 1:], lay, heads)
+
+
+@pytest.mark.parametrize('dim', [64, 128])
+@pytest.mark.parametrize('heads', [1, 5, 16])
+def test_no_heads_is_every_head_in_order(dim, heads):
+    lay = helpers.product_layout(*helpers.small_layout(), device='cuda')
+    x, y = (t.cuda() for t in helpers.qkv(lay.seq_len, heads, dim, seed=heads, n=2))
+    every = torch.arange(heads, device='cuda')
+
+    def run(h):
+        tiles = kernels.gather_tiles(x, lay, h)
+        out = torch.full((lay.seq_len + 1, heads, dim), 7., dtype=torch.bfloat16, device='cuda')
+        kernels.scatter_tiles_(out, tiles, lay, h)
+        return [tiles, out, *kernels.gather_and_pool(x, lay, h, second=True),
+                *kernels.pool_seq(x, lay, h), *kernels.pool_seq_pair(x, y, lay, h)[1]]
+
+    for a, b in zip(run(None), run(every)):
+        assert torch.equal(a, b)
