@@ -1,9 +1,9 @@
 // Flash-attention forwards for gfx950 (head_dim 128, bf16 in, fp32
-// accumulate). Two kernels share the step, fragment and load code below:
+// accumulate). Three kernels share the step, fragment and load code below:
 //   hfwd_kernel  the teacher's pass over all key tiles in tile order with
 //                the dense output (and the block heat statistics);
 //   tstats_kernel the same pass without the output (LSE and statistics
-//                only), four query tiles per K pass;
+//                only), four query tiles per K pass, pipelined by sub-block;
 //   sfwd_kernel  the block-sparse forward, the zero-order compensation and
 //                the dense forward of packed rows (two 4-wave workgroups
 //                per CU, described at its section).
@@ -631,8 +631,8 @@ __device__ __forceinline__ void pack_probs(const float (&ps)[16], u32x4 (&pk)[2]
 // a partial query tile, whose gathered q is zero): every valid key scores
 // exactly 0, so P is 1 on the valid keys and 0 on the masked ones, the
 // running max is 0 from the first valid key on and the row sum counts the
-// valid keys. Only the P.V products remain; the result is bit-identical to
-// sstep's on the same rows (the same products of the same exact P).
+// valid keys. Only the P.V products remain: the same products of the same
+// exact P as a full walk of those rows.
 __device__ __forceinline__ void sstep_zero_q(const lds_u8* slot, const HFrag& f, int la, int lb,
                                              int hi, WaveState& w) {
   if (la <= 0 && lb <= 0) return;  // no valid key: P is 0 everywhere
@@ -817,8 +817,7 @@ __device__ __forceinline__ void pstage(const lds_u8* kb, const lds_u8* vb, const
 
 // A step of 64 virtual keys (the summaries of key tiles key0 .. key0 + 63)
 // of the compensation of a given output: both sub-blocks' score products as
-// interleaved chains (pair_scores, no key masked: virtual keys past n_k
-// carry weight 0); then per sub-block p = exp2(s c - ref2) where the tile's
+// interleaved chains (no key masked: virtual keys past n_k carry weight 0); then per sub-block p = exp2(s c - ref2) where the tile's
 // weight (its real row count if dropped, else 0) is positive, den += p *
 // weight, and O^T += V^T P^T, sub-block a's terms before b's.
 //
@@ -989,9 +988,10 @@ __device__ __forceinline__ void vstep_fixed_half(const lds_u8* slot, const HFrag
 }
 
 // One step of 64 virtual keys inside the online softmax (compensated
-// attention): as sstep, with each key weighted by its tile's dropped
-// real-row count (the denominator gains p * weight; the value is the
-// tile's sum of V) and weight-0 keys masked out of the max.
+// attention): scores, one update of the running max for both sub-blocks, P.V
+// products; each key is weighted by its tile's dropped real-row count (the
+// denominator gains p * weight; the value is the tile's sum of V) and weight-0
+// keys are masked out of the max.
 __device__ __forceinline__ void sstep_virtual(const lds_u8* slot, const HFrag& fa,
                                               const HFrag& fb, float c, const uint8_t* wt,
                                               int key0, int hi, WaveState& w) {
