@@ -15,7 +15,8 @@
 //   dq_kernel         workgroup = (head, query tile), walking the forward
 //                     block lists (the key tiles of the row).
 //   dkv_kernel        workgroup = (head, key tile), walking the transposed
-//                     lists (the query tiles of the column).
+//                     lists (the query tiles of the column); dkv_wide_kernel
+//                     where a launch has many of them.
 // Per pair of a 64-row and a 64-key half:
 //   P  = exp2(S * scale * log2(e) - lse2)   (0 past the key tile's valid count)
 //   dP = dO V^T,  dS = P * (dP - D)
@@ -57,6 +58,15 @@ constexpr int kHiZeroFlag = 129;                 // 1 if rows 32 .. 63 have dO =
 constexpr int kRecBytes = kRecFloats * 4;
 constexpr int kDqThreads = 256;
 constexpr int kDkvThreads = 512;
+constexpr int kDkvWideThreads = 256;
+// Launches of at least this many (head, key tile) workgroups take 32 keys a
+// wave: one and a half rounds of the 512 that are resident. In a single round
+// the longer workgroups cost more than their LDS reads save. dK, dV with 16
+// and with 32 keys a wave: 276 items (23 tiles x 12 heads) 70 and 83 us; 592
+// (592 x 1) 271 and 266; 960 (20 x 48) 84 and 62; 1,008 (126 x 8) 155 and
+// 127; 1,184 (592 x 2) 502 and 478; 3,024 (126 x 24) 440 and 344; 9,472
+// (592 x 16) 3,821 and 3,264.
+constexpr int64_t kDkvWideItems = 768;
 constexpr int kSlot = 2 * kHalfBytes;            // K + V (dq) or Q + dO (dkv) of a step
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -829,6 +839,333 @@ __global__ void __launch_bounds__(kDkvThreads) __attribute__((amdgpu_waves_per_e
   }
 }
 
+// ---------------------------------------------------------------------------
+// dK, dV with 32 keys a wave, for launches of many workgroups. Workgroup =
+// (head, key tile), 4 waves, two workgroups per CU as in dq_kernel. A wave
+// owns 32 keys (K^T and V^T fragments in registers, one key per lane pair)
+// and per block of 32 query rows runs the whole chain on v_mfma_f32_32x32x16:
+//   S = Q K^T, dP - D = dO V^T - D   (8 MFMAs each, A = Q / dO rows from LDS)
+//   P = exp2(S c - lse2), dS = P (dP - D)
+//   dV^T += dO^T P, dK^T += Q^T dS   (8 MFMAs each, A = dO^T / Q^T from
+//                                     transposed reads)
+// The vector work of a block runs under products that do not need it: the
+// exponentials under dP's, dS under dV's, one piece a product.
+//
+// A block reads each row of Q and dO twice from LDS whatever the number of
+// keys, so 32 keys a wave halve dkv_kernel's LDS reads per product, which
+// bound it. The sums of 128 x 32 dK and dV take 128 registers and the
+// fragments of K and V 64, so it fits the 256 of two waves per SIMD only with
+// nothing kept that can be formed again (the lane's index, read and load
+// offsets) and fragments read two products ahead. It has to fit: with eight
+// registers spilled, reloads waited for the step's loads (a scratch read
+// counts as one), and the kernel took 17 % longer. A workgroup lasts about
+// twice as long as dkv_kernel's, two at a time on a CU, so a launch needs
+// more than a round of them (kDkvWideItems). dK, dV alone, 16 -> 32 keys:
+// 57,720 tokens x 16 heads, keep 0.1: 3.82 -> 3.26 ms; 13x24x42 tokens x 24
+// heads: 440 -> 344 us. Four fragments ahead in the first and last phase: the
+// same.
+//
+// Key tiles with few valid keys spread a step's rows over more waves, which
+// add their partial sums at the end: vc > 64: 4 key groups, each wave both
+// row blocks of a step; 32 < vc <= 64: 2 key groups x 2 row blocks; vc <= 32:
+// 1 x 2 (the other two waves only load).
+
+// The lane's index, formed anew at each call, so that what is derived from it
+// holds no register between its uses.
+__device__ __forceinline__ int fresh_lane() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
+}
+
+__global__ void __launch_bounds__(kDkvWideThreads, 2) dkv_wide_kernel(BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[2][kSlot + kRecBytes];
+  __shared__ uint16_t steps[2 * kMaxTiles];
+  __shared__ int32_t step_total, step_hz;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int li = lane & 31, hi = lane >> 5;
+  int64_t head, j;
+  front_first(blockIdx.x, p.n_heads, p.n_k_tiles, p.front, head, j);
+  const int vc = __builtin_amdgcn_readfirstlane(clamp_vc(p.valid_count[j]));
+  const int nq = (int)p.n_q_tiles;
+
+  if (wave == 0) {
+    const int64_t lr = head * p.n_k_tiles + j;
+    int nf, np;
+    list_counts(p.full_cnt_t, p.part_cnt_t, lr, p.list_ld_t, nf, np);
+    // A 64-row half whose rows all have dO = 0 and D = 0 (the padding rows
+    // of a partial query tile when the caller's gradient comes through the
+    // scatter, which drops them) adds exactly zero to dK and dV: no step. One
+    // whose rows 32 .. 63 alone have them is an upper-zero step: only its
+    // first 32 rows are computed; these come after the others.
+    const float* zrec = p.stats + head * 2 * p.n_q_tiles * kRecFloats + kZeroFlag;
+    int n_hz;
+    const int cnt = build_steps(p.full_idx_t + lr * p.list_ld_t, nf,
+                                p.part_idx_t + lr * p.list_ld_t, np, lane, steps, [&](int t) {
+                                  if (vc <= 0 || t < 0 || t >= nq) return 0;
+                                  const float* r0 = zrec + (2 * t) * kRecFloats;
+                                  const float* r1 = r0 + kRecFloats;
+                                  constexpr int h = kHiZeroFlag - kZeroFlag;
+                                  return (r0[0] != 0.f ? 0 : 1) | (r1[0] != 0.f ? 0 : 2) |
+                                         (r0[h] != 0.f ? 4 : 0) | (r1[h] != 0.f ? 8 : 0);
+                                }, n_hz);
+    if (lane == 0) {
+      step_total = cnt;
+      step_hz = n_hz;
+    }
+  }
+  // this wave's keys, and the row block of a step that it takes (rb < 0: both)
+  const int n_groups = vc > 64 ? 4 : vc > 32 ? 2 : 1;
+  const int kgrp = wave & (n_groups - 1);
+  const int rb = n_groups == 4 ? -1 : wave / n_groups;
+  const bool live = 32 * kgrp < vc && rb < 2;
+  const int key = 32 * kgrp + li;
+  const bool key_ok = key < vc;
+  const int64_t krow = j * kTile + key;
+  bf16x8 kf[8], vf[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    kf[s] = as_bf16x8(ld16(p.k + krow * p.ks + head * p.kh + 16 * s + 8 * hi));
+    vf[s] = as_bf16x8(ld16(p.v + krow * p.vs + head * p.vh + 16 * s + 8 * hi));
+  }
+  f32x16 acc_v[4], acc_k[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc_v[dt][e] = acc_k[dt][e] = 0.f;
+  __syncthreads();
+  // steps 0 .. n_full - 1 are the others, n_full .. n_steps - 1 upper-zero
+  const int n_full = __builtin_amdgcn_readfirstlane(step_total);
+  const int n_steps = n_full + __builtin_amdgcn_readfirstlane(step_hz);
+  auto entry = [&](int u) {
+    return __builtin_amdgcn_readfirstlane(
+        (int)steps[u < n_full ? u : 2 * kMaxTiles - 1 - (u - n_full)]);
+  };
+
+  const uint16_t* qbase = p.q + head * p.qh;
+  const uint16_t* dbase = p.dout + head * p.doh;
+  // Segment 4 wave + s of a step's Q or dO holds rows 16 wave + 4 s + lane / 16:
+  // swz of a row is 4 (lane / 16) + s, so its byte offset is the row's plus
+  // (chunk ^ s) 16, and 4 s rows go into the base. A read's offset likewise is
+  // one register xor a constant (k-step 2 s + hi: xor 32 s; transposed: dt:
+  // xor 64 dt, rows + 8: xor 2048 + 32). Kept as xors: 24 offsets held in
+  // registers would not fit beside the accumulators.
+  const float c = p.scale_log2;
+
+  auto load_step = [&](int u, lds_u8* slot) {
+    const int t = entry(u);
+    const int64_t row0 = (int64_t)(t >> 1) * kTile + (t & 1) * kHalf;
+    const int ln = fresh_lane();
+    const int r16 = ln >> 4;
+    const uint32_t ch = (uint32_t)(((ln & 15) ^ (4 * r16)) << 4);
+    const uint32_t qrow = (uint32_t)((16 * wave + r16) * p.qs * 2);
+    const uint32_t drow = (uint32_t)((16 * wave + r16) * p.dos * 2);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      dma16(reinterpret_cast<const char*>(qbase + (row0 + 4 * s) * p.qs), (ch ^ (s << 4)) + qrow,
+            slot + (4 * wave + s) * 1024);
+      dma16(reinterpret_cast<const char*>(dbase + (row0 + 4 * s) * p.dos), (ch ^ (s << 4)) + drow,
+            slot + kHalfBytes + (4 * wave + s) * 1024);
+    }
+    if (wave == 0) {
+      const float* rec = p.stats + (head * 2 * p.n_q_tiles + t) * kRecFloats;
+      dma16(reinterpret_cast<const char*>(rec), (uint32_t)(ln * 16), slot + kSlot);
+    }
+  };
+
+  lds_u8* s0 = (lds_u8*)ring[0];
+  lds_u8* s1 = (lds_u8*)ring[1];
+  // FULL: every key of the tile valid.
+  auto body = [&](auto full) __attribute__((always_inline)) {
+    constexpr bool FULL = decltype(full)::value;
+    // rows 32 b .. 32 b + 31 of the step in `slot`
+    auto compute = [&](int b, const lds_u8* slot) __attribute__((always_inline)) {
+      const int ln = fresh_lane(), hi = ln >> 5;
+      const Frag f = frag_offsets(ln);
+      const uint32_t ra = f.row[0], ta = f.tr[0][0];
+      const lds_u8* qs = slot + b * 8192;
+      const lds_u8* ds = slot + kHalfBytes + b * 8192;
+      const lds_u8* rec = slot + kSlot + 128 * b + 16 * hi;  // rows 8 m + 4 hi + {0..3}: + 32 m
+      f32x16 st, dp;
+      u32x4 qa[8], da[8];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) qa[s] = lds16(qs + (ra ^ (32 * s)));
+#pragma unroll
+      for (int e = 0; e < 16; ++e) st[e] = 0.f;
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        if (s + 2 < 8) qa[s + 2] = lds16(qs + (ra ^ (32 * (s + 2))));
+        else da[s - 6] = lds16(ds + (ra ^ (32 * (s - 6))));
+        if (s >= 4) {
+          const f32x4 nd = *reinterpret_cast<const lds_f32x4*>(rec + 256 + 32 * (s - 4));
+#pragma unroll
+          for (int m = 0; m < 4; ++m) dp[4 * (s - 4) + m] = nd[m];  // -D
+        }
+        st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(qa[s]), kf[s], st, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // dP, and the exponentials of S two at a time
+      u32x4 pp[2], pd[2];
+      float pr[16];
+      f32x4 l4;
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        if (s + 2 < 8) da[s + 2] = lds16(ds + (ra ^ (32 * (s + 2))));
+        if ((s & 1) == 0) l4 = *reinterpret_cast<const lds_f32x4*>(rec + 16 * s);
+        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(da[s]), vf[s], dp, 0, 0, 0);
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          const int e = 2 * s + m;
+          const float x = __builtin_amdgcn_exp2f(fmaf(st[e], c, -l4[e & 3]));
+          pr[e] = FULL || key_ok ? x : 0.f;
+        }
+        pp[s >> 2][s & 3] = pack_bf16x2(pr[2 * s], pr[2 * s + 1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // dV, and dS two at a time
+      auto tr = [&](const lds_u8* base, int i) {  // product i: 16 rows i / 4, head-dims 32 (i % 4)
+        const uint32_t at = ta ^ (64 * (i & 3));
+        const lds_u8* x = base + (i >> 2) * 4096;
+        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(x + at));
+        const i16x4 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(x + (at ^ 2080)));
+        return __builtin_bit_cast(u32x4, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
+      };
+      u32x4 ta_[8], tq[8];
+      ta_[0] = tr(ds, 0);
+      ta_[1] = tr(ds, 1);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (i + 2 < 8) ta_[i + 2] = tr(ds, i + 2);
+        else tq[i - 6] = tr(qs, i - 6);
+        acc_v[i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            as_bf16x8(ta_[i]), as_bf16x8(pp[i >> 2]), acc_v[i & 3], 0, 0, 0);
+        float y[2];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          y[m] = pr[2 * i + m] * dp[2 * i + m];  // dp holds dP - D
+          if (!FULL) y[m] = key_ok ? y[m] : 0.f;
+        }
+        pd[i >> 2][i & 3] = pack_bf16x2(y[0], y[1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (i + 2 < 8) tq[i + 2] = tr(qs, i + 2);
+        acc_k[i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            as_bf16x8(tq[i]), as_bf16x8(pd[i >> 2]), acc_k[i & 3], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // Step u: wait for this wave's loads (the only ones in flight), barrier
+    // (every wave's loads of step u are in LDS and every wave is done reading
+    // the other slot), issue step u + 1 into the other slot, compute step u.
+    auto run = [&](int u, lds_u8* cur, lds_u8* nxt) __attribute__((always_inline)) {
+      VEDA_WAIT_VM(0);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (u + 1 < n_steps) load_step(u + 1, nxt);
+      if (!live) return;
+      const int last = u < n_full ? 1 : 0;  // the last row block with anything to add
+      if constexpr (FULL) {
+        compute(0, cur);
+        if (last) compute(1, cur);
+      } else {
+        const int end = rb < 0 ? last : min(last, rb);
+#pragma unroll 1
+        for (int b = max(rb, 0); b <= end; ++b) compute(b, cur);
+      }
+    };
+    if (n_steps > 0) load_step(0, s0);
+    for (int u = 0; u < n_steps; u += 2) {
+      run(u, s0, s1);
+      if (u + 1 >= n_steps) break;
+      run(u + 1, s1, s0);
+    }
+  };
+  if (vc == kTile)
+    body(std::true_type{});
+  else
+    body(std::false_type{});
+
+  __syncthreads();  // every wave is done with the ring
+  const int ln = fresh_lane();
+  if (n_groups < 4) {
+    // row block 1's waves hand their partial sums to row block 0's, dV
+    // first, then dK
+    lds_f32x4* red = reinterpret_cast<lds_f32x4*>(s0) + ln;
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+      f32x16(&a)[4] = pass == 0 ? acc_v : acc_k;
+      if (rb == 1) {
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            red[(kgrp * 16 + 4 * dt + g) * 64] =
+                f32x4{a[dt][4 * g], a[dt][4 * g + 1], a[dt][4 * g + 2], a[dt][4 * g + 3]};
+          }
+      }
+      __syncthreads();
+      if (rb == 0) {
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 x = red[(kgrp * 16 + 4 * dt + g) * 64];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) a[dt][4 * g + m] += x[m];
+          }
+      }
+      __syncthreads();
+    }
+    // the waves past the key groups write the zeros of the tile's other keys
+    if (rb > 0) {
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc_v[dt][e] = acc_k[dt][e] = 0.f;
+    }
+  }
+  // Wave w writes rows 32 w .. + 31 of the tile as whole rows, by way of its
+  // 8 KB of the ring (as dq_kernel), dV first, then dK.
+  lds_u8* stage = s0 + wave * 8192;
+#pragma unroll
+  for (int pass = 0; pass < 2; ++pass) {
+    const f32x16(&a)[4] = pass == 0 ? acc_v : acc_k;
+    const float m = pass == 0 ? 1.f : p.scale;
+    uint16_t* base = pass == 0 ? p.dv : p.dk;
+    const int64_t ss = pass == 0 ? p.dvs : p.dks, sh = pass == 0 ? p.dvh : p.dkh;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int e0 = 4 * g;
+        *reinterpret_cast<__attribute__((address_space(3))) u32x2*>(
+            stage + (ln & 31) * 256 + (((4 * dt + g) ^ (ln & 15)) << 4) + 8 * (ln >> 5)) =
+            u32x2{pack_bf16x2(a[dt][e0] * m, a[dt][e0 + 1] * m),
+                  pack_bf16x2(a[dt][e0 + 2] * m, a[dt][e0 + 3] * m)};
+      }
+    asm volatile("" ::: "memory");
+    const bool row16 = ((reinterpret_cast<uintptr_t>(base) & 15) | ((ss | sh) & 7)) == 0;
+    uint16_t* rows = base + (j * kTile + 32 * wave) * ss + head * sh;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int rr = 4 * i + (ln >> 4), ch = ln & 15;
+      const u32x4 x = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(
+          stage + rr * 256 + ((ch ^ (rr & 15)) << 4));
+      uint16_t* dst = rows + rr * ss + 8 * ch;
+      if (row16) {
+        *reinterpret_cast<u32x4*>(dst) = x;
+      } else {  // rows 8-byte aligned only
+        *reinterpret_cast<u32x2*>(dst) = u32x2{x[0], x[1]};
+        *reinterpret_cast<u32x2*>(dst + 4) = u32x2{x[2], x[3]};
+      }
+    }
+    asm volatile("" ::: "memory");
+  }
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
 
@@ -920,7 +1257,10 @@ extern "C" int veda_block_sparse_bwd(
     if (int rc = check_launch("veda_block_sparse_bwd (dq)")) return rc;
   }
   if (k_items > 0) {
-    dkv_kernel<<<(unsigned)k_items, kDkvThreads, 0, s>>>(p);
+    if (k_items >= kDkvWideItems)
+      dkv_wide_kernel<<<(unsigned)k_items, kDkvWideThreads, 0, s>>>(p);
+    else
+      dkv_kernel<<<(unsigned)k_items, kDkvThreads, 0, s>>>(p);
     return check_launch("veda_block_sparse_bwd (dk, dv)");
   }
   return VEDA_OK;
