@@ -817,8 +817,9 @@ __device__ __forceinline__ void pstage(const lds_u8* kb, const lds_u8* vb, const
 
 // A step of 64 virtual keys (the summaries of key tiles key0 .. key0 + 63)
 // of the compensation of a given output: both sub-blocks' score products as
-// interleaved chains (no key masked: virtual keys past n_k carry weight 0); then per sub-block p = exp2(s c - ref2) where the tile's
-// weight (its real row count if dropped, else 0) is positive, den += p *
+// interleaved chains (no key masked: virtual keys past n_k carry weight 0);
+// then per sub-block p = exp2(s c - ref2) where the tile's weight (its real
+// row count if dropped, else 0) is positive, den += p *
 // weight, and O^T += V^T P^T, sub-block a's terms before b's.
 //
 // With the reference fixed, nothing of sub-block a waits for b's scores (no
