@@ -715,23 +715,36 @@ __device__ __forceinline__ void sstep_half_zero(const lds_u8* slot, const HFrag&
 // (the same board multiplies random bf16 matrices at 1.5 and zeros at 2.0
 // PFLOP/s). Sparse walks, where K and V come from beyond L2: sequence order
 // 6.08 -> 5.92 ms the whole layer (with the dead waves dropped), 14.64 ->
-// 14.12 at keep 0.2, tile order 5.58 -> 5.54 ms.
+// 14.12 at keep 0.2; tile order 5.56 -> 5.51 ms, 12.67 -> 12.35 at keep 0.2.
 //
-// The reference of a row is the maximum of its first sub-block; later
-// probabilities are taken against it as it stands, with no maximum taken,
-// unless a lane's 16 probabilities sum to kLazyLimit or more (or are not
-// finite), or a row has no reference yet: then the sub-block runs the online
-// softmax (raise_reference), which rescales O and l and takes the
-// probabilities again.
-constexpr float kLazyLimit = 4096.f;
+// The reference of a row is the maximum of its first step's 64 keys (narrow
+// walks: of its first sub-block); later probabilities are taken against it as
+// it stands, with no maximum taken, unless a lane's 16 probabilities sum to
+// kLazyLimit or more (or are not finite), or a row has no reference yet: then
+// the sub-block runs the online softmax (raise_reference), which raises the
+// references that a score passes by more than kRescaleSlack (2^8, which
+// kLazyLimit does not let by), rescales O and l and takes the probabilities
+// again. A key whose score is the reference has the probability 1, which bf16
+// holds exactly; with references from 32 keys, raised only past 2^12, the
+// largest probability of more rows is rounded (short training step: 2.28e-3
+// from 64 bits instead of 2.26e-3). Neither takes time: 57,720 tokens x 48
+// heads, keep 0.1, tile order 5.54 -> 5.51 ms.
+constexpr float kLazyLimit = 256.f;
 
 // The pipeline's state beside WaveState: the factor O is still to be scaled
-// by (the reference rose in the last softmax) and whether every row of the
-// wave has a reference.
+// by (the reference rose in the last softmax), whether every row of the wave
+// has a reference, and the sum of a step's first sub-block until the second's
+// joins it (l adds up whole steps).
 struct PipeState {
   float alpha;
   bool have_ref;
+  float first_sum = 0.f;
 };
+
+// Which sub-block a stage's softmax is of: none; the only one of its step
+// (narrow walks), whose sum is added to l at once; or the first or the second
+// of a step of 64 keys, whose sums are added together.
+enum { kNoSm = 0, kSmOnly = 1, kSmFirst = 2, kSmSecond = 3 };
 
 __device__ __forceinline__ void raise_reference(const f32x16& s, float c, u32x4 (&pk)[2],
                                                 WaveState& w, PipeState& ps) {
@@ -756,7 +769,21 @@ __device__ __forceinline__ void raise_reference(const f32x16& s, float c, u32x4 
   ps.have_ref = __ballot(m_new != -INFINITY) == ~0ull;
 }
 
-template <bool QK, bool SM, bool PV, typename Hook>
+// The references of a walk's rows from its first step's two sub-blocks (la
+// and lb valid keys).
+__device__ __forceinline__ void first_reference(f32x16& sa, f32x16& sb, float c, int la, int lb,
+                                                int hi, WaveState& w, PipeState& ps) {
+  mask_scores(sa, la, hi);
+  mask_scores(sb, lb, hi);
+  float mloc = -INFINITY;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) mloc = fmaxf(mloc, fmaxf(sa[e], sb[e]));
+  w.m_run = half_swap_max(mloc) * c;
+  w.mu = w.m_run == -INFINITY ? 0.f : w.m_run;
+  ps.have_ref = __ballot(w.m_run != -INFINITY) == ~0ull;
+}
+
+template <bool QK, int SM, bool PV, typename Hook>
 __device__ __forceinline__ void pstage(const lds_u8* kb, const lds_u8* vb, const HFrag& f, float c,
                                        int lim, int hi, f32x16& sn, f32x16& sp, u32x4 (&pn)[2],
                                        const u32x4 (&pp)[2], WaveState& w, PipeState& ps, Hook hook) {
@@ -808,10 +835,15 @@ __device__ __forceinline__ void pstage(const lds_u8* kb, const lds_u8* vb, const
   ps.alpha = 1.f;
   if (SM) {
     const float lsum = (l4[0] + l4[1]) + (l4[2] + l4[3]);
-    if (__builtin_expect(ps.have_ref && __ballot(lsum < kLazyLimit) == ~0ull, 1))
-      w.l_run += lsum;
-    else if (lim > 0)
-      raise_reference(sp, c, pn, w, ps);
+    if (__builtin_expect(!(ps.have_ref && __ballot(lsum < kLazyLimit) == ~0ull), 0)) {
+      if (SM == kSmSecond) w.l_run += ps.first_sum;
+      ps.first_sum = 0.f;
+      if (lim > 0) raise_reference(sp, c, pn, w, ps);
+    } else if (SM == kSmFirst) {
+      ps.first_sum = lsum;
+    } else {
+      w.l_run += SM == kSmSecond ? ps.first_sum + lsum : lsum;
+    }
   }
 }
 
@@ -1696,11 +1728,13 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
       const lds_u8* const kz = s0;  // unused operands of partial stages
       const int h = 8192 * (wave & 1);  // a narrow wave's sub-block
       if constexpr (K == 0) {
-        pstage<true, false, false>(s0, kz, fa, c, 32, hi, sa, sb, pb, pa, w, ps, NoHook{});
-        pstage<true, true, false>(s0 + 8192, kz, fa, c, (int)(r0.a & 63u), hi, sb, sa, pa, pb, w, ps,
-                                  NoHook{});
+        pstage<true, kNoSm, false>(s0, kz, fa, c, 32, hi, sa, sb, pb, pa, w, ps, NoHook{});
+        pstage<true, kNoSm, false>(s0 + 8192, kz, fa, c, 32, hi, sb, sa, pa, pb, w, ps, NoHook{});
+        first_reference(sa, sb, c, (int)(r0.a & 63u), (int)(r0.b & 63u), hi, w, ps);
+        pstage<false, kSmFirst, false>(kz, kz, fa, c, (int)(r0.a & 63u), hi, sb, sa, pa, pb, w, ps,
+                                   NoHook{});
       } else if constexpr (K == 3) {
-        pstage<true, false, false>(s0 + h, kz, fa, c, 32, hi, sa, sb, pb, pa, w, ps, NoHook{});
+        pstage<true, kNoSm, false>(s0 + h, kz, fa, c, 32, hi, sa, sb, pb, pa, w, ps, NoHook{});
       }
       // iteration u < n - 1: K of step u + 1 in nxt, V of step u in cur
       auto iter = [&](lds_u8* cur, lds_u8* nxt, uint32_t lcur, uint32_t lnxt, int u)
@@ -1717,13 +1751,13 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
         auto hook = [&](int j) { issue(kb, vb, o2, ov, j, lcur, lnxt); };
         const int la0 = (int)(r0.a & 63u), lb0 = (int)(r0.b & 63u), la1 = (int)(r1.a & 63u);
         if constexpr (K == 0) {
-          pstage<true, true, true>(nxt, cur, fa, c, lb0, hi, sa, sb, pb, pa, w, ps, hook);
-          pstage<true, true, true>(nxt + 8192, cur + 8192, fa, c, la1, hi, sb, sa, pa, pb, w, ps,
+          pstage<true, kSmSecond, true>(nxt, cur, fa, c, lb0, hi, sa, sb, pb, pa, w, ps, hook);
+          pstage<true, kSmFirst, true>(nxt + 8192, cur + 8192, fa, c, la1, hi, sb, sa, pa, pb, w, ps,
                                    NoHook{});
         } else if constexpr (K == 3) {
-          pstage<true, true, false>(nxt + h, kz, fa, c, (wave & 1) ? lb0 : la0, hi, sb, sa, pa, pb, w,
+          pstage<true, kSmOnly, false>(nxt + h, kz, fa, c, (wave & 1) ? lb0 : la0, hi, sb, sa, pa, pb, w,
                                     ps, hook);
-          pstage<false, false, true>(kz, cur + h, fa, c, 32, hi, sb, sa, pb, pa, w, ps, NoHook{});
+          pstage<false, kNoSm, true>(kz, cur + h, fa, c, 32, hi, sb, sa, pb, pa, w, ps, NoHook{});
           sa = sb;
         } else {
 #pragma unroll
@@ -1748,12 +1782,12 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
       if (virt_next) load_virtual(0, s0 + (n_lsteps & 1) * kSlotBytes);
       const int la0 = (int)(r0.a & 63u), lb0 = (int)(r0.b & 63u);
       if constexpr (K == 0) {
-        pstage<false, true, true>(kz, cur, fa, c, lb0, hi, sa, sb, pb, pa, w, ps, NoHook{});
-        pstage<false, false, true>(kz, cur + 8192, fa, c, 32, hi, sb, sa, pa, pb, w, ps, NoHook{});
+        pstage<false, kSmSecond, true>(kz, cur, fa, c, lb0, hi, sa, sb, pb, pa, w, ps, NoHook{});
+        pstage<false, kNoSm, true>(kz, cur + 8192, fa, c, 32, hi, sb, sa, pa, pb, w, ps, NoHook{});
       } else if constexpr (K == 3) {
-        pstage<false, true, false>(kz, kz, fa, c, (wave & 1) ? lb0 : la0, hi, sb, sa, pa, pb, w, ps,
+        pstage<false, kSmOnly, false>(kz, kz, fa, c, (wave & 1) ? lb0 : la0, hi, sb, sa, pa, pb, w, ps,
                                    NoHook{});
-        pstage<false, false, true>(kz, cur + h, fa, c, 32, hi, sb, sa, pb, pa, w, ps, NoHook{});
+        pstage<false, kNoSm, true>(kz, cur + h, fa, c, 32, hi, sb, sa, pb, pa, w, ps, NoHook{});
       } else {
         if constexpr (K == 1) sstep_zero_q(cur, fa, la0, lb0, hi, w);
         if constexpr (K == 4) sstep_half_zero(cur + h, fa, (wave & 1) ? lb0 : la0, hi, w);
@@ -1862,10 +1896,10 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
       kp += k_step;
       vp += v_step;
       sync();
-      pstage<true, true, true>(nxt, cur, fa, c, 32, hi, sa, sb, pb, pa, w, ps,
+      pstage<true, kSmSecond, true>(nxt, cur, fa, c, 32, hi, sa, sb, pb, pa, w, ps,
                                [&](int j) { issue(kb, vb, j, lcur, lnxt); });
       if (M) mask_front(sa, u + 1, 0);
-      pstage<true, true, true>(nxt + 8192, cur + 8192, fa, c, 32, hi, sb, sa, pa, pb, w, ps,
+      pstage<true, kSmFirst, true>(nxt + 8192, cur + 8192, fa, c, 32, hi, sb, sa, pa, pb, w, ps,
                                NoHook{});
       if (M) mask_front(sb, u + 1, 1);
     };
@@ -1892,10 +1926,12 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
       }
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      pstage<true, false, false>(s0, s0, fa, c, 32, hi, sa, sb, pb, pa, w, ps, NoHook{});
+      pstage<true, kNoSm, false>(s0, s0, fa, c, 32, hi, sa, sb, pb, pa, w, ps, NoHook{});
       mask_front(sa, 0, 0);
-      pstage<true, true, false>(s0 + 8192, s0, fa, c, 32, hi, sb, sa, pa, pb, w, ps, NoHook{});
+      pstage<true, kNoSm, false>(s0 + 8192, s0, fa, c, 32, hi, sb, sa, pb, pa, w, ps, NoHook{});
       mask_front(sb, 0, 1);
+      first_reference(sa, sb, c, 32, 32, hi, w, ps);
+      pstage<false, kSmFirst, false>(s0, s0, fa, c, 32, hi, sb, sa, pa, pb, w, ps, NoHook{});
       int u = 0;
       for (; u + 4 < n_steps; u += 2) {
         iter(std::false_type{}, u, s0, s1, lds_s0, lds_s1);
@@ -1909,8 +1945,8 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
       }
       lds_u8* const cur = s0 + ((n_steps - 1) & 1) * kSlotBytes;
       sync();
-      pstage<false, true, true>(s0, cur, fa, c, 32, hi, sa, sb, pb, pa, w, ps, NoHook{});
-      pstage<false, false, true>(s0, cur + 8192, fa, c, 32, hi, sb, sa, pa, pb, w, ps, NoHook{});
+      pstage<false, kSmSecond, true>(s0, cur, fa, c, 32, hi, sa, sb, pb, pa, w, ps, NoHook{});
+      pstage<false, kNoSm, true>(s0, cur + 8192, fa, c, 32, hi, sb, sa, pa, pb, w, ps, NoHook{});
     }
   } else {
     // compensation of a given output: the virtual steps, step u in slot
