@@ -1753,10 +1753,10 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
         if constexpr (K == 0) {
           pstage<true, kSmSecond, true>(nxt, cur, fa, c, lb0, hi, sa, sb, pb, pa, w, ps, hook);
           pstage<true, kSmFirst, true>(nxt + 8192, cur + 8192, fa, c, la1, hi, sb, sa, pa, pb, w, ps,
-                                   NoHook{});
+                                       NoHook{});
         } else if constexpr (K == 3) {
-          pstage<true, kSmOnly, false>(nxt + h, kz, fa, c, (wave & 1) ? lb0 : la0, hi, sb, sa, pa, pb, w,
-                                    ps, hook);
+          pstage<true, kSmOnly, false>(nxt + h, kz, fa, c, (wave & 1) ? lb0 : la0, hi, sb, sa, pa, pb,
+                                       w, ps, hook);
           pstage<false, kNoSm, true>(kz, cur + h, fa, c, 32, hi, sb, sa, pb, pa, w, ps, NoHook{});
           sa = sb;
         } else {
@@ -1786,7 +1786,7 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
         pstage<false, kNoSm, true>(kz, cur + 8192, fa, c, 32, hi, sb, sa, pa, pb, w, ps, NoHook{});
       } else if constexpr (K == 3) {
         pstage<false, kSmOnly, false>(kz, kz, fa, c, (wave & 1) ? lb0 : la0, hi, sb, sa, pa, pb, w, ps,
-                                   NoHook{});
+                                      NoHook{});
         pstage<false, kNoSm, true>(kz, cur + h, fa, c, 32, hi, sb, sa, pb, pa, w, ps, NoHook{});
       } else {
         if constexpr (K == 1) sstep_zero_q(cur, fa, la0, lb0, hi, w);
@@ -1838,43 +1838,45 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
   } else {
   if constexpr (DENSE) {
     // Dense walk, the list walk's pipeline over key rows: step u is rows
-    // 64 u .. + 63 of the used rows, the last step the last 64 of them with
-    // the keys of the step before it masked (fewer than 64 rows in all: one
-    // step whose loads are clamped to them).
+    // 64 u .. + 63 of the used rows. In the last step rows past `used` may not
+    // exist, so every lane reads a row below it; those keys are masked. Only
+    // the last used row is read in their place: a masked probability is 0,
+    // but 0 times an infinite V row is NaN, so a row that is read again makes
+    // NaN of the infinity it would give (the last row of a partial step does).
     const int rem = (int)(p.used - (int64_t)(n_steps - 1) * kHalf);  // keys of the last step
-    const bool clamp = n_steps == 1 && rem < kHalf;
     const int lr = lane >> 4, pc = lane & 15;
     const uint32_t lds_s0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(s0 + 4096 * wave));
     const uint32_t lds_s1 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(s1 + 4096 * wave));
-    // first row of step u for this wave's loads (its offsets count from row
-    // 0 of the step for waves 0, 1 and from row 32 for waves 2, 3); past the
-    // last step the last one again
-    auto row_of = [&](int u) {
-      const int64_t row = min((int64_t)u * kHalf, max(p.used - kHalf, (int64_t)0));
-      return row + (wave >= 2 ? 32 : 0);
+    // this wave's loads of K or V of step u (past the last step the last one
+    // again): the base of its rows and the lane's byte offset of each segment
+    struct Src {
+      const char* base;
+      uint32_t off[4];
     };
-    auto k_base = [&](int u) { return reinterpret_cast<const char*>(kbase + row_of(u) * p.ks); };
-    auto v_base = [&](int u) { return reinterpret_cast<const char*>(vbase + row_of(u) * p.vs); };
-    // load j of an iteration: K segment j (j < 4) or V segment j - 4
-    auto issue = [&](const char* kb, const char* vb, int j, uint32_t lk, uint32_t lv) {
-      if (j < 4)
-        dma16_m0(kb, dma.k[j], lk + j * 1024);
-      else
-        dma16_m0(vb, dma.v[j - 4], lv + kHalfBytes + (j - 4) * 1024);
-    };
-    // keys 32 sub .. of step u: the count from the front that is masked (the
-    // last step holds `rem` new keys, at its end), or for the clamped step
-    // the count that is valid
-    auto mask_front = [&](f32x16& s, int u, int sub) {
-      if (u != n_steps - 1 || rem == kHalf) return;
-      if (clamp) {
-        mask_scores(s, rem - 32 * sub, hi);
-        return;
-      }
-      const int l = kHalf - rem - 32 * sub - 4 * hi;
+    auto src_of = [&](const uint16_t* x, int64_t stride, int u, bool v) {
+      const int lim = u >= n_steps - 1 ? rem : kHalf;
+      Src r;
+      r.base = reinterpret_cast<const char*>(x + (int64_t)min(u, n_steps - 1) * kHalf * stride);
 #pragma unroll
-      for (int e = 0; e < 16; ++e)
-        if (8 * (e >> 2) + (e & 3) < l) s[e] = -INFINITY;
+      for (int j = 0; j < 4; ++j) {
+        const int row = 4 * (4 * wave + j) + lr;
+        const int chunk = pc ^ (v ? (row & 3) << 2 : row & 15);
+        r.off[j] = (uint32_t)((min(row, lim - 1) * stride + (chunk << 3)) * 2);
+      }
+      return r;
+    };
+    auto k_src = [&](int u) { return src_of(kbase, p.ks, u, false); };
+    auto v_src = [&](int u) { return src_of(vbase, p.vs, u, true); };
+    // load j of an iteration: K segment j (j < 4) or V segment j - 4
+    auto issue = [&](const Src& k, const Src& v, int j, uint32_t lk, uint32_t lv) {
+      if (j < 4)
+        dma16_m0(k.base, k.off[j], lk + j * 1024);
+      else
+        dma16_m0(v.base, v.off[j - 4], lv + kHalfBytes + (j - 4) * 1024);
+    };
+    // the keys of sub-block `sub` of step u that are past `used`
+    auto mask_last = [&](f32x16& s, int u, int sub) {
+      if (u == n_steps - 1) mask_scores(s, rem - 32 * sub, hi);
     };
     f32x16 sa, sb;
     u32x4 pa[2], pb[2];
@@ -1885,51 +1887,52 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
       asm volatile("" ::: "memory");
     };
     const int64_t k_step = 2 * kHalf * p.ks, v_step = 2 * kHalf * p.vs;
-    const char *kp = k_base(2), *vp = v_base(1);
+    // steps before the last: first rows of waves 0, 1 (sub-block a) and 2, 3
+    const int64_t at = wave >= 2 ? 32 : 0;
+    const char* kp = reinterpret_cast<const char*>(kbase + (2 * kHalf + at) * p.ks);
+    const char* vp = reinterpret_cast<const char*>(vbase + (kHalf + at) * p.vs);
     auto iter = [&](auto masked, int u, lds_u8* cur, lds_u8* nxt, uint32_t lcur, uint32_t lnxt)
         __attribute__((always_inline)) {
       // M: step u + 2 may be the last one; otherwise its rows follow the
       // previous step's, and kp / vp walk along
       constexpr bool M = decltype(masked)::value;
-      const char* kb = M ? k_base(u + 2) : kp;
-      const char* vb = M ? v_base(u + 1) : vp;
+      Src ks, vs;
+      if constexpr (M) {
+        ks = k_src(u + 2);
+        vs = v_src(u + 1);
+      } else {
+        ks.base = kp;
+        vs.base = vp;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          ks.off[j] = dma.k[j];
+          vs.off[j] = dma.v[j];
+        }
+      }
       kp += k_step;
       vp += v_step;
       sync();
       pstage<true, kSmSecond, true>(nxt, cur, fa, c, 32, hi, sa, sb, pb, pa, w, ps,
-                               [&](int j) { issue(kb, vb, j, lcur, lnxt); });
-      if (M) mask_front(sa, u + 1, 0);
+                                     [&](int j) { issue(ks, vs, j, lcur, lnxt); });
+      if (M) mask_last(sa, u + 1, 0);
       pstage<true, kSmFirst, true>(nxt + 8192, cur + 8192, fa, c, 32, hi, sb, sa, pa, pb, w, ps,
-                               NoHook{});
-      if (M) mask_front(sb, u + 1, 1);
+                                    NoHook{});
+      if (M) mask_last(sb, u + 1, 1);
     };
     if (n_steps > 0) {
-      if (clamp) {
+      // K of step 0, then K of step 1 and V of step 0 in flight
+      const Src k0 = k_src(0), k1 = k_src(1), v0 = v_src(0);
 #pragma unroll
-        for (int u4 = 0; u4 < 4; ++u4) {
-          const int row = 4 * (4 * wave + u4) + lr, src = min(row, rem - 1);
-          dma16(reinterpret_cast<const char*>(kbase),
-                (uint32_t)((src * p.ks + ((pc ^ (row & 15)) << 3)) * 2), s0 + (4 * wave + u4) * 1024);
-          dma16(reinterpret_cast<const char*>(vbase),
-                (uint32_t)((src * p.vs + ((pc ^ ((row & 3) << 2)) << 3)) * 2),
-                s0 + kHalfBytes + (4 * wave + u4) * 1024);
-        }
-        VEDA_WAIT_VM(0);
-      } else {
-        // K of step 0, then K of step 1 and V of step 0 in flight
-        const char *k0 = k_base(0), *k1 = k_base(1), *v0 = v_base(0);
+      for (int j = 0; j < 4; ++j) issue(k0, v0, j, lds_s0, lds_s0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) issue(k0, v0, j, lds_s0, lds_s0);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) issue(k1, v0, j, lds_s1, lds_s0);
-        VEDA_WAIT_VM(8);
-      }
+      for (int j = 0; j < 8; ++j) issue(k1, v0, j, lds_s1, lds_s0);
+      VEDA_WAIT_VM(8);
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       pstage<true, kNoSm, false>(s0, s0, fa, c, 32, hi, sa, sb, pb, pa, w, ps, NoHook{});
-      mask_front(sa, 0, 0);
+      mask_last(sa, 0, 0);
       pstage<true, kNoSm, false>(s0 + 8192, s0, fa, c, 32, hi, sb, sa, pb, pa, w, ps, NoHook{});
-      mask_front(sb, 0, 1);
+      mask_last(sb, 0, 1);
       first_reference(sa, sb, c, 32, 32, hi, w, ps);
       pstage<false, kSmFirst, false>(s0, s0, fa, c, 32, hi, sb, sa, pa, pb, w, ps, NoHook{});
       int u = 0;
