@@ -2291,8 +2291,11 @@ tstats_kernel(FwdParams p) {
   for (int g = 0; g < 2; ++g)
 #pragma unroll
     for (int s = 0; s < 8; ++s) asm volatile("" : : "v"(qf[g][s]));
-  // a wave whose 64 query rows are all zero (padding): every score is 0
-  const bool q_zero = __ballot(any != 0) == 0;
+  // a wave whose 64 query rows are all padding, and zero: every score is 0
+  // (real zero rows take the products: 0 times a key that is not finite is not 0)
+  const bool padding =
+      item_ok && qtile >= 0 && qtile < nk && 64 * (wave & 1) >= p.valid_count[qtile];
+  const bool q_zero = (padding || !item_ok) && __ballot(any != 0) == 0;
   __syncthreads();  // sub-block list ready
   const int n_slots = (__builtin_amdgcn_readfirstlane(sub_total) + kStatSubs - 1) / kStatSubs;
 
