@@ -110,7 +110,7 @@ def load() -> ctypes.CDLL:
 
 def call(name: str, *args) -> None:
     """Calls one entry point; maps its status to ValueError / NativeError."""
-    lib = load()
+    lib = _lib or load()
     status = getattr(lib, name)(*args)
     if status != 0:
         msg = lib.veda_last_error().decode()

@@ -139,12 +139,15 @@ def _zeroed(out: torch.Tensor, groups, used: int) -> torch.Tensor:
     """The [S + 1, H, D] scatter buffer with zeros wherever no kernel writes.
     The reference zero-fills all of it (attention.py:732). When the plan's
     groups hold every head, every (real row, head) is written (each real row
-    is one valid slot of every layout), so only rows [used, S] need the zeros;
-    the scatter never writes those."""
-    if sum(g.heads.numel() for g in groups) == out.shape[1]:
-        out[used:].zero_()
-    else:
+    is one valid slot of every layout), so only rows [used, S) need the zeros;
+    row S is no part of the result. A layer without padding rows so makes no
+    fill (7 us of host time, about what the direct ops' checks of their
+    arguments take in a layer)."""
+    seq_len = out.shape[0] - 1
+    if sum(g.heads.numel() for g in groups) != out.shape[1]:
         out.zero_()
+    elif used < seq_len:
+        out[used:seq_len].zero_()
     return out
 
 

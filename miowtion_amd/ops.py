@@ -12,7 +12,9 @@ Every op refuses CPU tensors with NotImplementedError: there is no CPU path.
 
 from __future__ import annotations
 
+import functools
 import math
+import typing
 
 import torch
 
@@ -26,27 +28,47 @@ _dispatch_modes = torch._C._len_torch_dispatch_stack
 _function_modes = torch._C._len_torch_function_stack
 _transforms = torch._C._functorch.peek_interpreter_stack
 _tracing = torch._C._get_tracing_state
-_raw_stream = torch._C._cuda_getCurrentRawStream
+_forward_ad = torch.autograd.forward_ad
+_profiling = torch.autograd._profiler_enabled
+_Tensor = torch.Tensor
+# absent from a torch built without a GPU, where no op gets as far as a stream
+_raw_stream = getattr(torch._C, '_cuda_getCurrentRawStream', None)
 
 
-def _ordinary(args) -> bool:
+def _ordinary(args, kinds) -> bool:
     """Whether a call with these arguments may run its launch code directly:
-    nothing of what the dispatcher adds for the op is in play. That is: plain
-    GPU tensors, none of which autograd would have to follow; no dispatch or
-    function mode (fake tensors, a device context, a profiling mode); no
-    functorch transform, forward-mode level or tracing; not under compile."""
+    nothing of what the dispatcher adds for the op is in play. That is: every
+    argument of exactly a type that the op's schema names (`kinds`), so no
+    proxy, subclass or number to convert; plain GPU tensors that autograd would
+    not have to follow and whose memory holds their values (no lazy negation or
+    conjugation, no efficient zero tensor, which has no memory); no dispatch or
+    function mode (fake tensors, a device context); no functorch transform,
+    forward-mode level or tracing; not under compile or a profiler. Inference
+    mode needs none of this: outputs are inference tensors and versions rise as
+    through the dispatcher."""
     if (torch.compiler.is_compiling() or _dispatch_modes() or _function_modes()
-            or _transforms() is not None or torch.autograd.forward_ad._current_level >= 0
-            or _tracing() is not None):
+            or _transforms() is not None or _forward_ad._current_level >= 0
+            or _tracing() is not None or _profiling() or len(args) > len(kinds)):
         return False
     grad = torch.is_grad_enabled()
-    for a in args:
-        if type(a) is torch.Tensor:
-            if not a.is_cuda or (grad and a.requires_grad):
+    for a, kind in zip(args, kinds):
+        t = type(a)
+        if t is _Tensor:
+            if (not a.is_cuda or (grad and a.requires_grad) or kind[0] is not _Tensor
+                    or a.is_neg() or a.is_conj() or a._is_zerotensor()):
                 return False
-        elif isinstance(a, torch.Tensor):  # a subclass
+        elif t not in kind:
             return False
     return True
+
+
+def _on_gpu(fn):
+    """fn behind the device check, as the dispatcher runs it."""
+    @functools.wraps(fn)
+    def checked(*args, **kwargs):
+        _require_gpu(*args, *kwargs.values())
+        return fn(*args, **kwargs)
+    return checked
 
 
 class _Op:
@@ -55,21 +77,22 @@ class _Op:
     A custom op's way through the dispatcher costs about 24 us of host time, a
     direct call 5: a layer makes nine, which at a four-frame preview's sizes
     is more than its kernels take (200 us of host work for 84 us of kernels).
-    Every other call (gradients, modes, transforms, tracing, tensors that are
-    not on the GPU) goes through the registered op, torch.ops.veda.*, as
+    Every other call goes through the registered op, torch.ops.veda.*, as
     before. Arguments written in place have their version raised either way.
     """
 
     def __init__(self, fn, name: str, mutates_args):
         self._fn = fn
-        self._op = torch.library.custom_op(name, mutates_args=mutates_args)(fn)
+        self._op = torch.library.custom_op(name, mutates_args=mutates_args)(_on_gpu(fn))
         code = fn.__code__
         names = code.co_varnames[:code.co_argcount]
+        hints = typing.get_type_hints(fn)
+        self._kinds = tuple(typing.get_args(hints[a]) or (hints[a],) for a in names)
         self._mutated = tuple(names.index(a) for a in mutates_args)
         self.__doc__ = fn.__doc__
 
     def __call__(self, *args, **kwargs):
-        if kwargs or not _ordinary(args):
+        if kwargs or not _ordinary(args, self._kinds):
             return self._op(*args, **kwargs)
         out = self._fn(*args)
         for i in self._mutated:
@@ -84,9 +107,9 @@ def _custom_op(name: str, mutates_args=()):
     return lambda fn: _Op(fn, name, mutates_args)
 
 
-def _require_gpu(*tensors: torch.Tensor) -> None:
-    for t in tensors:
-        if t is not None and not t.is_cuda:
+def _require_gpu(*args) -> None:
+    for t in args:
+        if isinstance(t, torch.Tensor) and not t.is_cuda:
             raise NotImplementedError(
                 'miowtion_amd kernels run on the GPU only (got a tensor on '
                 f'{t.device}); there is no CPU fallback')
@@ -122,7 +145,6 @@ def gather(x: torch.Tensor, gather_index: torch.Tensor, slot_valid: torch.Tensor
     """Returns [tiles] or [tiles, feats] or [tiles, feats, sq, var]; `tiles`
     is an empty tensor when write_rows is False (pool-only). heads None: every
     head of x in order."""
-    _require_gpu(x, gather_index, slot_valid, valid_count, heads)
     _check_rows('x', x)
     n_slots = gather_index.numel()
     if n_slots % TILE:
@@ -173,7 +195,6 @@ def pool_pair(x: torch.Tensor, x2: torch.Tensor, gather_index: torch.Tensor,
               second: bool) -> list[torch.Tensor]:
     """The pooling of two tensors laid out alike in one launch: [feats,
     feats2], or [feats, sq, var, feats2, sq2, var2] with `second`."""
-    _require_gpu(x, x2, gather_index, slot_valid, valid_count, heads)
     _check_rows('x', x)
     _check_rows('x2', x2)
     if x2.shape != x.shape or x2.stride() != x.stride():
@@ -204,7 +225,6 @@ def _(x, x2, gather_index, slot_valid, valid_count, heads, second):
 @_custom_op('veda::scatter_', mutates_args=('out',))
 def scatter_(out: torch.Tensor, tiled: torch.Tensor, scatter_index: torch.Tensor,
              slot_valid: torch.Tensor, heads: torch.Tensor | None) -> None:
-    _require_gpu(out, tiled, scatter_index, slot_valid, heads)
     _check_rows('out', out)
     _check_rows('tiled', tiled)
     n_slots, hp = scatter_index.numel(), _n_heads(out, heads)
@@ -221,7 +241,6 @@ def scatter_(out: torch.Tensor, tiled: torch.Tensor, scatter_index: torch.Tensor
 @_custom_op('veda::gather_lse', mutates_args=())
 def gather_lse(lse: torch.Tensor, gather_index: torch.Tensor, slot_valid: torch.Tensor,
                heads: torch.Tensor) -> torch.Tensor:
-    _require_gpu(lse, gather_index, slot_valid, heads)
     if lse.dtype != torch.float32 or lse.dim() != 2:
         raise ValueError('lse must be fp32 [S, H]')
     out = torch.empty(gather_index.numel(), heads.numel(), dtype=torch.float32,
@@ -248,7 +267,6 @@ def select_topk(scores: torch.Tensor, block_start: int, n_cols: int, kv_ok: torc
                 index: torch.Tensor, keep: torch.Tensor, col0: int) -> None:
     """One column block of the top-k; writes index/keep[:, :, col0:col0+k_hi].
     rows: the video tile of every score row; None: row r is tile r."""
-    _require_gpu(scores, kv_ok, rows, extra, index, keep)
     if scores.dtype != torch.float32 or scores.stride(-1) != 1:
         raise ValueError('scores must be fp32 with contiguous columns')
     if index.stride() != keep.stride() or index.stride(-1) != 1:
@@ -264,7 +282,6 @@ def select_topk(scores: torch.Tensor, block_start: int, n_cols: int, kv_ok: torc
 @_custom_op('veda::dense_block_mask', mutates_args=())
 def dense_block_mask(index: torch.Tensor, keep: torch.Tensor, kv_ok: torch.Tensor,
                      n_video: int, global_rows: bool) -> torch.Tensor:
-    _require_gpu(index, keep, kv_ok)
     heads, n_sel, k_total = index.shape
     n = kv_ok.numel()
     if global_rows and n_sel != n_video:
@@ -290,7 +307,6 @@ def index_lists(block_mask: torch.Tensor, kv_ok: torch.Tensor,
                 full_tile: torch.Tensor) -> list[torch.Tensor]:
     """-> [part_cnt, part_idx, full_cnt, full_idx], cnt [1, H', R] and idx
     [1, H', R, n] int32 (miowtion/kernels/fa4.py:275-296)."""
-    _require_gpu(block_mask, kv_ok, full_tile)
     if block_mask.dtype != torch.bool or block_mask.dim() != 3:
         raise ValueError('block_mask must be bool [H\', R, n_tiles]')
     heads, rows, n = block_mask.shape
@@ -328,7 +344,6 @@ def index_lists_t(block_mask: torch.Tensor, kv_ok: torch.Tensor,
     """The Q-direction lists of a block mask [H', R, n] (fa4.py:282-296):
     rows are key tiles, entries query tiles; cnt [1, H', n] and idx
     [1, H', n, R] int32, in index_lists' order."""
-    _require_gpu(block_mask, kv_ok, full_tile)
     if block_mask.dtype != torch.bool or block_mask.dim() != 3:
         raise ValueError('block_mask must be bool [H\', R, n_tiles]')
     heads, rows, n = block_mask.shape
@@ -358,7 +373,6 @@ def selection_lists(index: torch.Tensor, keep: torch.Tensor, kv_ok: torch.Tensor
     """index_lists of dense_block_mask(index, keep, kv_ok, n_video,
     global_rows=True) in one kernel, for at most SELECTION_LISTS_MAX_TILES
     tiles."""
-    _require_gpu(index, keep, kv_ok, full_tile)
     heads, n_sel, k_total = index.shape
     n = kv_ok.numel()
     if n_sel != n_video:
@@ -391,7 +405,6 @@ def block_sparse_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     """-> [out] or [out, lse [H', R*128]]; lists as returned by index_lists.
     front_tiles: the last query tiles of every head to dispatch first (the
     rows the mask makes dense); it changes the order only."""
-    _require_gpu(q, k, v, part_cnt, part_idx, full_cnt, full_idx, valid_count)
     for name, t in (('q', q), ('k', k), ('v', v)):
         _check_rows(name, t)
     if q.shape[-1] != 128:
@@ -440,8 +453,6 @@ def block_sparse_fwd_seq_(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v
     receives the rows through scatter_index (what gather, block_sparse_fwd
     and scatter_ do in sequence). heads maps the H' heads of k / v / lists
     to heads of q and out."""
-    _require_gpu(out, q, k, v, gather_index, scatter_index, slot_valid, heads, part_cnt,
-                 part_idx, full_cnt, full_idx, valid_count)
     for name, t in (('out', out), ('q', q), ('k', k), ('v', v)):
         _check_rows(name, t)
     if q.shape[-1] != 128 or out.shape[1:] != q.shape[1:] or out.dtype != q.dtype:
@@ -484,8 +495,6 @@ def block_sparse_fwd_seq_kv_(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor
     gather_index[t]), out [S + 1, H, D] receives the rows through
     scatter_index. heads maps the H' heads of the lists to heads of q, k, v
     and out."""
-    _require_gpu(out, q, k, v, gather_index, scatter_index, slot_valid, heads, part_cnt,
-                 part_idx, full_cnt, full_idx, valid_count)
     for name, t in (('out', out), ('q', q), ('k', k), ('v', v)):
         _check_rows(name, t)
     if q.shape[-1] != 128 or out.shape[1:] != q.shape[1:] or out.dtype != q.dtype:
@@ -536,8 +545,6 @@ def block_sparse_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: tor
     """-> [dq, dk, dv] of block_sparse_fwd (fa4_sm8x/interface.py:2099
     _flash_attn_bwd with the Q-direction lists). lse: the forward's [H', R*128]
     fp32 LSE; dlse: its gradient or None; *_t: index_lists(transpose=True)."""
-    _require_gpu(q, k, v, out, dout, lse, dlse, part_cnt, part_idx, full_cnt, full_idx,
-                 part_cnt_t, part_idx_t, full_cnt_t, full_idx_t, valid_count)
     for name, t in (('q', q), ('k', k), ('v', v), ('out', out), ('dout', dout)):
         _check_rows(name, t)
     if q.shape[-1] != 128:
@@ -589,7 +596,6 @@ def dense_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, used: int,
               return_lse: bool) -> list[torch.Tensor]:
     """Dense attention of rows [0, used) of packed [S, H, D]; -> [out] or
     [out, lse [S, H]] with 0 on rows [used, S)."""
-    _require_gpu(q, k, v)
     for name, t in (('q', q), ('k', k), ('v', v)):
         _check_rows(name, t)
     if q.shape != k.shape or q.shape != v.shape or q.shape[-1] != 128:
@@ -623,7 +629,6 @@ def block_heat(q: torch.Tensor, k: torch.Tensor, lse: torch.Tensor, valid_count:
                q_tiles: torch.Tensor, reduce: str) -> torch.Tensor:
     """[H', R, n_tiles] fp32 block heat; the real rows of tile t are its first
     valid_count[t] slots (the tile layout's prefix rule)."""
-    _require_gpu(q, k, lse, valid_count, q_tiles)
     if reduce not in ('max', 'sum'):
         raise ValueError(f"reduce must be 'max' or 'sum': {reduce!r}")
     _check_rows('q', q)
@@ -670,7 +675,6 @@ def dense_heat(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor | None,
     Returns [heat [H', R, n] fp32, lse [H', R*128] fp32 (natural log)] and,
     when v is given, out [R*128, H', 128] bf16 as a third entry.
     """
-    _require_gpu(q, k, v, valid_count, q_tiles)
     if reduce not in ('max', 'sum'):
         raise ValueError(f"reduce must be 'max' or 'sum': {reduce!r}")
     _check_rows('q', q)
@@ -735,7 +739,6 @@ def _(q, k, v, valid_count, q_tiles, reduce, workspace_bytes=HEAT_WORKSPACE_BYTE
 def tile_summaries(k: torch.Tensor, v: torch.Tensor, valid_count: torch.Tensor) -> list[torch.Tensor]:
     """[kc, vc], both [n, H', D] bf16: mean of K and sum of V over each key
     tile's real rows (compensation_triton.py:80-99)."""
-    _require_gpu(k, v, valid_count)
     _check_rows('k', k)
     _check_rows('v', v)
     if k.shape != v.shape or k.shape[-1] != 128 or k.shape[0] % TILE:
@@ -764,7 +767,6 @@ def zero_order_compensation(o_kept: torch.Tensor, lse_kept: torch.Tensor, q: tor
                             valid_count: torch.Tensor) -> torch.Tensor:
     """(o_kept + sum over dropped tiles of p vc) / (1 + sum of p B), p =
     exp(q . kc / sqrt(D) - lse_kept); shapes as the reference's compensate()."""
-    _require_gpu(o_kept, lse_kept, q, kc, vc, block_mask, valid_count)
     for name, t in (('o_kept', o_kept), ('q', q), ('kc', kc), ('vc', vc)):
         _check_rows(name, t)
     rows, heads, d = o_kept.shape
@@ -807,8 +809,6 @@ def compensated_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     (compensation_triton.attention, :228-258). Lists as index_lists returns
     them for block_mask (the kept blocks, kv_ok applied); kc / vc the tile
     summaries."""
-    _require_gpu(q, k, v, part_cnt, part_idx, full_cnt, full_idx, kc, vc, block_mask,
-                 valid_count)
     for name, t in (('q', q), ('k', k), ('v', v), ('kc', kc), ('vc', vc)):
         _check_rows(name, t)
     rq, heads, d = q.shape
@@ -848,7 +848,6 @@ def _(q, k, v, part_cnt, part_idx, full_cnt, full_idx, kc, vc, block_mask, valid
 def summaries_from_means(feats_k: torch.Tensor, feats_v: torch.Tensor,
                          valid_count: torch.Tensor) -> list[torch.Tensor]:
     """tile_summaries' [kc, vc] from the pooled features [H', n, 3D] of K and V."""
-    _require_gpu(feats_k, feats_v, valid_count)
     for name, t in (('feats_k', feats_k), ('feats_v', feats_v)):
         if t.dtype != torch.float32 or t.dim() != 3 or not t.is_contiguous():
             raise ValueError(f"{name} must be contiguous fp32 [H', n, 3D]")
@@ -884,8 +883,6 @@ def compensated_attention_seq_(out: torch.Tensor, q: torch.Tensor, k: torch.Tens
     gather_index, and its rows written into out [S + 1, H, D] through
     scatter_index; k / v tile-ordered. heads maps the H' heads of k, v and the
     lists to heads of q and out."""
-    _require_gpu(out, q, k, v, gather_index, scatter_index, slot_valid, heads, part_cnt, part_idx,
-                 full_cnt, full_idx, kc, vc, block_mask, valid_count)
     for name, t in (('out', out), ('q', q), ('k', k), ('v', v), ('kc', kc), ('vc', vc)):
         _check_rows(name, t)
     if q.shape[-1] != 128 or out.shape[1:] != q.shape[1:] or out.dtype != q.dtype:
@@ -952,7 +949,6 @@ def _embed_args(feats, weight, weight_scale, residual):
 @_custom_op('veda::predictor_embed', mutates_args=())
 def predictor_embed(feats: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor | None,
                     heads: torch.Tensor, residual: bool) -> torch.Tensor:
-    _require_gpu(feats, weight, weight_scale, heads)
     f, w, wd = _embed_args(feats, weight, weight_scale, residual)
     hp, n, kd = f.shape
     n_out = w.shape[2]
@@ -974,7 +970,6 @@ def predictor_embed_pair(feats: torch.Tensor, feats2: torch.Tensor, weight: torc
                          weight_scale2: torch.Tensor | None, heads: torch.Tensor,
                          residual: bool) -> list[torch.Tensor]:
     """Two predictor_embed of the same shapes and weight format in one launch."""
-    _require_gpu(feats, feats2, weight, weight2, weight_scale, weight_scale2, heads)
     f, w, wd = _embed_args(feats, weight, weight_scale, residual)
     f2, w2, wd2 = _embed_args(feats2, weight2, weight_scale2, residual)
     if f2.shape != f.shape or w2.shape != w.shape or wd2 != wd:
@@ -1000,7 +995,6 @@ def predictor_logits(a: torch.Tensor, b: torch.Tensor, scale: float, gain: torch
                      heads: torch.Tensor | None, log_count: torch.Tensor | None,
                      base: torch.Tensor | None) -> torch.Tensor:
     """scale * a b^T (+ gain[heads] log_count) (+ base), fp32 [H', n_q, n_k]."""
-    _require_gpu(a, b, gain, heads, log_count, base)
     if a.dtype != torch.float32 or b.dtype != torch.float32 or a.dim() != 3 or b.dim() != 3:
         raise ValueError('a and b must be fp32 [H\', n, dim]')
     hp, nq, dim = a.shape
