@@ -537,7 +537,7 @@ int veda_predictor_embed(const float* feats, int64_t n_heads, int64_t n_tiles,
 
 /*
  * Two veda_predictor_embed calls of the same sizes, weight format and heads
- * (the query and key projections) in one launch.
+ * (the query and key projections) in one launch (two above 32,767 heads).
  */
 int veda_predictor_embed_pair(const float* feats, const float* feats2,
                               int64_t n_heads, int64_t n_tiles, int64_t k_dim,

@@ -452,10 +452,15 @@ extern "C" int veda_predictor_embed_pair(const float* feats, const float* feats2
                                          float* out, float* out2, void* stream) {
   VEDA_REQUIRE(feats2 != nullptr && w2 != nullptr && out2 != nullptr,
                "predictor_embed_pair: the second product's operands are required");
-  VEDA_REQUIRE(n_heads < 32768, "predictor_embed_pair: too many heads for one launch");
-  return embed_launch(feats, feats2, n_heads, n_tiles, k_dim, w, w2, w_dtype, w_scale, w_scale2,
-                      w_heads, heads, n_out, residual, out, out2,
-                      reinterpret_cast<hipStream_t>(stream));
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (n_heads <= 32767)  // both products' heads in the grid's z, 65,535 at most
+    return embed_launch(feats, feats2, n_heads, n_tiles, k_dim, w, w2, w_dtype, w_scale, w_scale2,
+                        w_heads, heads, n_out, residual, out, out2, s);
+  if (int rc = embed_launch(feats, nullptr, n_heads, n_tiles, k_dim, w, nullptr, w_dtype, w_scale,
+                            nullptr, w_heads, heads, n_out, residual, out, nullptr, s))
+    return rc;
+  return embed_launch(feats2, nullptr, n_heads, n_tiles, k_dim, w2, nullptr, w_dtype, w_scale2,
+                      nullptr, w_heads, heads, n_out, residual, out2, nullptr, s);
 }
 
 extern "C" int veda_predictor_logits(const float* a, const float* b, int64_t n_heads, int64_t n_q,

@@ -64,3 +64,13 @@ def test_a_pair_embeds_as_its_products_alone(fmt, m, k, n):
     got = ops.predictor_embed_pair(*feats, wa, wb, sa, sb, heads, k >= n)
     assert torch.equal(got[0], ops.predictor_embed(feats[0], wa, sa, heads, k >= n))
     assert torch.equal(got[1], ops.predictor_embed(feats[1], wb, sb, heads, k >= n))
+
+
+def test_a_pair_of_more_heads_than_one_launch_takes():
+    g = torch.Generator().manual_seed(1)
+    feats = [torch.randn(32768, 1, 4, generator=g).cuda() for _ in range(2)]
+    (wa, sa, _), (wb, sb, _) = (_weights('bf16', 4, 4, 8, 0, g) for _ in range(2))
+    heads = torch.randint(0, 4, (32768,), generator=g).cuda()
+    got = ops.predictor_embed_pair(*feats, wa, wb, sa, sb, heads, False)
+    assert torch.equal(got[0], ops.predictor_embed(feats[0], wa, sa, heads, False))
+    assert torch.equal(got[1], ops.predictor_embed(feats[1], wb, sb, heads, False))
