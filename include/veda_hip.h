@@ -202,7 +202,8 @@ int veda_index_lists_t(const uint8_t* block_mask, int64_t n_heads,
  * which come last in tile order), so that their long walks do not end the
  * launch; 0 is the plain (head, tile) order. The same argument of
  * veda_compensated_attention and veda_block_sparse_bwd (there it also
- * orders the key tiles of the dK / dV kernel) means the same.
+ * orders the key tiles of the dK / dV kernel, and may change the order of
+ * their sums: veda_block_sparse_bwd) means the same.
  */
 int veda_block_sparse_fwd(const void* q, int64_t q_stride_s, int64_t q_stride_h,
                           const void* k, int64_t k_stride_s, int64_t k_stride_h,
@@ -468,6 +469,11 @@ int veda_summaries_from_means(const float* feats_k, const float* feats_v,
  * through the scatter is zero on padding rows. workspace: at least
  * n_heads * n_q_tiles * 2048 bytes of device memory, 16-byte aligned
  * (per-row statistics; contents on entry do not matter).
+ * dk and dv are summed in one of two orders, by the number of (head, key
+ * tile) pairs of the call and, with front_tiles > 0, by how much longer than
+ * the mean its longest transposed list is: equal calls give equal bits, but a
+ * head's dk and dv may differ in their last bits between calls of different
+ * heads. dq is the same in every call.
  */
 int veda_block_sparse_bwd(const void* q, int64_t q_stride_s, int64_t q_stride_h,
                           const void* k, int64_t k_stride_s, int64_t k_stride_h,

@@ -9,14 +9,14 @@
 //                     units (+inf for a row with no key, so its P is 0) and
 //                     D = rowsum(dO * O) - dLSE in fp32 (the LSE output's
 //                     gradient adds dLSE * P to dS), stored as a 1 KB record
-//                     [lse2 x 64 | -D x 64 | 0 x 128] that one wave loads
+//                     [lse2 x 64 | -D x 64 | flags, 0 x 125] that one wave loads
 //                     into LDS with one DMA. -D is the initial accumulator
 //                     of the dP products, so they produce dP - D directly.
 //   dq_kernel         workgroup = (head, query tile), walking the forward
 //                     block lists (the key tiles of the row).
 //   dkv_kernel        workgroup = (head, key tile), walking the transposed
 //                     lists (the query tiles of the column); dkv_wide_kernel
-//                     where a launch has many of them.
+//                     where a launch has many of them and no few long ones.
 // Per pair of a 64-row and a 64-key half:
 //   P  = exp2(S * scale * log2(e) - lse2)   (0 past the key tile's valid count)
 //   dP = dO V^T,  dS = P * (dP - D)
@@ -51,10 +51,11 @@ namespace {
 
 constexpr int kD = 128;
 constexpr int kMaxTiles = 2048;                  // tiles per list row (FA4's cap)
-constexpr int kRecFloats = 256;                  // stats record: 64 lse2, 64 -D, the zero
-                                                 // flag, zeros
+constexpr int kRecFloats = 256;                  // stats record: 64 lse2, 64 -D, the flags,
+                                                 // zeros
 constexpr int kZeroFlag = 128;                   // 1 if every row has dO = 0 and D = 0
 constexpr int kHiZeroFlag = 129;                 // 1 if rows 32 .. 63 have dO = 0 and D = 0
+constexpr int kWideFlag = 130;                   // record 0: 1 if dK, dV take 32 keys a wave
 constexpr int kRecBytes = kRecFloats * 4;
 constexpr int kDqThreads = 256;
 constexpr int kDkvThreads = 512;
@@ -67,6 +68,18 @@ constexpr int kDkvWideThreads = 256;
 // 127; 1,184 (592 x 2) 502 and 478; 3,024 (126 x 24) 440 and 344; 9,472
 // (592 x 16) 3,821 and 3,264.
 constexpr int64_t kDkvWideItems = 768;
+// With global key tiles (`front`, kept by every query tile) a few walks are
+// many times the others' length, and where they end the launch, each alone on
+// its CU, the 16-key form is the faster one: it has two waves on every SIMD.
+// The form then goes by the mean work of a resident workgroup against the
+// longest walk, which only the lists know: the statistics kernel sums them up
+// and both forms are launched, one of which leaves at once (10 us at 2,000
+// workgroups). Whole backward with 16 and with 32 keys a wave, by that ratio
+// (tiles x heads, global tiles): 0.43 (600 x 3, 8) 2,880 and 3,318 us; 0.61
+// (134 x 8, 8) 883 and 922; 0.64 (268 x 8, 8) 2,210 and 2,229; 0.82 (142 x 8,
+// 16) 1,201 and 1,103; 0.87 (276 x 8, 16) 2,955 and 2,802; 1.2 (134 x 16, 8)
+// 1,566 and 1,432.
+constexpr int kResident = 512;                   // workgroups of either form at once
 constexpr int kSlot = 2 * kHalfBytes;            // K + V (dq) or Q + dO (dkv) of a step
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -107,6 +120,7 @@ struct BwdParams {
   uint16_t* dv;
   int64_t dqs, dqh, dks, dkh, dvs, dvh;
   int64_t front;  // the last `front` query tiles (dQ) and key tiles (dK, dV) go first
+  int pick;       // dK, dV: both forms are launched, kWideFlag says which one works
 };
 
 __device__ __forceinline__ int swz(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
@@ -218,6 +232,37 @@ __device__ __forceinline__ void list_counts(const int32_t* fc, const int32_t* pc
 }
 
 // ---------------------------------------------------------------------------
+// Whether dK and dV take 32 keys a wave, from the lengths of the transposed
+// lists: their mean for a resident workgroup at least 2/3 of the longest. For
+// the whole block, the same in every thread.
+__device__ __forceinline__ bool pick_wide(const BwdParams& p) {
+  __shared__ int64_t sums[4];
+  __shared__ int tops[4];
+  const int tid = threadIdx.x;
+  int64_t sum = 0;
+  int top = 0;
+  for (int64_t lr = tid; lr < p.n_heads * p.n_k_tiles; lr += 256) {
+    int nf, np;
+    list_counts(p.full_cnt_t, p.part_cnt_t, lr, p.list_ld_t, nf, np);
+    sum += nf + np;
+    top = max(top, nf + np);
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    sum += __shfl_xor(sum, off);
+    top = max(top, __shfl_xor(top, off));
+  }
+  if ((tid & 63) == 0) {
+    sums[tid >> 6] = sum;
+    tops[tid >> 6] = top;
+  }
+  __syncthreads();
+  sum = sums[0] + sums[1] + sums[2] + sums[3];
+  top = max(max(tops[0], tops[1]), max(tops[2], tops[3]));
+  return 3 * sum >= 2 * (int64_t)kResident * top;
+}
+
+// ---------------------------------------------------------------------------
 // Row statistics. Block = one 64-row record; 16 lanes per row, each lane 8
 // head-dims.
 
@@ -258,8 +303,10 @@ __global__ void __launch_bounds__(256) bwd_stats_kernel(BwdParams p) {
   }
   const bool zero = __syncthreads_and(!live) != 0;
   const bool zero_hi = __syncthreads_and(!live_hi) != 0;
+  const bool wide = p.pick && rec == 0 && pick_wide(p);  // block-uniform
   if (tid < 128)
-    out[kZeroFlag + tid] = (tid == 0 && zero) || (tid == 1 && zero_hi) ? 1.f : 0.f;
+    out[kZeroFlag + tid] =
+        (tid == 0 && zero) || (tid == 1 && zero_hi) || (tid == 2 && wide) ? 1.f : 0.f;
 }
 
 // ---------------------------------------------------------------------------
@@ -568,6 +615,7 @@ __global__ void __launch_bounds__(kDkvThreads) __attribute__((amdgpu_waves_per_e
   __shared__ __attribute__((aligned(1024))) uint8_t ring[2][kSlot + kRecBytes];
   __shared__ uint16_t steps[2 * kMaxTiles];
   __shared__ int32_t step_total, step_hz;
+  if (p.pick && p.stats[kWideFlag] != 0.f) return;  // the other form works
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int n = lane & 15, g = lane >> 4;
@@ -856,11 +904,12 @@ __global__ void __launch_bounds__(kDkvThreads) __attribute__((amdgpu_waves_per_e
 // bound it. The sums of 128 x 32 dK and dV take 128 registers and the
 // fragments of K and V 64, so it fits the 256 of two waves per SIMD only with
 // nothing kept that can be formed again (the lane's index, read and load
-// offsets) and fragments read two products ahead. It has to fit: with eight
+// offsets) and fragments read two products ahead. It has to fit: with ten
 // registers spilled, reloads waited for the step's loads (a scratch read
-// counts as one), and the kernel took 17 % longer. A workgroup lasts about
-// twice as long as dkv_kernel's, two at a time on a CU, so a launch needs
-// more than a round of them (kDkvWideItems). dK, dV alone, 16 -> 32 keys:
+// counts as one): 10.6 ms at 57,720 tokens x 48 heads, 9.5 with none. A
+// workgroup lasts about twice as long as dkv_kernel's, two at a time on a CU,
+// so a launch needs more than a round of them (kDkvWideItems) and no few walks
+// much longer than the rest (pick_wide). dK, dV alone, 16 -> 32 keys:
 // 57,720 tokens x 16 heads, keep 0.1: 3.82 -> 3.26 ms; 13x24x42 tokens x 24
 // heads: 440 -> 344 us. Four fragments ahead in the first and last phase: the
 // same.
@@ -882,6 +931,7 @@ __global__ void __launch_bounds__(kDkvWideThreads, 2) dkv_wide_kernel(BwdParams 
   __shared__ __attribute__((aligned(1024))) uint8_t ring[2][kSlot + kRecBytes];
   __shared__ uint16_t steps[2 * kMaxTiles];
   __shared__ int32_t step_total, step_hz;
+  if (p.pick && p.stats[kWideFlag] == 0.f) return;  // the other form works
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int li = lane & 31, hi = lane >> 5;
@@ -1250,6 +1300,11 @@ extern "C" int veda_block_sparse_bwd(
   p.front = front_tiles;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int64_t q_items = n_heads * n_q_tiles, k_items = n_heads * n_k_tiles;
+  // Every key tile is kept by the `front` query tiles, and the `front` key
+  // tiles by all: the ratio is at least n_heads (2 front + 1) / kResident, and
+  // from 2/3 on the lists need not be asked.
+  p.pick = front_tiles > 0 && k_items >= kDkvWideItems && q_items > 0 &&
+           3 * n_heads * (2 * front_tiles + 1) < 2 * (int64_t)kResident;
   if (q_items > 0) {
     bwd_stats_kernel<<<(unsigned)(2 * q_items), 256, 0, s>>>(p);
     if (int rc = check_launch("veda_block_sparse_bwd (stats)")) return rc;
@@ -1257,9 +1312,10 @@ extern "C" int veda_block_sparse_bwd(
     if (int rc = check_launch("veda_block_sparse_bwd (dq)")) return rc;
   }
   if (k_items > 0) {
-    if (k_items >= kDkvWideItems)
+    const bool many = k_items >= kDkvWideItems;
+    if (many)
       dkv_wide_kernel<<<(unsigned)k_items, kDkvWideThreads, 0, s>>>(p);
-    else
+    if (!many || p.pick)
       dkv_kernel<<<(unsigned)k_items, kDkvThreads, 0, s>>>(p);
     return check_launch("veda_block_sparse_bwd (dk, dv)");
   }
