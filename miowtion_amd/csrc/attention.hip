@@ -715,7 +715,8 @@ __device__ __forceinline__ void sstep_half_zero(const lds_u8* slot, const HFrag&
 // (the same board multiplies random bf16 matrices at 1.5 and zeros at 2.0
 // PFLOP/s). Sparse walks, where K and V come from beyond L2: sequence order
 // 6.08 -> 5.92 ms the whole layer (with the dead waves dropped), 14.64 ->
-// 14.12 at keep 0.2; tile order 5.56 -> 5.51 ms, 12.67 -> 12.35 at keep 0.2.
+// 14.12 at keep 0.2; tile order 5.56 -> 5.51 ms, 12.67 -> 12.35 at keep 0.2
+// (5.44 and 12.18 with NextFrags).
 //
 // The reference of a row is the maximum of its first step's 64 keys (narrow
 // walks: of its first sub-block); later probabilities are taken against it as
@@ -783,10 +784,29 @@ __device__ __forceinline__ void first_reference(f32x16& sa, f32x16& sb, float c,
   ps.have_ref = __ballot(w.m_run != -INFINITY) == ~0ull;
 }
 
-template <bool QK, int SM, bool PV, typename Hook>
+// Fragments of the stage that follows on the same slots (sub-block b after a):
+// the first four of K and the first of V^T, read in the place of a stage's
+// last reads, so that its products do not begin with a wait for LDS. Four K
+// fragments ahead of their products and one of V^T (two transposed reads
+// each): a read waits behind all of a wave's earlier ones. Two and two, and
+// no fragments carried over, took 5 % longer where a walk is alone on its CU
+// (6x32x32 tokens + 1,024 text rows x 3 heads 113.4 -> 105.6 us) and 1 to 2 %
+// in full launches (57,720 x 48, keep 0.1 5.49 -> 5.44 ms, keep 0.2 12.42 ->
+// 12.18); three and three, or four and four, without carrying 3 to 6 % longer.
+struct NextFrags {
+  u32x4 k[4];
+  bf16x8 v;
+};
+
+// What a stage does with NextFrags: nothing, read them for the next stage, or
+// take them as its own first fragments.
+enum { kNoNext = 0, kReadNext = 1, kTakeNext = 2 };
+
+template <bool QK, int SM, bool PV, int NEXT = kNoNext, typename Hook>
 __device__ __forceinline__ void pstage(const lds_u8* kb, const lds_u8* vb, const HFrag& f, float c,
                                        int lim, int hi, f32x16& sn, f32x16& sp, u32x4 (&pn)[2],
-                                       const u32x4 (&pp)[2], WaveState& w, PipeState& ps, Hook hook) {
+                                       const u32x4 (&pp)[2], WaveState& w, PipeState& ps, Hook hook,
+                                       NextFrags* next = nullptr) {
   typedef const __attribute__((address_space(3))) u32x4* lds_u32x4;
   if (SM) mask_scores(sp, lim, hi);
   if (PV && __any(ps.alpha != 1.f)) {
@@ -801,12 +821,10 @@ __device__ __forceinline__ void pstage(const lds_u8* kb, const lds_u8* vb, const
 #pragma unroll
     for (int e = 0; e < 16; ++e) sn[e] = 0.f;
 #pragma unroll
-    for (int k = 0; k < 2; ++k) kf[k] = *reinterpret_cast<lds_u32x4>(kb + f.k[k]);
+    for (int k = 0; k < 4; ++k)
+      kf[k] = NEXT == kTakeNext ? next->k[k] : *reinterpret_cast<lds_u32x4>(kb + f.k[k]);
   }
-  if (PV) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) va[j] = vt_frag(vb, f, 0, j);
-  }
+  if (PV) va[0] = NEXT == kTakeNext ? next->v : vt_frag(vb, f, 0, 0);
   float l4[4];
   const float mu = w.mu;
   __builtin_amdgcn_sched_barrier(0);
@@ -814,7 +832,8 @@ __device__ __forceinline__ void pstage(const lds_u8* kb, const lds_u8* vb, const
   for (int j = 0; j < 8; ++j) {
     hook(j);
     if (QK) {
-      if (j + 2 < 8) kf[j + 2] = *reinterpret_cast<lds_u32x4>(kb + f.k[j + 2]);
+      if (j + 4 < 8) kf[j + 4] = *reinterpret_cast<lds_u32x4>(kb + f.k[j + 4]);
+      else if (NEXT == kReadNext) next->k[j - 4] = *reinterpret_cast<lds_u32x4>(kb + 8192 + f.k[j - 4]);
       sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kf[j]), w.qf[j], sn, 0, 0, 0);
     }
     if (SM) {
@@ -826,7 +845,8 @@ __device__ __forceinline__ void pstage(const lds_u8* kb, const lds_u8* vb, const
       pn[j >> 2][j & 3] = pk;
     }
     if (PV) {
-      if (j + 2 < 8) va[j + 2] = vt_frag(vb, f, (j + 2) >> 2, (j + 2) & 3);
+      if (j + 1 < 8) va[j + 1] = vt_frag(vb, f, (j + 1) >> 2, (j + 1) & 3);
+      else if (NEXT == kReadNext) next->v = vt_frag(vb + 8192, f, 0, 0);
       w.o[j & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[j], as_bf16x8(pp[j >> 2]), w.o[j & 3],
                                                            0, 0, 0);
     }
@@ -1751,9 +1771,11 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
         auto hook = [&](int j) { issue(kb, vb, o2, ov, j, lcur, lnxt); };
         const int la0 = (int)(r0.a & 63u), lb0 = (int)(r0.b & 63u), la1 = (int)(r1.a & 63u);
         if constexpr (K == 0) {
-          pstage<true, kSmSecond, true>(nxt, cur, fa, c, lb0, hi, sa, sb, pb, pa, w, ps, hook);
-          pstage<true, kSmFirst, true>(nxt + 8192, cur + 8192, fa, c, la1, hi, sb, sa, pa, pb, w, ps,
-                                       NoHook{});
+          NextFrags next;
+          pstage<true, kSmSecond, true, kReadNext>(nxt, cur, fa, c, lb0, hi, sa, sb, pb, pa, w, ps,
+                                                   hook, &next);
+          pstage<true, kSmFirst, true, kTakeNext>(nxt + 8192, cur + 8192, fa, c, la1, hi, sb, sa, pa,
+                                                  pb, w, ps, NoHook{}, &next);
         } else if constexpr (K == 3) {
           pstage<true, kSmOnly, false>(nxt + h, kz, fa, c, (wave & 1) ? lb0 : la0, hi, sb, sa, pa, pb,
                                        w, ps, hook);
@@ -1912,11 +1934,12 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
       kp += k_step;
       vp += v_step;
       sync();
-      pstage<true, kSmSecond, true>(nxt, cur, fa, c, 32, hi, sa, sb, pb, pa, w, ps,
-                                     [&](int j) { issue(ks, vs, j, lcur, lnxt); });
+      NextFrags next;
+      pstage<true, kSmSecond, true, kReadNext>(nxt, cur, fa, c, 32, hi, sa, sb, pb, pa, w, ps,
+                                               [&](int j) { issue(ks, vs, j, lcur, lnxt); }, &next);
       if (M) mask_last(sa, u + 1, 0);
-      pstage<true, kSmFirst, true>(nxt + 8192, cur + 8192, fa, c, 32, hi, sb, sa, pa, pb, w, ps,
-                                    NoHook{});
+      pstage<true, kSmFirst, true, kTakeNext>(nxt + 8192, cur + 8192, fa, c, 32, hi, sb, sa, pa, pb, w,
+                                              ps, NoHook{}, &next);
       if (M) mask_last(sb, u + 1, 1);
     };
     if (n_steps > 0) {
