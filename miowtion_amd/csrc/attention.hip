@@ -47,7 +47,9 @@ constexpr int kD = 128;
 constexpr int kThreads = 512;
 constexpr int kMaxBlocks = 2048;                 // key tiles per row (FA4's cap)
 // LDS offset in ring slot 1 of the Q fragments a narrow walk hands from wave
-// 0 to wave 1 (8 KB, past the set-up's 12 KB step-list scratch)
+// 0 to wave 1: 8 KB in the slot's V half, which is loaded only after the
+// walk's second barrier (its K half, where the set-up's 12 KB step-list
+// scratch is, is loaded right after the set-up's last barrier).
 constexpr int kNarrowQ = 16384;
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr float kRescaleSlack = 8.f;             // log2 units
@@ -145,8 +147,9 @@ struct WaveState {
 // step. The two key halves merge at the end.
 
 constexpr int kSlotBytes = 2 * kHalfBytes;      // 32 KB: K + V
-static_assert(3 * kMaxBlocks * 2 <= kNarrowQ && kNarrowQ + 8 * 64 * 16 <= kSlotBytes,
-              "narrow-walk Q fragments overlap the step-list scratch or leave the slot");
+static_assert(3 * kMaxBlocks * 2 <= kHalfBytes && kNarrowQ >= kHalfBytes &&
+                  kNarrowQ + 8 * 64 * 16 <= kSlotBytes,
+              "step-list scratch in the slot's K half, narrow-walk Q fragments in its V half");
 
 // Per-lane byte offsets of the HBM -> LDS loads of one step. Wave w fills K
 // and V segments 2w, 2w + 1 (1 KB = rows 4 seg .. 4 seg + 3 of the half);
@@ -715,8 +718,8 @@ __device__ __forceinline__ void sstep_half_zero(const lds_u8* slot, const HFrag&
 // (the same board multiplies random bf16 matrices at 1.5 and zeros at 2.0
 // PFLOP/s). Sparse walks, where K and V come from beyond L2: sequence order
 // 6.08 -> 5.92 ms the whole layer (with the dead waves dropped), 14.64 ->
-// 14.12 at keep 0.2; tile order 5.56 -> 5.51 ms, 12.67 -> 12.35 at keep 0.2
-// (5.44 and 12.18 with NextFrags).
+// 14.12 at keep 0.2; tile order 5.69 -> 5.64 ms, 13.04 -> 12.75 at keep 0.2
+// (5.60 and 12.54 with NextFrags).
 //
 // The reference of a row is the maximum of its first step's 64 keys (narrow
 // walks: of its first sub-block); later probabilities are taken against it as
@@ -789,10 +792,11 @@ __device__ __forceinline__ void first_reference(f32x16& sa, f32x16& sb, float c,
 // last reads, so that its products do not begin with a wait for LDS. Four K
 // fragments ahead of their products and one of V^T (two transposed reads
 // each): a read waits behind all of a wave's earlier ones. Two and two, and
-// no fragments carried over, took 5 % longer where a walk is alone on its CU
-// (6x32x32 tokens + 1,024 text rows x 3 heads 113.4 -> 105.6 us) and 1 to 2 %
-// in full launches (57,720 x 48, keep 0.1 5.49 -> 5.44 ms, keep 0.2 12.42 ->
-// 12.18); three and three, or four and four, without carrying 3 to 6 % longer.
+// no fragments carried over, took 7 % longer where a walk is alone on its CU
+// (6x32x32 tokens + 1,024 text rows x 3 heads 114.2 -> 106.3 us) and 1 to 2 %
+// in full launches (57,720 x 48, keep 0.1 5.64 -> 5.60 ms, keep 0.2 12.75 ->
+// 12.54); three and three, or four and four, without carrying 3 to 6 % longer
+// than two and two.
 struct NextFrags {
   u32x4 k[4];
   bf16x8 v;
@@ -1248,8 +1252,9 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
     const int nf = min(max(p.full_cnt[li_], 0), min(ld, kMaxBlocks));
     const int np = min(max(p.part_cnt[li_], 0), min(ld, kMaxBlocks - nf));
     for (int j = tid; j < nk; j += kThreads2) tvc[j] = (uint8_t)min(max(p.valid_count[j], 0), kTile);
-    // scratch in ring slot 1 (12 KB), which no load targets before the
-    // walk's first barrier: both lists, then the walk order (j << 1 | full)
+    // scratch in ring slot 1 (12 KB), done with at the set-up's last barrier,
+    // before any load targets the slot: both lists, then the walk order (j <<
+    // 1 | full)
     uint16_t* sf = reinterpret_cast<uint16_t*>(&ring[1][0]);
     uint16_t* sp = sf + kMaxBlocks;
     uint16_t* sm = sp + kMaxBlocks;
@@ -1415,8 +1420,7 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
     if ((MODE == kSparse || MODE == kVirtualOnly) && lane == 0)
       zflag[wave] = (q_zero ? 1 : 0) | (dead ? 2 : 0);
     // wave 0's Q fragments for wave 1 of a narrow walk (below), in ring
-    // slot 1 past the step-list scratch; no load reaches slot 1 before the
-    // walk's first barrier
+    // slot 1's V half (kNarrowQ)
     if ((MODE == kSparse || MODE == kVirtualOnly) && wave == 0) {
 #pragma unroll
       for (int s = 0; s < 8; ++s)
@@ -1482,8 +1486,8 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
       for (int s = 0; s < 8; ++s)
         w.qf[s] = as_bf16x8(*reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(
             (const lds_u8*)ring[1] + kNarrowQ + (s * 64 + lane) * 16));
-      // read before this wave reaches the walk's first barrier, after which
-      // loads may target slot 1
+      // read before this wave reaches the walk's first barrier; the V half of
+      // slot 1 is loaded after the second (kNarrowQ)
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
   }
@@ -2240,7 +2244,9 @@ __global__ void __launch_bounds__(kThreads2, 2) sfwd_kernel(FwdParams p) {
 // Before, a wave multiplied and then exponentiated, sixteen 32-row waves met
 // at a barrier every 64 keys, and the two phases of all four waves of a SIMD
 // fell together: 4,800 cycles per step at full clock against 2,048 of
-// products. TSTATSTABLE
+// products. The pass with its combine, 37x24x42 tokens x 56 heads: 27.0 ->
+// 22.9 ms; on constant data 24.7 -> 20.7, of which 17.0 stay without the
+// exponentials.
 //
 // K goes through a ring of three 128-row slots (four sub-blocks, each wave
 // one 1 KB segment of each), two in flight while one is used, with one

@@ -73,8 +73,8 @@ constexpr int64_t kDkvWideItems = 768;
 // its CU, the 16-key form is the faster one: it has two waves on every SIMD.
 // The form then goes by the mean work of a resident workgroup against the
 // longest walk, which only the lists know: the statistics kernel sums them up
-// and both forms are launched, one of which leaves at once (10 us at 2,000
-// workgroups). Whole backward with 16 and with 32 keys a wave, by that ratio
+// and both forms are launched, one of which leaves at once (below 6 us at
+// 1,000 to 2,000 workgroups). Whole backward with 16 and with 32 keys a wave, by that ratio
 // (tiles x heads, global tiles): 0.43 (600 x 3, 8) 2,880 and 3,318 us; 0.61
 // (134 x 8, 8) 883 and 922; 0.64 (268 x 8, 8) 2,210 and 2,229; 0.82 (142 x 8,
 // 16) 1,201 and 1,103; 0.87 (276 x 8, 16) 2,955 and 2,802; 1.2 (134 x 16, 8)
