@@ -63,6 +63,26 @@ def test_a_pair_pools_as_its_tensors_alone(dim, second):
         kernels.pool_seq_pair(x, y[:, 1:], lay, heads)
 
 
+@pytest.mark.parametrize('heads', [28, 25])
+@pytest.mark.parametrize('second', [False, True])
+def test_a_large_pair_pools_as_its_tensors_alone(heads, second):
+    """A pair whose launch takes the one-wave form (441 tiles x 7 head groups,
+    the last workgroup cut), its tensors alone, and chunks of their heads,
+    which take the split form."""
+    spec = ([(64, (40, 22, 62))], 54624, 56320, '4x2x16')
+    lay = helpers.product_layout(*spec, device='cuda')
+    g = torch.Generator('cuda').manual_seed(heads)
+    x, y = (torch.randn(56320, heads, 128, generator=g, device='cuda').to(torch.bfloat16) for _ in range(2))
+    groups = lay.n_tiles * -(-heads // 4)
+    assert 2 * groups >= 2560 > lay.n_tiles and groups % 4
+    pair = kernels.pool_seq_pair(x, y, lay, None, second)
+    for got, t in zip(pair, (x, y)):
+        for a, b in zip(got, kernels.pool_seq(t, lay, None, second)):
+            assert torch.equal(a, b)
+        few = torch.cat([kernels.pool_seq(t, lay, h)[0] for h in torch.arange(heads, device='cuda').split(4)])
+        assert second or torch.equal(got[0], few)
+
+
 @pytest.mark.parametrize('dim', [64, 128])
 @pytest.mark.parametrize('heads', [1, 5, 16])
 def test_no_heads_is_every_head_in_order(dim, heads):
