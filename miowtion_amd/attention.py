@@ -135,6 +135,12 @@ def _chunk_heads(tile_layout: tiling.TileLayout, collect_bytes: int) -> int:
     return max(1, collect_bytes // (tile_layout.num_slots * _HEAD_DIM_BYTES))
 
 
+def _head_chunks(heads: torch.Tensor, tile_layout: tiling.TileLayout, collect_bytes: int):
+    """A group's heads in chunks of at most _chunk_heads (usually one chunk)."""
+    chunk = _chunk_heads(tile_layout, collect_bytes)
+    return (heads,) if 0 < heads.numel() <= chunk else heads.split(chunk)
+
+
 def _zeroed(out: torch.Tensor, groups, used: int) -> torch.Tensor:
     """The [S + 1, H, D] scatter buffer with zeros wherever no kernel writes.
     The reference zero-fills all of it (attention.py:732). When the plan's
@@ -196,7 +202,7 @@ class SparseStudent:
         self.last = {}
         for group in groups:
             tile_layout = self.clip.get(group.shape)
-            for heads in group.heads.split(_chunk_heads(tile_layout, self.clip.config.collect_bytes)):
+            for heads in _head_chunks(group.heads, tile_layout, self.clip.config.collect_bytes):
                 self._attend(q, k, v, layer_index, tile_layout, heads, out)
         return out[:seq_len]
 
@@ -295,7 +301,7 @@ class OracleStudent:
         self.last = {'lse': lse}
         for group in groups:
             tile_layout = self.clip.get(group.shape)
-            for heads in group.heads.split(_chunk_heads(tile_layout, self.clip.config.collect_bytes)):
+            for heads in _head_chunks(group.heads, tile_layout, self.clip.config.collect_bytes):
                 self._attend(q, k, v, lse, tile_layout, heads, out)
         return out[:seq_len]
 

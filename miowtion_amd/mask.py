@@ -135,14 +135,12 @@ def select_video_blocks(scores: torch.Tensor, layout: tiling.TileLayout,
     if scores.shape[1] != num_rows:
         raise ValueError(f'scores has {scores.shape[1]} query rows but rows has {num_rows}; '
                          'index the query axis by `rows` before calling')
-    widths = []
+    splits = []  # (k_lo, k_hi, frac) of each block; k_hi is its width
     for block in blocks:
         n_cols = block.stop - block.start
-        if block.budget.keeps_all:
-            widths.append(n_cols)
-        else:
-            widths.append(split_budget(block.budget.per_row(block.real_tokens, n_cols), n_cols)[1])
-    k_total = sum(widths)
+        splits.append((n_cols, n_cols, 0.0) if block.budget.keeps_all else
+                      split_budget(block.budget.per_row(block.real_tokens, n_cols), n_cols))
+    k_total = sum(k_hi for _, k_hi, _ in splits)
     index = torch.empty(heads, num_rows, k_total, dtype=torch.int64, device=device)
     keep = torch.empty(heads, num_rows, k_total, dtype=torch.bool, device=device)
     scores32 = scores if scores.dtype == torch.float32 else scores.float()
@@ -151,18 +149,15 @@ def select_video_blocks(scores: torch.Tensor, layout: tiling.TileLayout,
     if rows is not None:
         rows = rows.to(device=device, dtype=torch.int64).contiguous()
     col0 = 0
-    for block, width in zip(blocks, widths):
-        n_cols = block.stop - block.start
+    for block, (k_lo, k_hi, frac) in zip(blocks, splits):
         if block.budget.keeps_all:
-            index[:, :, col0:col0 + width] = torch.arange(block.start, block.stop, device=device)
-            keep[:, :, col0:col0 + width] = layout.kv_ok[block.start:block.stop]
+            index[:, :, col0:col0 + k_hi] = torch.arange(block.start, block.stop, device=device)
+            keep[:, :, col0:col0 + k_hi] = layout.kv_ok[block.start:block.stop]
         else:
-            budget = block.budget.per_row(block.real_tokens, n_cols)
-            k_lo, k_hi, frac = split_budget(budget, n_cols)
             extra = bresenham_extra(n_video, frac, device)
-            ops.select_topk(scores32, block.start, n_cols, layout.kv_ok, rows, k_lo, k_hi,
-                            extra, index, keep, col0)
-        col0 += width
+            ops.select_topk(scores32, block.start, block.stop - block.start, layout.kv_ok, rows,
+                            k_lo, k_hi, extra, index, keep, col0)
+        col0 += k_hi
     return Selection(index, keep)
 
 
